@@ -112,9 +112,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_x(int64_t n, const double *__rest
 }
 
 // Ap = A p and the partials of pAp = p.Ap.  One 256-row tile per block.
-// CI: column indices from the compact form.
-template <bool CI>
-__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CI) void k_cg_spmv_dot(const ColIdx ci, const double *__restrict__ vals,
+// CI: column indices from the compact form.  VF: the values' form.
+template <bool CI, int VF>
+__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CI) void k_cg_spmv_dot(const ColIdx ci, const ValSrc<double, double> src,
                                                         const double *__restrict__ p,
                                                         double *__restrict__ Ap, int64_t nrows,
                                                         double *partials) {
@@ -123,15 +123,15 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CI) void k_c
   if (row < nrows) {
     const size_t b = ell_base(row);
     const int slice = slice_of<true>(row);
-    double v[kSlots];
-    row_vals<double, true, kAllSlots>(vals, row, v);
+    RowVals<VF, double, double, true, kAllSlots> v;
+    v.load(src, row);
     const double sum = with_cols<CI, true>(ci, slice, [&](auto cm, const int *base) {
       constexpr int CM = decltype(cm)::value;
       double acc_row = 0.0;
 #pragma unroll
       for (int s = 0; s < kSlots; ++s) {
         const int c = col_at<CM, true>(ci, row, base, b, s);
-        acc_row += v[s] * p[c];
+        acc_row += v.at(s, c) * p[c];
       }
       return acc_row;
     });
@@ -420,10 +420,9 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
       else
         k_cg_px<false><<<tiles(np), kBlock, 0, c->stream>>>(np, z, p, x, c->scal, j == 1);
       tm.mark(3);
-      if (ci0.cbase)
-        k_cg_spmv_dot<true><<<T, kBlock, 0, c->stream>>>(ci0, L0.vals, p, Ap, np, c->partials);
-      else
-        k_cg_spmv_dot<false><<<T, kBlock, 0, c->stream>>>(ci0, L0.vals, p, Ap, np, c->partials);
+      with_forms<double>(L0, ci0, [&](auto CI, auto VF) {
+        k_cg_spmv_dot<CI(), VF()><<<T, kBlock, 0, c->stream>>>(ci0, val_src<double, double>(L0), p, Ap, np, c->partials);
+      });
       if ((rc = finish(c, 1, T, F_PAP))) return rc;
       tm.mark(4);
       k_cg_update_r<<<G, kBlock, 0, c->stream>>>(np, r, Ap, c->partials, c->scal);
@@ -517,10 +516,9 @@ static int cg_mixed(Ctx *c, int variant, const double *b, double *x, int max_ite
     restart = false;
     tm.mark(3);
     const ColIdx ci0 = col_idx(c, L0);
-    if (ci0.cbase)
-      k_cg_spmv_dot<true><<<T, kBlock, 0, c->stream>>>(ci0, L0.vals, p, Ap, np, c->partials);
-    else
-      k_cg_spmv_dot<false><<<T, kBlock, 0, c->stream>>>(ci0, L0.vals, p, Ap, np, c->partials);
+    with_forms<double>(L0, ci0, [&](auto CI, auto VF) {
+      k_cg_spmv_dot<CI(), VF()><<<T, kBlock, 0, c->stream>>>(ci0, val_src<double, double>(L0), p, Ap, np, c->partials);
+    });
     if ((rc = finish(c, 1, T, F_PAP))) return rc;
     tm.mark(4);
     k_cg_update<true><<<G, kBlock, 0, c->stream>>>(np, x, p, r, Ap, r32, c->partials, c->scal, dscale);

@@ -140,6 +140,24 @@ constexpr bool val_layout_ok() {
 }
 static_assert(val_layout_ok<2>() && val_layout_ok<4>(), "value layouts");
 
+// Where the kernels take a level's off-diagonal values from.  The stored
+// array always exists; the other two forms are used on stencil levels whose
+// stored values, checked entry by entry and bit for bit when the level is
+// set up, are what the form gives (k_compact_cols).  They are exact: the
+// products and sums are the same, only fewer bytes are read.  (Value
+// compression of this kind is known for CSR as CSR-VI: Kourtis, Goumas,
+// Koziris, "Optimizing sparse matrix-vector multiplication using index and
+// value compression", 2008.)
+enum ValForm : int {
+  kValsStored = 0,  // the value array, 8 / 4 / 2 bytes per slot
+  kValsSlot = 1,    // each slot holds one value over the whole level, or +0: 27 values and a 32-bit row mask
+  kValsField = 2,   // -(k_i + k_j)/2 of a per-row field k (the generated kappa operator), and the row mask
+};
+
+// What the building of a level's compact columns and value forms reports per
+// level: mismatches of each form, and the number of wide slices.
+enum FormFlag : int { kBadSlot = 0, kBadDiag, kBadField, kWideSlices, kFormFlags };
+
 // Column index format of a context (hpcgx_set_column_format).
 enum ColFormat : int { kColsExplicit = 0, kColsCompact = 1, kColsCompactAlways = 2 };
 
@@ -273,6 +291,17 @@ struct Level {
   // slices are wide (on a level of mostly wide slices the explicit indices
   // ran faster: a renumbered 128^3 hierarchy, 779 against 747 GFLOP/s)
   bool read_compact = false;
+  // Value form of the fp64 matrix (ValForm).  vmask: bit s set where slot s
+  // of the row stores an entry (bit 13: a row of the level, clear on
+  // padding); slotv: the 27 slot values of kValsSlot, then the same for the
+  // fp32 and the scaled fp16 copy; field: kappa in row order (generated kappa
+  // levels).  diag_one: every diagonal equals slot 13's value, else the
+  // diagonals are read from the value array.
+  int vform = kValsStored;
+  bool diag_one = false;
+  uint32_t *vmask = nullptr;
+  double *slotv = nullptr;
+  double *field = nullptr;
   float *dinv = nullptr;   // fp16 copy: 1/sqrt(a_ii), colour order
   float *sigma = nullptr;  // fp16 copy: sqrt(d_f/d_c) per injected row
   int *perm = nullptr;
@@ -301,7 +330,7 @@ struct Ctx {
   double *partials = nullptr;  // per-block partial sums, 2 x the largest level-0 grid
   double *folded = nullptr;    // second-level partials of large reductions (same allocation)
   int64_t reduce_cap = 0;      // largest grid the scratch covers
-  double *scal = nullptr;      // device scalars [S_COUNT]
+  double *scal = nullptr;      // device scalars [S_COUNT], then the levels' form flags (FormFlag)
   double *hist = nullptr;      // device norms of a deferred-stop batch
   int hist_cap = 0;
   std::vector<hipEvent_t> evpool;  // phase events of a deferred-stop batch (6 per iteration)

@@ -206,6 +206,82 @@ __device__ __forceinline__ void row_vals(const VT *__restrict__ vals, int64_t ro
       std::make_integer_sequence<int, val_units(W)>{});
 }
 
+// A launch's value source: the stored values, the row masks, the slot values
+// (kValsSlot) and the field (kValsField).
+template <class VT, class ACC>
+struct ValSrc {
+  const VT *vals;
+  const uint32_t *mask;
+  const ACC *slotv;
+  const double *field;
+  int diag_one;  // kValsSlot: the diagonal is slotv[13] on every row
+};
+
+// v where bit s of m is set, else +0: two or three integer operations, no
+// branch and no compare.
+__device__ __forceinline__ double bit_select(uint32_t m, int s, double v) {
+  const int k = (int)(m << (31 - s)) >> 31;
+  return __hiloint2double(__double2hiint(v) & k, __double2loint(v) & k);
+}
+__device__ __forceinline__ float bit_select(uint32_t m, int s, float v) {
+  const int k = (int)(m << (31 - s)) >> 31;
+  return __int_as_float(__float_as_int(v) & k);
+}
+
+// The off-diagonal values of one row in any form.  load() issues the row's
+// loads; at(s, c) is the value of slot s, whose column is c.
+template <int VF, class VT, class ACC, bool NT, uint32_t MASK>
+struct RowVals;
+
+template <class VT, class ACC, bool NT, uint32_t MASK>
+struct RowVals<kValsStored, VT, ACC, NT, MASK> {
+  ACC v[kSlots];
+  __device__ __forceinline__ void load(const ValSrc<VT, ACC> &src, int64_t row) {
+    row_vals<ACC, NT, MASK>(src.vals, row, v);
+  }
+  __device__ __forceinline__ ACC at(int s, int) const { return v[s]; }
+  // the diagonal of a stencil row
+  __device__ __forceinline__ ACC diag(const ValSrc<VT, ACC> &src, int64_t row) const {
+    if constexpr ((MASK >> kDiagSlot) & 1u) return v[kDiagSlot];
+    else return ld_val<ACC, NT>(src.vals + val_pos<val_width<VT>>(row, kDiagSlot));
+  }
+};
+
+template <class VT, class ACC, bool NT, uint32_t MASK>
+struct RowVals<kValsSlot, VT, ACC, NT, MASK> {
+  uint32_t m;
+  ACC d;
+  const ACC *slotv;
+  __device__ __forceinline__ void load(const ValSrc<VT, ACC> &src, int64_t row) {
+    slotv = src.slotv;
+    if constexpr (NT) m = __builtin_nontemporal_load(src.mask + row);
+    else m = src.mask[row];
+    if (src.diag_one) d = (m >> kDiagSlot) & 1u ? slotv[kDiagSlot] : (ACC)1;  // padding: the identity row
+    else d = ld_val<ACC, NT>(src.vals + val_pos<val_width<VT>>(row, kDiagSlot));
+  }
+  __device__ __forceinline__ ACC at(int s, int) const { return s == kDiagSlot ? d : bit_select(m, s, slotv[s]); }
+  __device__ __forceinline__ ACC diag(const ValSrc<VT, ACC> &, int64_t) const { return d; }
+};
+
+template <class VT, class ACC, bool NT, uint32_t MASK>
+struct RowVals<kValsField, VT, ACC, NT, MASK> {
+  uint32_t m;
+  ACC d;
+  double ki;
+  const double *field;
+  __device__ __forceinline__ void load(const ValSrc<VT, ACC> &src, int64_t row) {
+    field = src.field;
+    if constexpr (NT) m = __builtin_nontemporal_load(src.mask + row);
+    else m = src.mask[row];
+    ki = field[row];
+    d = ld_val<ACC, NT>(src.vals + val_pos<val_width<VT>>(row, kDiagSlot));
+  }
+  __device__ __forceinline__ ACC at(int s, int c) const {
+    return s == kDiagSlot ? d : bit_select(m, s, (ACC)(-((ki + field[c]) * 0.5)));
+  }
+  __device__ __forceinline__ ACC diag(const ValSrc<VT, ACC> &, int64_t) const { return d; }
+};
+
 // Column index of (row, slot): the explicit 32-bit index, or the compact
 // form (ColForm) with a per-slice base.
 struct ColIdx {
@@ -222,6 +298,45 @@ inline ColIdx col_idx(const Ctx *c, const Level &L) {
   if (L.cbase && ((c->col_format == kColsCompact && L.read_compact) || c->col_format == kColsCompactAlways))
     return ColIdx{L.cols, L.cbase, L.cdelta, L.cform};
   return ColIdx{L.cols, nullptr, nullptr, nullptr};
+}
+
+// The value source and form of a launch.  The forms other than the stored
+// array go with the compact columns: with explicit columns a launch reads the
+// matrix as the reference stores it.
+template <class VT, class ACC>
+inline ValSrc<VT, ACC> val_src(const Level &L) {
+  ValSrc<VT, ACC> v{nullptr, L.vmask, nullptr, L.field, L.diag_one ? 1 : 0};
+  if constexpr (sizeof(VT) == 8) {
+    v.vals = L.vals;
+    v.slotv = L.slotv;
+  } else if constexpr (sizeof(VT) == 4) {
+    v.vals = L.vals32;
+    if (L.slotv) v.slotv = reinterpret_cast<const float *>(L.slotv + kSlots);
+  } else {
+    v.vals = L.vals16;
+    if (L.slotv) v.slotv = reinterpret_cast<const float *>(L.slotv + kSlots) + kSlots;
+  }
+  return v;
+}
+template <class VT>
+inline int val_form(const Level &L, const ColIdx &ci) {
+  if (!ci.cbase) return kValsStored;
+  // the scaled fp16 values are one per slot only if the diagonals they are scaled by are
+  if constexpr (sizeof(VT) == 2) return L.vform == kValsSlot && L.diag_one ? kValsSlot : kValsStored;
+  else if constexpr (sizeof(VT) == 4) return L.vform == kValsSlot ? kValsSlot : kValsStored;
+  else return L.vform;
+}
+
+// Runs f(CI, VF) with the column and value forms of a launch as constants.
+template <class VT, class F>
+inline void with_forms(const Level &L, const ColIdx &ci, F &&f) {
+  if (!ci.cbase) return f(std::false_type{}, std::integral_constant<int, kValsStored>{});
+  const int vf = val_form<VT>(L, ci);
+  if constexpr (sizeof(VT) == 8) {
+    if (vf == kValsField) return f(std::true_type{}, std::integral_constant<int, kValsField>{});
+  }
+  if (vf == kValsSlot) return f(std::true_type{}, std::integral_constant<int, kValsSlot>{});
+  f(std::true_type{}, std::integral_constant<int, kValsStored>{});
 }
 
 // Slice of a row.  UNI: the 64 lanes of the wave hold the 64 rows of one
@@ -466,24 +581,24 @@ __device__ __forceinline__ int64_t chunk_index(int j) {
 // sparse kernels (one thread per row, 4 slices per block)
 
 // y = A x over rows [0, nrows); ComputeSPMV_ref.cpp:61-70
-template <class VT, class XT, class ACC, bool CI>
+template <class VT, class XT, class ACC, bool CI, int VF>
 __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_spmv(const ColIdx ci,
-                                                 const VT *__restrict__ vals,
+                                                 const ValSrc<VT, ACC> src,
                                                  const XT *__restrict__ x, XT *__restrict__ y,
                                                  int64_t nrows) {
   const int64_t row = tile_id() * kBlock + threadIdx.x;
   if (row >= nrows) return;
   const size_t b = ell_base(row);
   const int slice = slice_of<true>(row);
-  ACC v[kSlots];
-  row_vals<ACC, true, kAllSlots>(vals, row, v);
+  RowVals<VF, VT, ACC, true, kAllSlots> v;
+  v.load(src, row);
   y[row] = (XT)with_cols<CI, true>(ci, slice, [&](auto cm, const int *base) {
     constexpr int CM = decltype(cm)::value;
     ACC sum = 0;
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
       const int c = col_at<CM, true>(ci, row, base, b, s);
-      sum += v[s] * (ACC)x[c];
+      sum += v.at(s, c) * (ACC)x[c];
     }
     return sum;
   });
@@ -527,18 +642,18 @@ static_assert(masks_keep_units(2) && masks_keep_units(4), "zero-start masks spli
 // first block of any order, general levels included.
 // GEN: general level, the diagonal's slot is dslot[row] (stencil: slot 13).
 // gs_row is the update of one row; it returns r_i * x_i (new) for the fused r.z.
-template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI, bool GEN, bool SAFE>
-__device__ __forceinline__ double gs_row(const ColIdx &ci, const VT *__restrict__ vals,
+template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI, int VF, bool GEN, bool SAFE>
+__device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC> &src,
                                          const XT *__restrict__ r, XT *__restrict__ x, int64_t row,
                                          const uint8_t *__restrict__ dslot) {
   constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
   const size_t b = ell_base(row);
   const int slice = slice_of<true>(row);
-  ACC vr[kSlots];
-  row_vals<ACC, FINE, mask>(vals, row, vr);
+  RowVals<VF, VT, ACC, FINE, mask> vr;
+  vr.load(src, row);
   ACC d;
-  if constexpr (!GEN && ((mask >> kDiagSlot) & 1u)) d = vr[kDiagSlot];
-  else d = ld_val<ACC, FINE>(vals + val_pos<val_width<VT>>(row, GEN ? (int)dslot[row] : kDiagSlot));
+  if constexpr (!GEN) d = vr.diag(src, row);
+  else d = ld_val<ACC, FINE>(src.vals + val_pos<val_width<VT>>(row, (int)dslot[row]));
   auto row_sum = [&](auto cm, const int *base) {
     constexpr int CM = decltype(cm)::value;
     ACC sum = (ACC)r[row];
@@ -546,7 +661,7 @@ __device__ __forceinline__ double gs_row(const ColIdx &ci, const VT *__restrict_
     for (int s = 0; s < kSlots; ++s) {
       if (!((mask >> s) & 1u)) continue;
       const int c = col_at<CM, FINE>(ci, row, base, b, s);
-      const ACC v = vr[s];
+      const ACC v = vr.at(s, c);
       const ACC xc = (ACC)x[c];
       // SAFE (from x = 0 into a vector that may hold anything): a zero entry (a neighbour
       // outside the grid) may point at a row not written yet in this sweep,
@@ -569,16 +684,17 @@ __device__ __forceinline__ double gs_row(const ColIdx &ci, const VT *__restrict_
 // post-smoother's last forward block and its backward steps); the block
 // also leaves its partial sum of r_i x_i in rz[blockIdx.x], so the solver's
 // r.z needs no pass of its own.
-template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI = false, bool GEN = false, bool RZ = false,
-          bool SAFE = false>
+template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI = false, int VF = kValsStored, bool GEN = false,
+          bool RZ = false, bool SAFE = false>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(1, SparseOccupancy<VT, CI, ZK < 0 ? kSlots : __builtin_popcount(swept_before_mask(ZK))>::max_waves)))
-void k_gs(const ColIdx ci, const VT *__restrict__ vals,
+void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
                                                const XT *__restrict__ r, XT *__restrict__ x,
                                                int64_t row0, int64_t nrows,
                                                const uint8_t *__restrict__ dslot, double *rz = nullptr) {
   static_assert(!GEN || ZK <= 0, "general levels: full rows, or the first block from x = 0 (diagonal only)");
   static_assert(!RZ || ZK < 0, "r.z is taken from the post-smoother");
+  static_assert(VF == kValsStored || (CI && !GEN), "value forms: stencil levels with compact columns");
   // blocks of 256 threads, or of 64 for the small coarse fp64 steps (one wave
   // per block spreads them over more CUs); the r.z form always takes 256
 #ifndef HPCGX_FINE_ROT
@@ -588,21 +704,21 @@ void k_gs(const ColIdx ci, const VT *__restrict__ vals,
   if constexpr (RZ) {
     // every thread reaches the block reduction; rows past the block add 0
     double acc = 0.0;
-    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CI, GEN, SAFE>(ci, vals, r, x, row0 + t, dslot);
+    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CI, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
     const double v[1] = {acc};
     block_partials<1>(v, rz);
     return;
   }
   if (t >= nrows) return;
-  gs_row<VT, XT, ACC, ZK, FINE, CI, GEN, SAFE>(ci, vals, r, x, row0 + t, dslot);
+  gs_row<VT, XT, ACC, ZK, FINE, CI, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
 }
 
 // Residual at the injected rows and restriction, fused (ComputeMG_ref.cpp:49-51 +
 // ComputeRestriction_ref.cpp:51): rc[inj[t]] = r_f - (A x)_f for the t-th
 // injected row f = row0 + t (frow[t] when frow is given).  (A x)_f is summed
 // from 0 like SpMV, then subtracted.  SCALE: fp16 V-cycle, times sigma[t].
-template <class VT, class XT, class ACC, bool SCALE, bool CI = false>
-__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_restrict(const ColIdx ci, const VT *__restrict__ vals,
+template <class VT, class XT, class ACC, bool SCALE, bool CI, int VF>
+__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_restrict(const ColIdx ci, const ValSrc<VT, ACC> src,
                                                      const XT *__restrict__ r,
                                                      const XT *__restrict__ x,
                                                      XT *__restrict__ rc, const int *__restrict__ inj,
@@ -612,15 +728,15 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_restr
   if (t >= count) return;
   const int64_t row = frow ? (int64_t)frow[t] : row0 + t;
   const size_t b = ell_base(row);
-  ACC v[kSlots];
-  row_vals<ACC, true, kAllSlots>(vals, row, v);
+  RowVals<VF, VT, ACC, true, kAllSlots> v;
+  v.load(src, row);
   auto row_ax = [&](auto cm, const int *base) {
     constexpr int CM = decltype(cm)::value;
     ACC ax = 0;
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
       const int c = col_at<CM, true>(ci, row, base, b, s);
-      ax += v[s] * (ACC)x[c];
+      ax += v.at(s, c) * (ACC)x[c];
     }
     return ax;
   };

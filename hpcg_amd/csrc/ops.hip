@@ -10,19 +10,10 @@ namespace hpcgx {
 
 static inline unsigned tiles(int64_t rows) { return (unsigned)((rows + kBlock - 1) / kBlock); }
 
-template <class VT>
-static const VT *vals_of(const Level &L);
-template <>
-const double *vals_of<double>(const Level &L) { return L.vals; }
-template <>
-const float *vals_of<float>(const Level &L) { return L.vals32; }
-template <>
-const __half *vals_of<__half>(const Level &L) { return L.vals16; }
-
 // rz (fp64 stencil levels only): the step also leaves the partials of r.x
 // over its rows there, tiles(rows) of them.
 template <class VT, class XT, class ACC, int ZK, bool FINE, bool SAFE = false>
-static void gs_block(Ctx *c, const Level &L, const VT *v, const XT *r, XT *x, int k, double *rz = nullptr) {
+static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *rz = nullptr) {
   const int64_t r0 = L.lay.start[k], nr = L.lay.start[k + 1] - r0;
   if (nr <= 0) return;
   const ColIdx ci = col_idx(c, L);
@@ -41,43 +32,42 @@ static void gs_block(Ctx *c, const Level &L, const VT *v, const XT *r, XT *x, in
   const unsigned bs = (!FINE && sizeof(VT) == 8 && nr < (int64_t)(HPCGX_ONE_WAVE_ROWS)) ? kSlice : kBlock;
   const unsigned g = (unsigned)((nr + bs - 1) / bs);
   hipStream_t st = c->stream;
+  const ValSrc<VT, ACC> v = val_src<VT, ACC>(L);
   if constexpr (ZK < 0 && sizeof(VT) == 8 && sizeof(XT) == 8) {
     if (rz) {
       // 256-thread blocks: the partials are per block of 4 waves, tiles(nr) of them
-      if (ci.cbase)
-        k_gs<VT, XT, ACC, -1, FINE, true, false, true><<<tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, nullptr, rz);
-      else
-        k_gs<VT, XT, ACC, -1, FINE, false, false, true><<<tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, nullptr, rz);
+      with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+        k_gs<VT, XT, ACC, -1, FINE, CI(), VF(), false, true><<<tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, nullptr, rz);
+      });
       return;
     }
   }
   if constexpr (ZK <= 0) {  // general levels: full rows, or the first block from x = 0
     if (L.dslot) {
       if (ci.cbase)
-        k_gs<VT, XT, ACC, ZK, FINE, true, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
+        k_gs<VT, XT, ACC, ZK, FINE, true, kValsStored, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
       else
-        k_gs<VT, XT, ACC, ZK, FINE, false, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
+        k_gs<VT, XT, ACC, ZK, FINE, false, kValsStored, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
       return;
     }
   }
-  if (ci.cbase)
-    k_gs<VT, XT, ACC, ZK, FINE, true, false, false, SAFE><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
-  else
-    k_gs<VT, XT, ACC, ZK, FINE, false, false, false, SAFE><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
+  with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+    k_gs<VT, XT, ACC, ZK, FINE, CI(), VF(), false, false, SAFE><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
+  });
 }
 
 // The zero-start forward sweep of the default order: block k reads only the
 // blocks swept before it.
 template <class VT, class XT, class ACC, bool FINE, bool SAFE>
-static void zero_start_forward(Ctx *c, const Level &L, const VT *v, const XT *r, XT *x) {
-  gs_block<VT, XT, ACC, 0, FINE, SAFE>(c, L, v, r, x, 0);
-  gs_block<VT, XT, ACC, 1, FINE, SAFE>(c, L, v, r, x, 1);
-  gs_block<VT, XT, ACC, 2, FINE, SAFE>(c, L, v, r, x, 2);
-  gs_block<VT, XT, ACC, 3, FINE, SAFE>(c, L, v, r, x, 3);
-  gs_block<VT, XT, ACC, 4, FINE, SAFE>(c, L, v, r, x, 4);
-  gs_block<VT, XT, ACC, 5, FINE, SAFE>(c, L, v, r, x, 5);
-  gs_block<VT, XT, ACC, 6, FINE, SAFE>(c, L, v, r, x, 6);
-  gs_block<VT, XT, ACC, 7, FINE, SAFE>(c, L, v, r, x, 7);
+static void zero_start_forward(Ctx *c, const Level &L, const XT *r, XT *x) {
+  gs_block<VT, XT, ACC, 0, FINE, SAFE>(c, L, r, x, 0);
+  gs_block<VT, XT, ACC, 1, FINE, SAFE>(c, L, r, x, 1);
+  gs_block<VT, XT, ACC, 2, FINE, SAFE>(c, L, r, x, 2);
+  gs_block<VT, XT, ACC, 3, FINE, SAFE>(c, L, r, x, 3);
+  gs_block<VT, XT, ACC, 4, FINE, SAFE>(c, L, r, x, 4);
+  gs_block<VT, XT, ACC, 5, FINE, SAFE>(c, L, r, x, 5);
+  gs_block<VT, XT, ACC, 6, FINE, SAFE>(c, L, r, x, 6);
+  gs_block<VT, XT, ACC, 7, FINE, SAFE>(c, L, r, x, 7);
 }
 
 template <class XT>
@@ -109,22 +99,21 @@ static bool default_order(const Level &L) {
 template <class VT, class XT, class ACC, bool FINE>
 static void sweep(Ctx *c, const Level &L, const XT *r, XT *x, bool zero_start, double *rz = nullptr,
                   int64_t *nrz = nullptr, bool untrusted_x = false) {
-  const VT *v = vals_of<VT>(L);
   if (zero_start && !default_order(L)) {
     k_zero<XT><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(x, L.lay.npad);
-    gs_block<VT, XT, ACC, 0, FINE>(c, L, v, r, x, 0);
-    for (int k = 1; k < L.lay.ncol; ++k) gs_block<VT, XT, ACC, -1, FINE>(c, L, v, r, x, k);
+    gs_block<VT, XT, ACC, 0, FINE>(c, L, r, x, 0);
+    for (int k = 1; k < L.lay.ncol; ++k) gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, k);
   } else if (zero_start) {
-    if (untrusted_x) zero_start_forward<VT, XT, ACC, FINE, true>(c, L, v, r, x);
-    else zero_start_forward<VT, XT, ACC, FINE, false>(c, L, v, r, x);
+    if (untrusted_x) zero_start_forward<VT, XT, ACC, FINE, true>(c, L, r, x);
+    else zero_start_forward<VT, XT, ACC, FINE, false>(c, L, r, x);
   } else {
-    for (int k = 0; k + 1 < L.lay.ncol; ++k) gs_block<VT, XT, ACC, -1, FINE>(c, L, v, r, x, k);
+    for (int k = 0; k + 1 < L.lay.ncol; ++k) gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, k);
     const int last = L.lay.ncol - 1;
-    gs_block<VT, XT, ACC, -1, FINE>(c, L, v, r, x, last, rz);
+    gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, last, rz);
     if (rz) rz += tiles(L.lay.start[last + 1] - L.lay.start[last]);
   }
   for (int k = L.lay.ncol - 2; k >= 0; --k) {
-    gs_block<VT, XT, ACC, -1, FINE>(c, L, v, r, x, k, rz);
+    gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, k, rz);
     if (rz) rz += tiles(L.lay.start[k + 1] - L.lay.start[k]);
   }
   if (nrz) {
@@ -166,12 +155,10 @@ static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64
   }
   const int64_t nc = L.ninj, r0 = L.lay.start[L.lay.inj];
   const ColIdx ci = col_idx(c, L);
-  if (ci.cbase)
-    k_restrict<VT, XT, ACC, SCALE, true><<<tiles(nc), kBlock, 0, c->stream>>>(ci, vals_of<VT>(L), r, x, rc_v,
-                                                                             L.inj, L.sigma, r0, nc, L.frow);
-  else
-    k_restrict<VT, XT, ACC, SCALE, false><<<tiles(nc), kBlock, 0, c->stream>>>(ci, vals_of<VT>(L), r, x, rc_v,
-                                                                              L.inj, L.sigma, r0, nc, L.frow);
+  with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+    k_restrict<VT, XT, ACC, SCALE, CI(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
+        ci, val_src<VT, ACC>(L), r, x, rc_v, L.inj, L.sigma, r0, nc, L.frow);
+  });
   HPCGX_CHECK_LAUNCH(c);
   // the coarse level's x may hold anything: a V-cycle on a non-finite input
   // leaves non-finite values in the context's coarse vectors
@@ -299,10 +286,10 @@ __global__ __launch_bounds__(kBlock) void k_to_double(const float *__restrict__ 
 int spmv_fp64(Ctx *c, int level, const double *x, double *y) {
   const Level &L = c->levels[level];
   const ColIdx ci = col_idx(c, L);
-  if (ci.cbase)
-    k_spmv<double, double, double, true><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(ci, L.vals, x, y, L.lay.npad);
-  else
-    k_spmv<double, double, double, false><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(ci, L.vals, x, y, L.lay.npad);
+  with_forms<double>(L, ci, [&](auto CI, auto VF) {
+    k_spmv<double, double, double, CI(), VF()><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(
+        ci, val_src<double, double>(L), x, y, L.lay.npad);
+  });
   HPCGX_CHECK_LAUNCH(c);
   return HPCGX_OK;
 }
@@ -402,12 +389,10 @@ int hpcgx_restrict(hpcgx_ctx *c, int level, const double *r, const double *x, do
   const Level &L = c->levels[level];
   const int64_t nc = L.ninj;
   const ColIdx ci = col_idx(c, L);
-  if (ci.cbase)
-    k_restrict<double, double, double, false, true><<<tiles(nc), kBlock, 0, c->stream>>>(
-        ci, L.vals, r, x, rc_out, L.inj, nullptr, L.lay.start[L.lay.inj], nc, L.frow);
-  else
-    k_restrict<double, double, double, false, false><<<tiles(nc), kBlock, 0, c->stream>>>(
-        ci, L.vals, r, x, rc_out, L.inj, nullptr, L.lay.start[L.lay.inj], nc, L.frow);
+  with_forms<double>(L, ci, [&](auto CI, auto VF) {
+    k_restrict<double, double, double, false, CI(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
+        ci, val_src<double, double>(L), r, x, rc_out, L.inj, nullptr, L.lay.start[L.lay.inj], nc, L.frow);
+  });
   HPCGX_CHECK_LAUNCH(c);
   return HPCGX_OK;
 }

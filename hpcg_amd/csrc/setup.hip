@@ -174,6 +174,14 @@ int ensure_stage(Ctx *c, int64_t n) {
   return HPCGX_OK;
 }
 
+// One allocation per level for the forms: the slot values (27 in fp64, 27
+// each for the fp32 and fp16 copies as fp32, padded to 512 bytes), the row
+// masks and the slices' column forms.
+constexpr size_t kSlotvBytes = 512;
+static size_t form_bytes(const Level &L) {
+  return kSlotvBytes + L.lay.npad * sizeof(uint32_t) + (size_t)(L.lay.npad / kSlice);
+}
+
 static void free_level(Ctx *c, Level &L) {
   const size_t m = (size_t)L.lay.npad * kSlots;
   dfree(c, L.cols, m * sizeof(int));
@@ -182,7 +190,8 @@ static void free_level(Ctx *c, Level &L) {
   dfree(c, L.vals16, m * sizeof(__half));
   dfree(c, L.cbase, (size_t)(L.lay.npad / kSlice) * kMeta * sizeof(int));
   dfree(c, L.cdelta, m * sizeof(int8_t));
-  dfree(c, L.cform, (size_t)(L.lay.npad / kSlice));
+  dfree(c, L.slotv, form_bytes(L));  // with vmask and cform
+  dfree(c, L.field, L.lay.npad * sizeof(double));
   dfree(c, L.dinv, L.lay.npad * sizeof(float));
   dfree(c, L.sigma, L.ninj * sizeof(float));
   dfree(c, L.perm, L.lay.n * sizeof(int));
@@ -243,7 +252,8 @@ __global__ __launch_bounds__(kBlock) void k_fill(double *__restrict__ v, const i
 __global__ __launch_bounds__(kBlock) void k_generate(LayoutDev L, int64_t npad, int *__restrict__ cols,
                                                      double *__restrict__ vals,
                                                      int *__restrict__ iperm, int *__restrict__ perm,
-                                                     const double *__restrict__ kappa, bool values) {
+                                                     const double *__restrict__ kappa, bool values,
+                                                     double *__restrict__ field) {
   const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (p >= npad) return;
   int k = 0;
@@ -253,6 +263,7 @@ __global__ __launch_bounds__(kBlock) void k_generate(LayoutDev L, int64_t npad, 
   const size_t b = ell_base(p);
   if (idx >= (int64_t)nbx * nby * nbz) {  // padding: identity row
     iperm[p] = -1;
+    if (field) field[p] = 0.0;
     for (int s = 0; s < kSlots; ++s) {
       cols[b + s * kSlice] = (int)p;
       vals[val_pos<2>(p, s)] = s == kDiagSlot ? 1.0 : 0.0;
@@ -267,6 +278,7 @@ __global__ __launch_bounds__(kBlock) void k_generate(LayoutDev L, int64_t npad, 
   iperm[p] = (int)i;
   perm[i] = (int)p;
   const double ki = kappa ? kappa[i] : 1.0;
+  if (field) field[p] = ki;
   int nn = 0;
   double dsum = 0.0;
   for (int s = 0; s < kSlots; ++s) {
@@ -477,7 +489,8 @@ static int pack_stencil_device(Ctx *c, Level &L, RowAcc rows, bool *stencil) {
   int64_t hpcg_nnz = 0;
   if (rows_are_hpcg(rows, lay, &hpcg_nnz)) {
     if ((rc = alloc_level(c, L))) return rc;
-    k_generate<<<nblk(npad), kBlock, 0, c->stream>>>(L.ldev, npad, L.cols, L.vals, L.iperm, L.perm, nullptr, true);
+    k_generate<<<nblk(npad), kBlock, 0, c->stream>>>(L.ldev, npad, L.cols, L.vals, L.iperm, L.perm, nullptr, true,
+                                                      nullptr);
     HPCGX_CHECK_LAUNCH(c);
     L.perm_h.resize(n);
     L.iperm_h.resize(npad);
@@ -489,7 +502,8 @@ static int pack_stencil_device(Ctx *c, Level &L, RowAcc rows, bool *stencil) {
     return HPCGX_OK;
   }
   if ((rc = ensure_upload_staging(c)) || (rc = alloc_level(c, L))) return rc;
-  k_generate<<<nblk(npad), kBlock, 0, c->stream>>>(L.ldev, npad, L.cols, L.vals, L.iperm, L.perm, nullptr, false);
+  k_generate<<<nblk(npad), kBlock, 0, c->stream>>>(L.ldev, npad, L.cols, L.vals, L.iperm, L.perm, nullptr, false,
+                                                    nullptr);
   HPCGX_CHECK_LAUNCH(c);
   HPCGX_HIP(c, hipMemsetAsync(c->up_err, 0, 64 * sizeof(int), c->stream));
   std::atomic<int64_t> nnz(0);
@@ -1054,6 +1068,14 @@ __global__ void k_sigma(const double *__restrict__ fvals, const uint8_t *__restr
   sigma[t] = (float)sqrt(df / dc);
 }
 
+// Whether a row's diagonal is not what kValsSlot's diagonal gives: the slot's
+// value on a row of the level, 1 on padding.  A diagonal that is not positive
+// is left to the stored form (the scaled copy divides by its root).
+__device__ __forceinline__ bool diag_differs(double d, bool real, double slot_diag) {
+  if (!real) return d != 1.0;
+  return !(slot_diag > 0.0) || __double_as_longlong(d) != __double_as_longlong(slot_diag);
+}
+
 // Compact column indices, one wave per 64-row slice.  For each slot the
 // columns of the rows with a nonzero value (and of the diagonal, whatever its
 // value) are base + lane + d with d in [-128, 127]; a zero-valued slot
@@ -1065,11 +1087,21 @@ __global__ void k_sigma(const double *__restrict__ fvals, const uint8_t *__restr
 // take base + lane (a row of the level), is uniform: base + lane is its
 // column, with no per-entry index.  The form depends only on the columns and
 // on which entries are zero, never on the matrix being a stencil.
+//
+// vmask given (stencil levels): the pass also writes the row masks of the
+// value forms and checks every stored value against both forms, bit for bit:
+// against slotv[s] (kValsSlot), the diagonal apart, and with a field given
+// against -((k_i + k_j) * 0.5) (kValsField).  A mismatch raises the form's
+// flag.  An entry stored as -0 counts as no entry for the columns and as one
+// for the values, so it rules both forms out.
 __global__ __launch_bounds__(kBlock) void k_compact_cols(const int *__restrict__ cols,
                                                          const double *__restrict__ vals,
                                                          const uint8_t *__restrict__ dslot,
                                                          int *__restrict__ cbase, int8_t *__restrict__ cdelta,
-                                                         uint8_t *__restrict__ cform, int64_t nslices, int64_t npad) {
+                                                         uint8_t *__restrict__ cform, int64_t nslices, int64_t npad,
+                                                         const int *__restrict__ iperm, const double *__restrict__ slotv,
+                                                         const double *__restrict__ field, uint32_t *__restrict__ vmask,
+                                                         int *flags) {
   const int lane = threadIdx.x & 63;
   const int64_t slice = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
   if (slice >= nslices) return;
@@ -1077,9 +1109,19 @@ __global__ __launch_bounds__(kBlock) void k_compact_cols(const int *__restrict__
   const size_t b = (size_t)slice * (kSlots * kSlice) + lane;
   const int ds = dslot ? dslot[row] : kDiagSlot;
   bool wide = false, uniform = true;
+  uint32_t mask = 0;
+  bool bad_slot = false, bad_field = false;
+  const double ki = vmask && field ? field[row] : 0.0;
   for (int s = 0; s < kSlots; ++s) {
     const int col = cols[b + s * kSlice];
-    const bool live = vals[val_pos<2>(row, s)] != 0.0 || s == ds;
+    const double a = vals[val_pos<2>(row, s)];
+    const bool live = a != 0.0 || s == ds;
+    if (vmask && s != ds) {
+      const long long bits = __double_as_longlong(a);
+      if (bits != 0) mask |= 1u << s;
+      bad_slot |= bits != 0 && (!live || bits != __double_as_longlong(slotv[s]));
+      if (field) bad_field |= bits != 0 && (!live || bits != __double_as_longlong(-((ki + field[col]) * 0.5)));
+    }
     int lo = live ? col - lane : INT_MAX, hi = live ? col - lane : INT_MIN;
     for (int m = 32; m >= 1; m >>= 1) {
       lo = min(lo, __shfl_xor(lo, m, 64));
@@ -1110,34 +1152,120 @@ __global__ __launch_bounds__(kBlock) void k_compact_cols(const int *__restrict__
   const int form = any_wide ? kFormWide : all_uniform ? kFormUniform : kFormDelta;
   if (lane == 0) cform[slice] = (uint8_t)form;
   if (lane < kMeta - kSlots) cbase[slice * kMeta + kSlots + lane] = lane == 0 ? form : 0;  // the form, then padding
+  if (lane == 0 && form == kFormWide) atomicAdd(&flags[kWideSlices], 1);
+  if (!vmask) return;
+  const bool real = iperm[row] >= 0;
+  if (real) mask |= 1u << kDiagSlot;
+  vmask[row] = mask;
+  const bool bad_diag = diag_differs(vals[val_pos<2>(row, kDiagSlot)], real, slotv[kDiagSlot]);
+  const bool bs = __any(bad_slot), bd = __any(bad_diag), bf = !field || __any(bad_field);
+  // a flag already up is not raised again: on a level without the form every wave would queue on it
+  if (lane == 0) {
+    if (bs && !__hip_atomic_load(&flags[kBadSlot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&flags[kBadSlot], 1);
+    if (bd && !__hip_atomic_load(&flags[kBadDiag], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&flags[kBadDiag], 1);
+    if (bf && !__hip_atomic_load(&flags[kBadField], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&flags[kBadField], 1);
+  }
 }
 
-static int build_compact_cols(Ctx *c, Level &L) {
-  if (L.cbase) return HPCGX_OK;
+// The diagonals alone, after they were replaced.
+__global__ __launch_bounds__(kBlock) void k_check_diag(const double *__restrict__ vals, const uint32_t *__restrict__ vmask,
+                                                       const double *__restrict__ slotv, int64_t npad, int *flags) {
+  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const bool bad = p < npad && diag_differs(vals[val_pos<2>(p, kDiagSlot)], (vmask[p] >> kDiagSlot) & 1u, slotv[kDiagSlot]);
+  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(&flags[kBadDiag], 1);
+}
+
+// The candidate value of each slot: the first stored entry met in that slot
+// among 32 rows spread over each colour block (all rows of a small block; a
+// slot that they all miss keeps +0).  k_compact_cols then checks every row.
+// One workgroup, a row per thread; also clears the flags and derives the slot
+// values of the lower-precision copies with the roundings of k_to_f32 and
+// k_to_f16_scaled.
+constexpr int kSampleRows = 32;
+__global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(LayoutDev L, const double *__restrict__ vals,
+                                                                        double *slotv, int *flags) {
+  __shared__ int first[kSlots];
+  const int t = threadIdx.x;
+  if (t < kSlots) first[t] = INT_MAX;
+  if (t < kFormFlags) flags[t] = 0;
+  __syncthreads();
+  const int k = t / kSampleRows, i = t % kSampleRows;
+  const int64_t count = (int64_t)L.nb[k][0] * L.nb[k][1] * L.nb[k][2];
+  const bool in = i < count;
+  // evenly spaced and shifted by one row each, so the samples of a block do
+  // not all lie at the same x
+  const int64_t p = L.start[k] + (count <= kSampleRows ? (in ? i : 0) : (count / kSampleRows * i + i) % count);
+  double v[kSlots];
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) v[s] = in ? vals[val_pos<2>(p, s)] : 0.0;
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    const unsigned long long b = __ballot(v[s] != 0.0);
+    if (b && __builtin_ctzll(b) == (t & 63)) atomicMin(&first[s], (int)p);
+  }
+  __syncthreads();
+  if (t >= kSlots) return;
+  const double a = first[t] == INT_MAX ? 0.0 : vals[val_pos<2>(first[t], t)];
+  const double d = first[kDiagSlot] == INT_MAX ? 1.0 : vals[val_pos<2>(first[kDiagSlot], kDiagSlot)];
+  const double di = 1.0 / sqrt(d);
+  slotv[t] = a;
+  float *lo = reinterpret_cast<float *>(slotv + kSlots);
+  lo[t] = (float)a;
+  lo[kSlots + t] = __half2float(__float2half_rn((float)(t == kDiagSlot ? 1.0 : a * di * di)));
+}
+__global__ void k_clear_flags(int *flags) {
+  if (threadIdx.x < kFormFlags) flags[threadIdx.x] = 0;
+}
+
+// Launches the building of a level's compact columns and value forms; the
+// flags come back in read_forms.
+static int build_compact_cols(Ctx *c, Level &L, int *flags) {
   const int64_t ns = L.lay.npad / kSlice;
   int rc;
   if ((rc = dalloc(c, (void **)&L.cbase, (size_t)ns * kMeta * sizeof(int), false))) return rc;
   if ((rc = dalloc(c, (void **)&L.cdelta, (size_t)L.lay.npad * kSlots * sizeof(int8_t), false))) return rc;
-  if ((rc = dalloc(c, (void **)&L.cform, (size_t)ns, false))) return rc;
+  if ((rc = dalloc(c, (void **)&L.slotv, form_bytes(L), false))) return rc;
+  uint32_t *mask = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(L.slotv) + kSlotvBytes);
+  L.cform = reinterpret_cast<uint8_t *>(mask + L.lay.npad);
+  if (!L.lay.general) {
+    L.vmask = mask;
+    k_slot_values<<<1, kColours * kSampleRows, 0, c->stream>>>(L.ldev, L.vals, L.slotv, flags);
+  } else {
+    k_clear_flags<<<1, 64, 0, c->stream>>>(flags);
+  }
+  HPCGX_CHECK_LAUNCH(c);
   const int64_t grid = (ns + (kBlock / kSlice) - 1) / (kBlock / kSlice);
   k_compact_cols<<<grid, kBlock, 0, c->stream>>>(L.cols, L.vals, L.dslot, L.cbase, L.cdelta, L.cform, ns,
-                                                 L.lay.npad);
+                                                 L.lay.npad, L.iperm, L.slotv, L.field, L.vmask, flags);
   HPCGX_CHECK_LAUNCH(c);
-  std::vector<uint8_t> f(ns);
-  HPCGX_HIP(c, hipMemcpyAsync(f.data(), L.cform, ns, hipMemcpyDeviceToHost, c->stream));
-  HPCGX_HIP(c, hipStreamSynchronize(c->stream));
-  int64_t wide = 0;
-  for (const uint8_t v : f) wide += v == kFormWide;
-  L.read_compact = 2 * wide < ns;
   return HPCGX_OK;
 }
 
-// The compact index copies of every level (the default column format).
+// The compact index copies (the default column format) and value forms of
+// every level, with one wait for the host.
 static int build_compact_all(Ctx *c) {
   if (c->col_format == kColsExplicit) return HPCGX_OK;
-  for (auto &L : c->levels) {
-    int rc = build_compact_cols(c, L);
+  int *dev = reinterpret_cast<int *>(c->scal + S_COUNT);
+  bool built[kMaxLevels] = {};
+  const int nl = (int)c->levels.size();
+  for (int l = 0; l < nl; ++l) {
+    Level &L = c->levels[l];
+    if (L.cbase) continue;
+    int rc = build_compact_cols(c, L, dev + l * kFormFlags);
     if (rc) return rc;
+    built[l] = true;
+  }
+  int *flags = reinterpret_cast<int *>(c->hbuf);
+  HPCGX_HIP(c, hipMemcpyAsync(flags, dev, kMaxLevels * kFormFlags * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  HPCGX_HIP(c, hipStreamSynchronize(c->stream));
+  for (int l = 0; l < nl; ++l) {
+    if (!built[l]) continue;
+    Level &L = c->levels[l];
+    const int *f = flags + l * kFormFlags;
+    L.read_compact = 2 * (int64_t)f[kWideSlices] < L.lay.npad / kSlice;
+    if (!L.vmask) continue;
+    L.vform = !f[kBadSlot] ? kValsSlot : !f[kBadField] ? kValsField : kValsStored;
+    L.diag_one = L.vform == kValsSlot && !f[kBadDiag];
   }
   return HPCGX_OK;
 }
@@ -1238,7 +1366,7 @@ int hpcgx_create(int device, hpcgx_ctx **out) {
   c->stream = c->own_stream;
   int rc;
   if ((rc = noalloc_scratch_init(device)) || (rc = ensure_reduce(c, 4096)) ||
-      (rc = dalloc(c, (void **)&c->scal, S_COUNT * sizeof(double)))) {
+      (rc = dalloc(c, (void **)&c->scal, S_COUNT * sizeof(double) + kMaxLevels * kFormFlags * sizeof(int)))) {
     hpcgx_destroy(c);
     return rc;
   }
@@ -1350,6 +1478,7 @@ int hpcgx_problem_generate(hpcgx_ctx *c, int nx, int ny, int nz, int levels, con
     if (L.lay.npad >= ((int64_t)1 << 31)) return set_err(c, HPCGX_EINVAL, "problem_generate: too many rows for 32-bit columns");
     if ((rc = alloc_level(c, L))) return rc;
     if (kappa) {
+      if ((rc = dalloc(c, (void **)&L.field, L.lay.npad * sizeof(double), false))) return rc;
       if ((rc = dalloc(c, (void **)&kdev, L.lay.n * sizeof(double), false))) return rc;
       if (l == 0) {
         HPCGX_HIP(c, hipMemcpy(kdev, kappa, L.lay.n * sizeof(double), hipMemcpyHostToDevice));
@@ -1361,7 +1490,7 @@ int hpcgx_problem_generate(hpcgx_ctx *c, int nx, int ny, int nz, int levels, con
       }
     }
     k_generate<<<nblk(L.lay.npad), kBlock, 0, c->stream>>>(L.ldev, L.lay.npad, L.cols, L.vals, L.iperm,
-                                                          L.perm, kdev, true);
+                                                          L.perm, kdev, true, L.field);
     HPCGX_CHECK_LAUNCH(c);
     int64_t nnz = 1;
     for (const int d : {L.lay.nx, L.lay.ny, L.lay.nz}) nnz *= (int64_t)(3 * d - 2);
@@ -1463,6 +1592,15 @@ int hpcgx_level_set_diagonal(hpcgx_ctx *c, int level, const double *diag) {
   HPCGX_HIP(c, hipMemcpyAsync(c->stage, diag, L.lay.n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   k_set_diag<<<nblk(L.lay.n), kBlock, 0, c->stream>>>(L.vals, L.dslot, L.perm, c->stage, L.lay.n);
   HPCGX_CHECK_LAUNCH(c);
+  if (L.vform == kValsSlot) {  // one value on every row, or read from the array from now on
+    int *flags = reinterpret_cast<int *>(c->scal + S_COUNT), *bad = reinterpret_cast<int *>(c->hbuf);
+    k_clear_flags<<<1, 64, 0, c->stream>>>(flags);
+    k_check_diag<<<nblk(L.lay.npad), kBlock, 0, c->stream>>>(L.vals, L.vmask, L.slotv, L.lay.npad, flags);
+    HPCGX_CHECK_LAUNCH(c);
+    HPCGX_HIP(c, hipMemcpyAsync(bad, flags, kFormFlags * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HPCGX_HIP(c, hipStreamSynchronize(c->stream));
+    L.diag_one = !bad[kBadDiag];
+  }
   HPCGX_HIP(c, hipStreamSynchronize(c->stream));
   // the lower-precision copies (and the fp16 scaling) follow the new diagonal
   const int prepared = c->prepared;
