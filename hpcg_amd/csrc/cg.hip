@@ -142,6 +142,33 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CI) void k_c
   block_partials<1>(v, partials);
 }
 
+// The same by row runs, with the same partials in the same places.
+template <int VF>
+__global__ __launch_bounds__(kBlock) void k_cg_spmv_dot_run(const ColIdx ci, const ValSrc<double, double> src,
+                                                            const double *__restrict__ p, double *__restrict__ Ap,
+                                                            int64_t nrows, double *partials, int bt) {
+  const int64_t tile = level_tile(bt);
+  RunWave w;
+  w.init(ci, 0, nrows, tile);
+  double ax[2], acc[2] = {0.0, 0.0};
+  run_ax<VF>(ci, src, w, p, ax);
+  if (w.active) {
+    double pv[2];
+    ld_pair(p + w.lane_row(0), pv);
+    st_pair(Ap + w.lane_row(0), ax);
+    acc[0] = pv[0] * ax[0];
+    acc[1] = pv[1] * ax[1];
+  } else if (!w.run) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (w.has_row(j)) {
+        Ap[w.lane_row(j)] = ax[j];
+        acc[j] = p[w.lane_row(j)] * ax[j];
+      }
+  }
+  run_partials<false>(w, acc, tile, (nrows + kBlock - 1) / kBlock, partials);
+}
+
 // x += alpha p ; r -= alpha Ap ; normr2 = r.r
 // R32: also leave r in fp32 for the next mixed-precision V-cycle, times
 // rscale[i] when given (the scaled fp16 V-cycle's input dinv_i r_i, rounded
@@ -305,6 +332,22 @@ __global__ __launch_bounds__(kBlock) void k_kappa_grad(const int *__restrict__ c
   g[p] = -0.5 * acc - (double)(26 - nn) * lp * xp;
 }
 
+static void cg_spmv_dot(Ctx *c, const Level &L, const double *p, double *Ap) {
+  const ColIdx ci = col_idx(c, L);
+  const int64_t np = L.lay.npad;
+  const ValSrc<double, double> src = val_src<double, double>(L);
+  with_forms<double>(L, ci, [&](auto CI, auto VF) {
+    if constexpr (VF() != kValsStored) {
+      if (run_rows(L, np)) {
+        k_cg_spmv_dot_run<VF()><<<run_tiles(np), kBlock, 0, c->stream>>>(ci, src, p, Ap, np, c->partials,
+                                                                        block_tiles(L));
+        return;
+      }
+    }
+    k_cg_spmv_dot<CI(), VF()><<<tiles(np), kBlock, 0, c->stream>>>(ci, src, p, Ap, np, c->partials);
+  });
+}
+
 static double now_s() {
   using namespace std::chrono;
   return duration<double>(steady_clock::now().time_since_epoch()).count();
@@ -372,7 +415,6 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
   int rc;
   PhaseTimer tm{c, times != nullptr};
   const bool fuse_rz = precond && c->levels.size() > 1 && !L0.lay.general;
-  const ColIdx ci0 = col_idx(c, L0);
   // preamble: Ap = A x ; r = b - Ap ; normr = ||r||  (CG.cpp:86-90)
   if ((rc = spmv_fp64(c, 0, x, Ap))) return rc;
   k_cg_residual<false><<<G, kBlock, 0, c->stream>>>(np, b, Ap, r, nullptr, c->partials);
@@ -420,9 +462,7 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
       else
         k_cg_px<false><<<tiles(np), kBlock, 0, c->stream>>>(np, z, p, x, c->scal, j == 1);
       tm.mark(3);
-      with_forms<double>(L0, ci0, [&](auto CI, auto VF) {
-        k_cg_spmv_dot<CI(), VF()><<<T, kBlock, 0, c->stream>>>(ci0, val_src<double, double>(L0), p, Ap, np, c->partials);
-      });
+      cg_spmv_dot(c, L0, p, Ap);
       if ((rc = finish(c, 1, T, F_PAP))) return rc;
       tm.mark(4);
       k_cg_update_r<<<G, kBlock, 0, c->stream>>>(np, r, Ap, c->partials, c->scal);
@@ -515,10 +555,7 @@ static int cg_mixed(Ctx *c, int variant, const double *b, double *x, int max_ite
       k_cg_p<float><<<tiles(np), kBlock, 0, c->stream>>>(np, z32, p, c->scal, 0, dscale);
     restart = false;
     tm.mark(3);
-    const ColIdx ci0 = col_idx(c, L0);
-    with_forms<double>(L0, ci0, [&](auto CI, auto VF) {
-      k_cg_spmv_dot<CI(), VF()><<<T, kBlock, 0, c->stream>>>(ci0, val_src<double, double>(L0), p, Ap, np, c->partials);
-    });
+    cg_spmv_dot(c, L0, p, Ap);
     if ((rc = finish(c, 1, T, F_PAP))) return rc;
     tm.mark(4);
     k_cg_update<true><<<G, kBlock, 0, c->stream>>>(np, x, p, r, Ap, r32, c->partials, c->scal, dscale);

@@ -33,7 +33,8 @@ enum ColForm : uint8_t {
 };
 
 // Ints per slice in the compact index record: the 27 slot bases, then the
-// slice's form (ColForm), then padding to 128 bytes.  A wave reads a slice's
+// slice's form (ColForm), then whether the next slice continues it
+// (k_slice_runs), then padding to 128 bytes.  A wave reads a slice's
 // form and bases with scalar loads from one record, in one round trip.
 constexpr int kMeta = 32;
 
@@ -155,8 +156,9 @@ enum ValForm : int {
 };
 
 // What the building of a level's compact columns and value forms reports per
-// level: mismatches of each form, and the number of wide slices.
-enum FormFlag : int { kBadSlot = 0, kBadDiag, kBadField, kWideSlices, kFormFlags };
+// level: mismatches of each form, the number of wide slices and of slices that
+// continue in the next one.
+enum FormFlag : int { kBadSlot = 0, kBadDiag, kBadField, kWideSlices, kRunSlices, kFormFlags };
 
 // Column index format of a context (hpcgx_set_column_format).
 enum ColFormat : int { kColsExplicit = 0, kColsCompact = 1, kColsCompactAlways = 2 };
@@ -299,6 +301,7 @@ struct Level {
   // diagonals are read from the value array.
   int vform = kValsStored;
   bool diag_one = false;
+  bool runs = false;  // nine slices in ten continue in the next one (k_slice_runs)
   uint32_t *vmask = nullptr;
   double *slotv = nullptr;
   double *field = nullptr;

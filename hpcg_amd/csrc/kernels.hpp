@@ -52,6 +52,36 @@ __device__ __forceinline__ int64_t tile_id() {
   return xcd * per + (xcd < rem ? xcd : rem) + r;
 }
 
+// Tile of a whole-level pass that takes the 8 colour blocks together: XCD x
+// gets the x-th eighth of every block, the blocks in turn, so one XCD's L2
+// serves the 8 tiles that gather the same part of the vector.  bt: tiles per
+// block, a multiple of 8 (block_tiles), or 0 for tile_id.
+__device__ __forceinline__ int64_t level_tile(int bt) {
+  if (!bt) return tile_id();
+  const int xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+  return (int64_t)(i & 7) * bt + xcd * (bt >> 3) + (i >> 3);
+}
+
+// The block index b with tile_id<ROT>() == tile in a grid of G blocks: where
+// the one-row-per-lane launch of a pass leaves that tile's partial sum.
+template <bool ROT = false>
+__device__ __forceinline__ int64_t tile_slot(unsigned tile, unsigned G) {
+  const unsigned per = G >> 3, rem = G & 7, wide = rem * (per + 1);
+  unsigned xcd, r;
+  if (tile < wide) {
+    xcd = tile / (per + 1);
+    r = tile - xcd * (per + 1);
+  } else {
+    xcd = rem + (tile - wide) / per;
+    r = tile - wide - (xcd - rem) * per;
+  }
+  if constexpr (ROT) {
+    const unsigned len = per + (xcd < rem ? 1 : 0), shift = (xcd * len) >> 3;
+    r = r >= shift ? r - shift : r + len - shift;
+  }
+  return (int64_t)r * 8 + xcd;
+}
+
 // Occupancy of the fp64 sparse kernels (SpMV, Gauss-Seidel steps,
 // restriction).  With explicit 32-bit column indices: at most two waves per
 // SIMD, so a wave holds the column, value and gather loads of all its slots
@@ -580,6 +610,144 @@ __device__ __forceinline__ int64_t chunk_index(int j) {
 // ---------------------------------------------------------------------------
 // sparse kernels (one thread per row, 4 slices per block)
 
+// ---------------------------------------------------------------------------
+// Row runs: two consecutive fp64 rows per lane (kValsSlot and kValsField)
+//
+// Without the value stream a large pass is bound by the vector L1: it takes
+// a load of 64 lanes in 16 steps of four lanes whether a lane asks for 8 or 16
+// bytes (measured: 17 L1 accesses per 8-byte gather; on a 512^3 fine step the
+// address units were busy for 80 % of the time).  So a lane takes two
+// consecutive rows and gathers each slot's two neighbours with one 16-byte
+// load: in a uniform slice they are consecutive.  The wave covers two slices;
+// it takes this path where the second continues the first (k_slice_runs: both
+// uniform, each slot's base going on by 64), which holds but for a few slices
+// at the ends of blocks and strips; elsewhere it takes its slices one after
+// the other, a row per lane.  Products and sums of a row are the same, in the
+// same order.
+//
+// kValsSlot, a row per lane -> runs: 512^3 fine step 369 -> 301 us (1.6 GB,
+// 5.3 TB/s), 192^3 17.9 -> 14.7 us, 192^3 SpMV 113 -> 77 us; kValsField: 128^3
+// fine step 10.7 -> 9.0 us.  The fp32 and fp16 passes keep a row per lane:
+// 192^3 fine step 10.6 us, 11.0 with two rows and 11.6 with four.
+//
+// Launches of fewer rows keep it too (a wave of a run needs longer, with twice
+// the sums, and a small launch waits for its last wave): without / with runs,
+// 104^3 fine steps (140608 rows) 5.9 / 5.8 us, 96^3 (110592) 4.6 / 4.4, 48^3
+// (13824) 3.2 / 4.0.
+constexpr int64_t kRunMinRows = 1 << 17;
+
+// Whether a launch over `rows` rows of a level takes row runs.
+inline bool run_rows(const Level &L, int64_t rows) { return L.runs && rows >= kRunMinRows; }
+
+typedef double f64x2_u __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ void ld_pair(const double *p, double (&v)[2]) {
+  const f64x2_u t = *reinterpret_cast<const f64x2_u *>(p);
+  v[0] = t.x;
+  v[1] = t.y;
+}
+__device__ __forceinline__ void st_pair(double *p, const double (&v)[2]) {
+  f64x2_u t;
+  t.x = v[0];
+  t.y = v[1];
+  *reinterpret_cast<f64x2_u *>(p) = t;
+}
+
+// Whether the next slice continues a slice, in the slice's record.
+constexpr int kRunAt = kSlots + 1;
+
+// The off-diagonal values' inputs and the diagonals of a lane's two rows.
+template <int VF>
+struct RunVals {
+  uint32_t m[2];
+  double d[2], ki[2];
+  __device__ __forceinline__ void load(const ValSrc<double, double> &src, int64_t row) {
+    const u32x2_t t = *reinterpret_cast<const u32x2_t *>(src.mask + row);
+    m[0] = t.x;
+    m[1] = t.y;
+    if (VF == kValsSlot && src.diag_one) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) d[j] = (m[j] >> kDiagSlot) & 1u ? src.slotv[kDiagSlot] : 1.0;
+    } else {  // the diagonals of a slice are adjacent
+      ld_pair(src.vals + val_pos<2>(row, kDiagSlot), d);
+    }
+    if constexpr (VF == kValsField) ld_pair(src.field + row, ki);
+  }
+};
+
+// sum[j] += (SUB: -=) a x over the slots in MASK, ascending.  base: the
+// first slice's slot bases (scalars); e0: the lane's first row, from the
+// run's start; xd: x of the rows themselves.  SAFE as in gs_row.
+template <int VF, uint32_t MASK, bool SUB, bool SAFE>
+__device__ __forceinline__ void run_sum(const int (&base)[kSlots], unsigned e0, const ValSrc<double, double> &src,
+                                        const RunVals<VF> &v, const double *__restrict__ x, const double (&xd)[2],
+                                        double (&sum)[2]) {
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    if (!((MASK >> s) & 1u)) continue;
+    double xv[2] = {xd[0], xd[1]}, kv[2];
+    if (s != kDiagSlot) {
+      ld_pair(x + base[s] + e0, xv);
+      if constexpr (VF == kValsField) ld_pair(src.field + base[s] + e0, kv);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      double a;
+      if (s == kDiagSlot) a = v.d[j];
+      else if constexpr (VF == kValsField) a = bit_select(v.m[j], s, -((v.ki[j] + kv[j]) * 0.5));
+      else a = bit_select(v.m[j], s, src.slotv[s]);
+      const double t = a * (SAFE && a == 0.0 ? 0.0 : xv[j]);
+      if constexpr (SUB) sum[j] -= t;
+      else sum[j] += t;
+    }
+  }
+}
+
+// A wave's place in a launch over the 64-row slices of [row0, row0 + nrows),
+// nrows a multiple of 64: it takes the slices 2g and 2g + 1 of it.  On a run
+// the lane's rows are row + 2 lane and the next one (active: it has rows),
+// else row + 64 j + lane of slice j.
+struct RunWave {
+  int64_t row;  // first row of the wave
+  int slices;   // slices it takes (0: past the end)
+  bool run, active;
+  int base[kSlots];
+  __device__ __forceinline__ void init(const ColIdx &ci, int64_t row0, int64_t nrows, int64_t tile) {
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t g = (tile * (int64_t)(kBlock / kSlice) + w) * 2;
+    const int64_t left = (nrows >> 6) - g;
+    row = row0 + g * kSlice;
+    slices = left <= 0 ? 0 : left < 2 ? 1 : 2;
+    run = active = false;
+    if (slices) {
+      const int *rec = ci.cbase + (row >> 6) * kMeta;
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) base[s] = rec[s];
+      run = rec[kSlots] == kFormUniform && rec[kRunAt] >= slices - 1;
+      active = run && 2 * (threadIdx.x & 63) < (unsigned)slices * kSlice;
+    }
+  }
+  __device__ __forceinline__ int64_t lane_row(int j) const {
+    const unsigned lane = threadIdx.x & 63;
+    return run ? row + 2 * lane + j : row + j * kSlice + lane;
+  }
+  __device__ __forceinline__ bool has_row(int j) const { return run ? active : j < slices; }
+};
+
+// a[j] = v for a j known at run time, the array kept in registers.
+__device__ __forceinline__ void put(double (&a)[2], int j, double v) {
+  a[0] = j == 0 ? v : a[0];
+  a[1] = j == 1 ? v : a[1];
+}
+
+// Blocks of a row-run launch over `rows` rows.
+inline int block_tiles(const Level &L) {
+  const int64_t rows = L.lay.start[1];
+  for (int k = 0; k < kColours; ++k)
+    if (L.lay.start[k + 1] - L.lay.start[k] != rows) return 0;
+  return rows % (8 * 2 * kBlock) ? 0 : (int)(rows / (2 * kBlock));
+}
+inline unsigned run_tiles(int64_t rows) { return (unsigned)((rows + 2 * kBlock - 1) / (2 * kBlock)); }
+
 // y = A x over rows [0, nrows); ComputeSPMV_ref.cpp:61-70
 template <class VT, class XT, class ACC, bool CI, int VF>
 __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_spmv(const ColIdx ci,
@@ -602,6 +770,58 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_spmv(
     }
     return sum;
   });
+}
+
+// (A x) of a wave's rows (RunWave::lane_row), 0 where a lane has none.
+template <int VF>
+__device__ __forceinline__ void run_ax(const ColIdx &ci, const ValSrc<double, double> &src, const RunWave &w,
+                                       const double *__restrict__ x, double (&out)[2]) {
+  const unsigned lane = threadIdx.x & 63;
+  out[0] = out[1] = 0.0;
+  if (w.run) {
+    if (!w.active) return;
+    RunVals<VF> v;
+    v.load(src, w.row + 2 * lane);
+    double xd[2];
+    ld_pair(x + w.row + 2 * lane, xd);
+    run_sum<VF, kAllSlots, false, false>(w.base, 2 * lane, src, v, x, xd, out);
+    return;
+  }
+#pragma unroll 1
+  for (int j = 0; j < w.slices; ++j) {
+    const int64_t row = w.row + j * kSlice + lane;
+    RowVals<VF, double, double, false, kAllSlots> v;
+    v.load(src, row);
+    put(out, j, with_cols<true, true>(ci, slice_of<true>(row), [&](auto cm, const int *base) {
+      constexpr int CM = decltype(cm)::value;
+      double sum = 0;
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        const int c = col_at<CM, true>(ci, row, base, ell_base(row), s);
+        sum += v.at(s, c) * x[c];
+      }
+      return sum;
+    }));
+  }
+}
+
+// y = A x by row runs
+template <int VF>
+__global__ __launch_bounds__(kBlock) void k_spmv_run(const ColIdx ci, const ValSrc<double, double> src,
+                                                     const double *__restrict__ x, double *__restrict__ y,
+                                                     int64_t nrows, int bt) {
+  RunWave w;
+  w.init(ci, 0, nrows, level_tile(bt));
+  if (!w.slices) return;
+  double ax[2];
+  run_ax<VF>(ci, src, w, x, ax);
+  if (w.run) {
+    if (w.active) st_pair(y + w.lane_row(0), ax);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if (w.has_row(j)) y[w.lane_row(j)] = ax[j];
+  }
 }
 
 // Slots whose neighbour lies in a block swept before block k in the default
@@ -628,6 +848,10 @@ constexpr bool masks_keep_units(int W) {
   return true;
 }
 static_assert(masks_keep_units(2) && masks_keep_units(4), "zero-start masks split a value unit");
+
+#ifndef HPCGX_FINE_ROT
+#define HPCGX_FINE_ROT 1
+#endif
 
 // One Gauss-Seidel step on the rows of one colour block; ComputeSYMGS_ref.cpp:72-79:
 // sum = r_i - sum_j a_ij x_j (diagonal included) + x_i a_ii ; x_i = sum / a_ii.
@@ -697,9 +921,6 @@ void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
   static_assert(VF == kValsStored || (CI && !GEN), "value forms: stencil levels with compact columns");
   // blocks of 256 threads, or of 64 for the small coarse fp64 steps (one wave
   // per block spreads them over more CUs); the r.z form always takes 256
-#ifndef HPCGX_FINE_ROT
-#define HPCGX_FINE_ROT 1
-#endif
   const int64_t t = tile_id<HPCGX_FINE_ROT && FINE && sizeof(VT) == 8>() * (int64_t)blockDim.x + threadIdx.x;
   if constexpr (RZ) {
     // every thread reaches the block reduction; rows past the block add 0
@@ -711,6 +932,75 @@ void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
   }
   if (t >= nrows) return;
   gs_row<VT, XT, ACC, ZK, FINE, CI, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
+}
+
+// The partial sums of a value per row, as the one-row-per-lane launch leaves
+// them: v[j] belongs to row lane_row(j).  Each 64-row slice is reduced over row
+// distances 32, 16, .. 1 as wave_sum does it, and the four slices of a 256-row
+// tile as block_partials does; the tile's sum goes where that launch's block
+// would leave it.  ntiles: tiles of the launch.
+template <bool ROT>
+__device__ __forceinline__ void run_partials(const RunWave &w, double (&v)[2], int64_t tile, int64_t ntiles,
+                                             double *partials) {
+  __shared__ double sh[2 * kBlock / kSlice];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (w.run) {  // lanes 0..31 hold the first slice's rows, two each
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) {
+      v[0] += __shfl_down(v[0], off, 64);
+      v[1] += __shfl_down(v[1], off, 64);
+    }
+    if ((lane & 31) == 0) sh[2 * wave + (lane >> 5)] = v[0] + v[1];
+  } else {
+    const double a = wave_sum(v[0]), b = wave_sum(v[1]);
+    if (lane == 0) {
+      sh[2 * wave] = a;
+      sh[2 * wave + 1] = b;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const int64_t t = 2 * tile + threadIdx.x;
+    const double *q = sh + 4 * threadIdx.x;
+    if (t < ntiles) partials[tile_slot<ROT>((unsigned)t, (unsigned)ntiles)] = (q[0] + q[1]) + (q[2] + q[3]);
+  }
+}
+
+// One Gauss-Seidel step by row runs (k_gs on kValsSlot and kValsField levels).
+template <int ZK, bool FINE, int VF, bool RZ = false, bool SAFE = false>
+__global__ __launch_bounds__(kBlock) void k_gs_run(const ColIdx ci, const ValSrc<double, double> src,
+                                                   const double *__restrict__ r, double *__restrict__ x,
+                                                   int64_t row0, int64_t nrows, double *rz = nullptr) {
+  constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
+  constexpr bool ROT = HPCGX_FINE_ROT && FINE;
+  const int64_t tile = tile_id<ROT>();
+  RunWave w;
+  w.init(ci, row0, nrows, tile);
+  double acc[2] = {0.0, 0.0};
+  if (w.run) {
+    if (w.active) {
+      const int64_t row = w.lane_row(0);
+      RunVals<VF> v;
+      v.load(src, row);
+      double rv[2], xd[2] = {0.0, 0.0}, xn[2];
+      ld_pair(r + row, rv);
+      if constexpr (ZK < 0) ld_pair(x + row, xd);
+      double sum[2] = {rv[0], rv[1]};
+      run_sum<VF, mask, true, ZK >= 0 && SAFE>(w.base, 2 * (threadIdx.x & 63), src, v, x, xd, sum);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if constexpr (ZK < 0) sum[j] += xd[j] * v.d[j];
+        xn[j] = sum[j] / v.d[j];
+        acc[j] = rv[j] * xn[j];
+      }
+      st_pair(x + row, xn);
+    }
+  } else {
+#pragma unroll 1
+    for (int j = 0; j < w.slices; ++j)
+      put(acc, j, gs_row<double, double, double, ZK, FINE, true, VF, false, SAFE>(ci, src, r, x, w.lane_row(j), nullptr));
+  }
+  if constexpr (RZ) run_partials<ROT>(w, acc, tile, (nrows + kBlock - 1) / kBlock, rz);
 }
 
 // Residual at the injected rows and restriction, fused (ComputeMG_ref.cpp:49-51 +
@@ -751,6 +1041,25 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_restr
   ACC res = (ACC)r[row] - ax;
   if (SCALE) res = res * (ACC)sigma[t];
   rc[inj[t]] = (XT)res;
+}
+
+// k_restrict over the block of injected rows by row runs; the rows that pad
+// the block to whole slices are not written.
+template <int VF>
+__global__ __launch_bounds__(kBlock) void k_restrict_run(const ColIdx ci, const ValSrc<double, double> src,
+                                                         const double *__restrict__ r, const double *__restrict__ x,
+                                                         double *__restrict__ rc, const int *__restrict__ inj,
+                                                         int64_t row0, int64_t count) {
+  RunWave w;
+  w.init(ci, row0, (count + kSlice - 1) / kSlice * kSlice, tile_id());
+  if (!w.slices) return;
+  double ax[2];
+  run_ax<VF>(ci, src, w, x, ax);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int64_t row = w.lane_row(j), t = row - row0;
+    if (w.has_row(j) && t < count) rc[inj[t]] = r[row] - ax[j];
+  }
 }
 
 // x_f += xc at the injected rows (ComputeProlongation_ref.cpp:49).

@@ -37,6 +37,12 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
     if (rz) {
       // 256-thread blocks: the partials are per block of 4 waves, tiles(nr) of them
       with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+        if constexpr (VF() != kValsStored) {
+          if (run_rows(L, nr)) {
+            k_gs_run<-1, FINE, VF(), true><<<run_tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, rz);
+            return;
+          }
+        }
         k_gs<VT, XT, ACC, -1, FINE, CI(), VF(), false, true><<<tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, nullptr, rz);
       });
       return;
@@ -52,6 +58,12 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
     }
   }
   with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+    if constexpr (VF() != kValsStored && sizeof(XT) == 8) {
+      if (run_rows(L, nr)) {
+        k_gs_run<ZK, FINE, VF(), false, SAFE><<<run_tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr);
+        return;
+      }
+    }
     k_gs<VT, XT, ACC, ZK, FINE, CI(), VF(), false, false, SAFE><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
   });
 }
@@ -156,6 +168,12 @@ static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64
   const int64_t nc = L.ninj, r0 = L.lay.start[L.lay.inj];
   const ColIdx ci = col_idx(c, L);
   with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+    if constexpr (VF() != kValsStored && sizeof(XT) == 8) {
+      if (!L.frow && run_rows(L, nc)) {
+        k_restrict_run<VF()><<<run_tiles(nc), kBlock, 0, c->stream>>>(ci, val_src<VT, ACC>(L), r, x, rc_v, L.inj, r0, nc);
+        return;
+      }
+    }
     k_restrict<VT, XT, ACC, SCALE, CI(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
         ci, val_src<VT, ACC>(L), r, x, rc_v, L.inj, L.sigma, r0, nc, L.frow);
   });
@@ -287,6 +305,13 @@ int spmv_fp64(Ctx *c, int level, const double *x, double *y) {
   const Level &L = c->levels[level];
   const ColIdx ci = col_idx(c, L);
   with_forms<double>(L, ci, [&](auto CI, auto VF) {
+    if constexpr (VF() != kValsStored) {
+      if (run_rows(L, L.lay.npad)) {
+        k_spmv_run<VF()><<<run_tiles(L.lay.npad), kBlock, 0, c->stream>>>(ci, val_src<double, double>(L), x, y, L.lay.npad,
+                                                                       block_tiles(L));
+        return;
+      }
+    }
     k_spmv<double, double, double, CI(), VF()><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(
         ci, val_src<double, double>(L), x, y, L.lay.npad);
   });
@@ -390,6 +415,13 @@ int hpcgx_restrict(hpcgx_ctx *c, int level, const double *r, const double *x, do
   const int64_t nc = L.ninj;
   const ColIdx ci = col_idx(c, L);
   with_forms<double>(L, ci, [&](auto CI, auto VF) {
+    if constexpr (VF() != kValsStored) {
+      if (!L.frow && run_rows(L, nc)) {
+        k_restrict_run<VF()><<<run_tiles(nc), kBlock, 0, c->stream>>>(ci, val_src<double, double>(L), r, x, rc_out, L.inj,
+                                                                      L.lay.start[L.lay.inj], nc);
+        return;
+      }
+    }
     k_restrict<double, double, double, false, CI(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
         ci, val_src<double, double>(L), r, x, rc_out, L.inj, nullptr, L.lay.start[L.lay.inj], nc, L.frow);
   });

@@ -175,9 +175,14 @@ int ensure_stage(Ctx *c, int64_t n) {
 }
 
 // One allocation per level for the forms: the slot values (27 in fp64, 27
-// each for the fp32 and fp16 copies as fp32, padded to 512 bytes), the row
-// masks and the slices' column forms.
-constexpr size_t kSlotvBytes = 512;
+// each for the fp32 and fp16 copies as fp32), each block's usual distance from
+// a row to its slots' columns (kBlockOffs), the row masks and the slices'
+// column forms.
+constexpr size_t kOffsAt = 512;
+constexpr size_t kSlotvBytes = 1536;
+static_assert(kOffsAt >= kSlots * 16 && kSlotvBytes >= kOffsAt + kColours * kSlots * sizeof(int), "");
+constexpr int kNoOffset = INT_MIN;
+static int *level_offs(const Level &L) { return reinterpret_cast<int *>(reinterpret_cast<char *>(L.slotv) + kOffsAt); }
 static size_t form_bytes(const Level &L) {
   return kSlotvBytes + L.lay.npad * sizeof(uint32_t) + (size_t)(L.lay.npad / kSlice);
 }
@@ -1081,7 +1086,8 @@ __device__ __forceinline__ bool diag_differs(double d, bool real, double slot_di
 // value) are base + lane + d with d in [-128, 127]; a zero-valued slot
 // (neighbour outside the grid, unused entry) may name any row of the level,
 // as its product is an exact zero: it takes its own row when reachable, else
-// the nearest reachable one.  A slice whose columns do not fit is wide and
+// the nearest reachable one (a slot without a stored entry in the slice: the
+// row at its block's usual distance).  A slice whose columns do not fit is wide and
 // keeps its explicit indices.  A slice in which every slot's stored entries
 // share one offset (column - lane), and whose zero-valued slots may then
 // take base + lane (a row of the level), is uniform: base + lane is its
@@ -1101,13 +1107,16 @@ __global__ __launch_bounds__(kBlock) void k_compact_cols(const int *__restrict__
                                                          uint8_t *__restrict__ cform, int64_t nslices, int64_t npad,
                                                          const int *__restrict__ iperm, const double *__restrict__ slotv,
                                                          const double *__restrict__ field, uint32_t *__restrict__ vmask,
-                                                         int *flags) {
+                                                         const int *__restrict__ offs, LayoutDev lay, int *flags) {
   const int lane = threadIdx.x & 63;
   const int64_t slice = (int64_t)blockIdx.x * (kBlock / kSlice) + (threadIdx.x >> 6);
   if (slice >= nslices) return;
   const int64_t row = slice * kSlice + lane;
   const size_t b = (size_t)slice * (kSlots * kSlice) + lane;
   const int ds = dslot ? dslot[row] : kDiagSlot;
+  int block = 0;
+  if (vmask)
+    while (block < kColours - 1 && slice * kSlice >= lay.start[block + 1]) ++block;
   bool wide = false, uniform = true;
   uint32_t mask = 0;
   bool bad_slot = false, bad_field = false;
@@ -1129,7 +1138,12 @@ __global__ __launch_bounds__(kBlock) void k_compact_cols(const int *__restrict__
     }
     int64_t base;
     if (lo == INT_MAX) {
-      base = slice * kSlice;  // no live lane: every lane names its own row
+      // no live lane: every lane names the row at the block's usual distance
+      // (so that the slice continues its neighbours), or its own row where
+      // that leaves the level
+      base = slice * kSlice;
+      const int off = vmask ? offs[block * kSlots + s] : kNoOffset;
+      if (off != kNoOffset && base + off >= 0 && base + off + kSlice <= npad) base += off;
     } else {
       if ((int64_t)hi - lo > 255) wide = true;
       if (hi != lo) uniform = false;
@@ -1178,12 +1192,15 @@ __global__ __launch_bounds__(kBlock) void k_check_diag(const double *__restrict_
 // The candidate value of each slot: the first stored entry met in that slot
 // among 32 rows spread over each colour block (all rows of a small block; a
 // slot that they all miss keeps +0).  k_compact_cols then checks every row.
+// offs[k][s]: how far the column of slot s lies from the row, on the first
+// such row of block k (kNoOffset: none).
 // One workgroup, a row per thread; also clears the flags and derives the slot
 // values of the lower-precision copies with the roundings of k_to_f32 and
 // k_to_f16_scaled.
 constexpr int kSampleRows = 32;
 __global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(LayoutDev L, const double *__restrict__ vals,
-                                                                        double *slotv, int *flags) {
+                                                                        const int *__restrict__ cols, double *slotv,
+                                                                        int *offs, int *flags) {
   __shared__ int first[kSlots];
   const int t = threadIdx.x;
   if (t < kSlots) first[t] = INT_MAX;
@@ -1196,12 +1213,21 @@ __global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(LayoutDe
   // not all lie at the same x
   const int64_t p = L.start[k] + (count <= kSampleRows ? (in ? i : 0) : (count / kSampleRows * i + i) % count);
   double v[kSlots];
-#pragma unroll
-  for (int s = 0; s < kSlots; ++s) v[s] = in ? vals[val_pos<2>(p, s)] : 0.0;
+  int c[kSlots];
 #pragma unroll
   for (int s = 0; s < kSlots; ++s) {
-    const unsigned long long b = __ballot(v[s] != 0.0);
-    if (b && __builtin_ctzll(b) == (t & 63)) atomicMin(&first[s], (int)p);
+    v[s] = in ? vals[val_pos<2>(p, s)] : 0.0;
+    c[s] = in ? cols[ell_base(p) + s * kSlice] : 0;
+  }
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    const unsigned mine = (unsigned)(__ballot(v[s] != 0.0) >> (t & 32));  // the block's 32 rows
+    if (!mine) {
+      if (i == 0) offs[k * kSlots + s] = kNoOffset;
+    } else if (__builtin_ctz(mine) == i) {
+      offs[k * kSlots + s] = c[s] - (int)p;
+      atomicMin(&first[s], (int)p);
+    }
   }
   __syncthreads();
   if (t >= kSlots) return;
@@ -1213,6 +1239,22 @@ __global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(LayoutDe
   lo[t] = (float)a;
   lo[kSlots + t] = __half2float(__float2half_rn((float)(t == kDiagSlot ? 1.0 : a * di * di)));
 }
+// Whether each slice continues in the next one: both are uniform and each
+// slot's base is 64 rows further.  Counts those that do.
+__global__ __launch_bounds__(kBlock) void k_slice_runs(int *__restrict__ cbase, int64_t nslices, int *flags) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  bool on = i + 1 < nslices;
+  if (on) {
+    const int *a = cbase + i * kMeta, *b = a + kMeta;
+    on = a[kSlots] == kFormUniform && b[kSlots] == kFormUniform;
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) on = on && b[s] == a[s] + kSlice;
+  }
+  if (i < nslices) cbase[i * kMeta + kRunAt] = on;
+  const int n = __popcll(__ballot(on));
+  if (n && (threadIdx.x & 63) == 0) atomicAdd(&flags[kRunSlices], n);
+}
+
 __global__ void k_clear_flags(int *flags) {
   if (threadIdx.x < kFormFlags) flags[threadIdx.x] = 0;
 }
@@ -1229,14 +1271,16 @@ static int build_compact_cols(Ctx *c, Level &L, int *flags) {
   L.cform = reinterpret_cast<uint8_t *>(mask + L.lay.npad);
   if (!L.lay.general) {
     L.vmask = mask;
-    k_slot_values<<<1, kColours * kSampleRows, 0, c->stream>>>(L.ldev, L.vals, L.slotv, flags);
+    k_slot_values<<<1, kColours * kSampleRows, 0, c->stream>>>(L.ldev, L.vals, L.cols, L.slotv, level_offs(L), flags);
   } else {
     k_clear_flags<<<1, 64, 0, c->stream>>>(flags);
   }
   HPCGX_CHECK_LAUNCH(c);
   const int64_t grid = (ns + (kBlock / kSlice) - 1) / (kBlock / kSlice);
   k_compact_cols<<<grid, kBlock, 0, c->stream>>>(L.cols, L.vals, L.dslot, L.cbase, L.cdelta, L.cform, ns,
-                                                 L.lay.npad, L.iperm, L.slotv, L.field, L.vmask, flags);
+                                                 L.lay.npad, L.iperm, L.slotv, L.field, L.vmask, level_offs(L), L.ldev,
+                                                 flags);
+  if (L.vmask) k_slice_runs<<<nblk(ns), kBlock, 0, c->stream>>>(L.cbase, ns, flags);
   HPCGX_CHECK_LAUNCH(c);
   return HPCGX_OK;
 }
@@ -1266,6 +1310,7 @@ static int build_compact_all(Ctx *c) {
     if (!L.vmask) continue;
     L.vform = !f[kBadSlot] ? kValsSlot : !f[kBadField] ? kValsField : kValsStored;
     L.diag_one = L.vform == kValsSlot && !f[kBadDiag];
+    L.runs = 10 * (int64_t)f[kRunSlices] >= 9 * (L.lay.npad / kSlice);
   }
   return HPCGX_OK;
 }
