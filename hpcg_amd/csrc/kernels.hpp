@@ -40,8 +40,7 @@ __device__ __forceinline__ size_t ell_base(int64_t row) {
 // fp32 / fp16 steps keep it too (rotated, the mixed 512^3 solves ran 1.7 %
 // slower).
 template <bool ROT = false>
-__device__ __forceinline__ int64_t tile_id() {
-  const int64_t G = gridDim.x, b = blockIdx.x;
+__device__ __forceinline__ int64_t tile_at(int64_t b, int64_t G) {
   const int64_t per = G >> 3, rem = G & 7, xcd = b & 7, idx = b >> 3;
   int64_t r = idx;
   if constexpr (ROT) {
@@ -50,6 +49,10 @@ __device__ __forceinline__ int64_t tile_id() {
     if (r >= len) r -= len;
   }
   return xcd * per + (xcd < rem ? xcd : rem) + r;
+}
+template <bool ROT = false>
+__device__ __forceinline__ int64_t tile_id() {
+  return tile_at<ROT>(blockIdx.x, gridDim.x);
 }
 
 // Tile of a whole-level pass that takes the 8 colour blocks together: XCD x
@@ -865,11 +868,11 @@ static_assert(masks_keep_units(2) && masks_keep_units(4), "zero-start masks spli
 // ZK == 0 reads no neighbour at all (x_i = r_i / a_ii), which holds for the
 // first block of any order, general levels included.
 // GEN: general level, the diagonal's slot is dslot[row] (stencil: slot 13).
-// gs_row is the update of one row; it returns r_i * x_i (new) for the fused r.z.
+// gs_value is a row's new value, from r_i; gs_row the update of one row, which
+// returns r_i * x_i (new) for the fused r.z.
 template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI, int VF, bool GEN, bool SAFE>
-__device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC> &src,
-                                         const XT *__restrict__ r, XT *__restrict__ x, int64_t row,
-                                         const uint8_t *__restrict__ dslot) {
+__device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &src, ACC ri, const XT *x, int64_t row,
+                                       const uint8_t *__restrict__ dslot) {
   constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
   const size_t b = ell_base(row);
   const int slice = slice_of<true>(row);
@@ -880,7 +883,7 @@ __device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC>
   else d = ld_val<ACC, FINE>(src.vals + val_pos<val_width<VT>>(row, (int)dslot[row]));
   auto row_sum = [&](auto cm, const int *base) {
     constexpr int CM = decltype(cm)::value;
-    ACC sum = (ACC)r[row];
+    ACC sum = ri;
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
       if (!((mask >> s) & 1u)) continue;
@@ -899,7 +902,14 @@ __device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC>
   };
   ACC sum = with_cols<CI, true>(ci, slice, row_sum);
   if (ZK < 0) sum += (ACC)x[row] * d;
-  const XT xn = (XT)(sum / d);
+  return (XT)(sum / d);
+}
+
+template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI, int VF, bool GEN, bool SAFE>
+__device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC> &src,
+                                         const XT *__restrict__ r, XT *__restrict__ x, int64_t row,
+                                         const uint8_t *__restrict__ dslot) {
+  const XT xn = gs_value<VT, XT, ACC, ZK, FINE, CI, VF, GEN, SAFE>(ci, src, (ACC)r[row], x, row, dslot);
   x[row] = xn;
   return (double)r[row] * (double)xn;
 }
@@ -1074,6 +1084,120 @@ __global__ __launch_bounds__(kBlock) void k_prolong(XT *__restrict__ x, const XT
   ACC v = (ACC)xc[inj[t]];
   if (SCALE) v = v * (ACC)sigma[t];
   x[row] = (XT)((ACC)x[row] + v);
+}
+
+// ---------------------------------------------------------------------------
+// The tail of the V-cycle in one workgroup
+//
+// A colour step of a small level takes a launch 2 to 4 us whatever its size
+// (start-up, a chain of dependent loads and sums, draining), and a V-cycle has
+// 15 or 30 of them per level.  From the first level of up to kTailRows rows
+// on, one workgroup runs the rest of the V-cycle: x and r live in LDS, a
+// barrier separates the colour steps, the matrix comes from L2.  The rows' sums
+// are those of the separate launches, in the same order.
+//
+// V-cycle, launches -> tail: 8^3 (3 levels) 289 -> 84 us, 16^3 299 -> 114 (fp32
+// 304 -> 107), 20^3 (2 levels) 133 -> 85 (fp32 141 -> 78).  The limit is a block of
+// a slice per wave: a 24^3 level (27 slices a block) takes one CU as long as a
+// launch per step takes 256 (64 us against 47 to 57), a 26^3 one longer (187
+// against 132).
+constexpr int kTailRows = 8192;       // padded rows of the tail's first level
+constexpr int kTailThreads = 1024;
+constexpr int kTailColours = 16;      // colours of a level it can sweep
+constexpr int kTailLds = 160 * 1024;  // LDS of a CU
+
+template <class VT, class XT, class ACC>
+struct TailLevel {
+  ColIdx ci;
+  ValSrc<VT, ACC> src;
+  const uint8_t *dslot;
+  const int *inj;    // the transfer to the next level
+  const int *frow;
+  const float *sigma;
+  int ninj, row0;
+  int npad, ncol;
+  int xoff, roff;    // x and r in LDS, in elements
+  int start[kTailColours + 1];
+};
+// r, x: the first level's.  load_x: start from x instead of 0.
+template <class VT, class XT, class ACC>
+struct TailArgs {
+  TailLevel<VT, XT, ACC> lv[kMaxLevels];
+  const XT *r;
+  XT *x;
+  int n, load_x;
+};
+
+template <class VT, class XT, class ACC, bool SCALE, bool CI, int VF, bool GEN>
+__global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, ACC> a) {
+  extern __shared__ double tail_shared[];
+  XT *lds = reinterpret_cast<XT *>(tail_shared);
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  auto sweep = [&](const TailLevel<VT, XT, ACC> &L) {  // forward, then backward without the last block
+    XT *x = lds + L.xoff;
+    for (int step = 0; step < 2 * L.ncol - 1; ++step) {
+      const int k = step < L.ncol ? step : 2 * L.ncol - 2 - step;
+      const int end = L.start[k + 1] >> 6;
+      for (int slice = (L.start[k] >> 6) + wave; slice < end; slice += nw) {
+        const int row = slice * kSlice + lane;
+        x[row] = gs_value<VT, XT, ACC, -1, false, CI, VF, GEN, false>(L.ci, L.src, (ACC)lds[L.roff + row], x, row, L.dslot);
+      }
+      __syncthreads();
+    }
+  };
+  const TailLevel<VT, XT, ACC> &F = a.lv[0];
+  for (int i = threadIdx.x; i < F.npad; i += blockDim.x) {
+    lds[F.xoff + i] = a.load_x ? a.x[i] : (XT)0;
+    lds[F.roff + i] = a.r[i];
+  }
+  for (int l = 1; l < a.n; ++l)
+    for (int i = threadIdx.x; i < a.lv[l].npad; i += blockDim.x) lds[a.lv[l].xoff + i] = lds[a.lv[l].roff + i] = (XT)0;
+  __syncthreads();
+  for (int l = 0;; ++l) {
+    const TailLevel<VT, XT, ACC> &L = a.lv[l];
+    const XT *x = lds + L.xoff;
+    sweep(L);
+    if (l + 1 == a.n) break;
+    // the next level's r: residual at the injected rows (k_restrict)
+    for (int t0 = wave * kSlice; t0 < L.ninj; t0 += nw * kSlice) {
+      const int t = t0 + lane;
+      if (t >= L.ninj) continue;
+      const int64_t row = L.frow ? L.frow[t] : L.row0 + t;
+      const size_t b = ell_base(row);
+      RowVals<VF, VT, ACC, false, kAllSlots> v;
+      v.load(L.src, row);
+      auto row_ax = [&](auto cm, const int *base) {
+        constexpr int CM = decltype(cm)::value;
+        ACC ax = 0;
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+          const int c = col_at<CM, false>(L.ci, row, base, b, s);
+          ax += v.at(s, c) * (ACC)x[c];
+        }
+        return ax;
+      };
+      ACC ax;
+      if constexpr (GEN) ax = with_cols<CI, false>(L.ci, slice_of<false>(row), row_ax);  // rows from a list
+      else ax = with_cols<CI, true>(L.ci, slice_of<true>(row), row_ax);
+      ACC res = (ACC)lds[L.roff + row] - ax;
+      if (SCALE) res = res * (ACC)L.sigma[t];
+      lds[a.lv[l + 1].roff + L.inj[t]] = (XT)res;
+    }
+    __syncthreads();
+  }
+  for (int l = a.n - 2; l >= 0; --l) {
+    const TailLevel<VT, XT, ACC> &L = a.lv[l];
+    for (int t = threadIdx.x; t < L.ninj; t += blockDim.x) {  // k_prolong
+      const int row = L.frow ? L.frow[t] : L.row0 + t;
+      ACC v = (ACC)lds[a.lv[l + 1].xoff + L.inj[t]];
+      if (SCALE) v = v * (ACC)L.sigma[t];
+      lds[L.xoff + row] = (XT)((ACC)lds[L.xoff + row] + v);
+    }
+    __syncthreads();
+    sweep(L);
+  }
+  for (int i = threadIdx.x; i < F.npad; i += blockDim.x) a.x[i] = lds[F.xoff + i];
 }
 
 // ---------------------------------------------------------------------------

@@ -1,6 +1,8 @@
 // Kernel drivers: SpMV, coloured symmetric Gauss-Seidel, fused residual +
 // restriction, prolongation, the V-cycle in fp64 / fp32 / scaled fp16, and
 // the vector reductions.
+#include <algorithm>
+#include <atomic>
 #include <initializer_list>
 #include <mutex>
 
@@ -144,6 +146,90 @@ static int symgs_launch(Ctx *c, int l, const XT *r, XT *x, bool zero_start, doub
   return HPCGX_OK;
 }
 
+// Runs the V-cycle from level l down (or, with load_x, a smoothing step of
+// level l alone) in one workgroup.  False: these levels take launches, being
+// too large, of different forms, or of more colours than the kernel sweeps.
+template <class VT, class XT, class ACC, bool SCALE>
+static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
+  const Level &F = c->levels[l];
+  if (F.lay.npad > kTailRows) return false;
+  TailArgs<VT, XT, ACC> a;
+  a.r = r;
+  a.x = x;
+  a.n = load_x ? 1 : (int)c->levels.size() - l;
+  a.load_x = load_x;
+  const ColIdx ci = col_idx(c, F);
+  int64_t off = 0;
+  int waves = 1;
+  for (int k = 0; k < a.n; ++k) {
+    const Level &L = c->levels[l + k];
+    TailLevel<VT, XT, ACC> &t = a.lv[k];
+    t.ci = col_idx(c, L);
+    if (L.lay.ncol > kTailColours || !L.dslot != !F.dslot || !t.ci.cbase != !ci.cbase ||
+        val_form<VT>(L, t.ci) != val_form<VT>(F, ci) || (L.frow && !F.dslot))
+      return false;
+    t.src = val_src<VT, ACC>(L);
+    t.dslot = L.dslot;
+    t.inj = L.inj;
+    t.frow = L.frow;
+    t.sigma = L.sigma;
+    t.ninj = (int)L.ninj;
+    t.row0 = (int)L.lay.start[L.lay.inj];
+    t.npad = (int)L.lay.npad;
+    t.ncol = L.lay.ncol;
+    for (int j = 0; j <= L.lay.ncol; ++j) t.start[j] = (int)L.lay.start[j];
+    for (int j = 0; j < L.lay.ncol; ++j) waves = std::max(waves, (t.start[j + 1] - t.start[j]) >> 6);
+    t.xoff = (int)off;
+    t.roff = (int)(off + L.lay.npad);
+    off += 2 * L.lay.npad;
+    if (off * (int64_t)sizeof(XT) > kTailLds) return false;
+  }
+  const unsigned lds = (unsigned)(off * sizeof(XT));
+  const unsigned bs = (unsigned)std::min(waves, kTailThreads / kSlice) * kSlice;
+  auto go = [&](auto CI, auto VF, auto GEN) {
+    const auto kernel = k_tail<VT, XT, ACC, SCALE, CI(), VF(), GEN()>;
+    static std::atomic<uint64_t> raised{0};  // devices on which the kernel may take all of a CU's LDS
+    const uint64_t bit = (uint64_t)1 << (c->device & 63);
+    if (!(raised.load() & bit)) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kTailLds);
+      raised.fetch_or(bit);
+    }
+    kernel<<<1, bs, lds, c->stream>>>(a);
+  };
+  if (F.dslot) {
+    constexpr std::integral_constant<int, kValsStored> stored{};
+    if (ci.cbase) go(std::true_type{}, stored, std::true_type{});
+    else go(std::false_type{}, stored, std::true_type{});
+  } else {
+    // a kappa level reads its stored values here: the field's 27 gathers would
+    // not come from LDS (20^3 fp64, 2 levels: 143 us against 93)
+    with_forms<VT>(F, ci, [&](auto CI, auto VF) {
+      go(CI, std::integral_constant<int, VF() == kValsSlot ? kValsSlot : kValsStored>{}, std::false_type{});
+    });
+  }
+  return true;
+}
+
+// r.x partials of a level that the tail solved, as its post-smoother's steps
+// leave them (k_gs with RZ): the tiles of the last block, then of the blocks
+// down to the first, each block's in the order of its launch.
+struct TailBlocks {
+  int start[kTailColours + 1];
+  int ncol;
+};
+__global__ __launch_bounds__(kBlock) void k_tail_rz(const TailBlocks L, const double *__restrict__ r,
+                                                    const double *__restrict__ x, double *rz) {
+  int k = L.ncol - 1, first = 0, n = 0;
+  for (;; --k) {
+    n = (L.start[k + 1] - L.start[k] + kBlock - 1) / kBlock;
+    if ((int)blockIdx.x < first + n) break;
+    first += n;
+  }
+  const int64_t row = L.start[k] + tile_at<HPCGX_FINE_ROT != 0>((int)blockIdx.x - first, n) * kBlock + threadIdx.x;
+  const double v[1] = {row < L.start[k + 1] ? r[row] * x[row] : 0.0};
+  block_partials<1>(v, rz);
+}
+
 // V-cycle of ComputeMG_ref.cpp:39-63: x = 0; pre-smooth; residual + restrict;
 // recurse; prolong; post-smooth.  The coarsest level gets one smoothing step.
 // rz / nrz: r.x partials of the result from the post-smoother (see sweep);
@@ -154,6 +240,20 @@ template <class VT, class XT, class ACC, bool SCALE>
 static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64_t *nrz = nullptr,
                   bool untrusted_x = false) {
   const Level &L = c->levels[l];
+  if (tail<VT, XT, ACC, SCALE>(c, l, r, x)) {
+    if constexpr (sizeof(VT) == 8) {
+      if (rz) {
+        TailBlocks b;
+        b.ncol = L.lay.ncol;
+        *nrz = 0;
+        for (int k = 0; k <= b.ncol; ++k) b.start[k] = (int)L.lay.start[k];
+        for (int k = 0; k < b.ncol; ++k) *nrz += tiles(b.start[k + 1] - b.start[k]);
+        k_tail_rz<<<(unsigned)*nrz, kBlock, 0, c->stream>>>(b, r, x, rz);
+      }
+    }
+    HPCGX_CHECK_LAUNCH(c);
+    return HPCGX_OK;
+  }
   int rc = symgs_launch<VT, XT, ACC>(c, l, r, x, true, nullptr, nullptr, untrusted_x);
   if (rc || l + 1 >= (int)c->levels.size()) return rc;
   Level &C = c->levels[l + 1];
@@ -320,6 +420,10 @@ int spmv_fp64(Ctx *c, int level, const double *x, double *y) {
 }
 
 int symgs_fp64(Ctx *c, int level, const double *r, double *x) {
+  if (tail<double, double, double, false>(c, level, r, x, true)) {
+    HPCGX_CHECK_LAUNCH(c);
+    return HPCGX_OK;
+  }
   return symgs_launch<double, double, double>(c, level, r, x, false);
 }
 
