@@ -112,9 +112,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_x(int64_t n, const double *__rest
 }
 
 // Ap = A p and the partials of pAp = p.Ap.  One 256-row tile per block.
-// CI: column indices from the compact form.  VF: the values' form.
-template <bool CI, int VF>
-__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CI) void k_cg_spmv_dot(const ColIdx ci, const ValSrc<double, double> src,
+// CF, VF: where the columns and the values come from.
+template <int CF, int VF>
+__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CF) void k_cg_spmv_dot(const ColIdx ci, const ValSrc<double, double> src,
                                                         const double *__restrict__ p,
                                                         double *__restrict__ Ap, int64_t nrows,
                                                         double *partials) {
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CI) void k_c
     const int slice = slice_of<true>(row);
     RowVals<VF, double, double, true, kAllSlots> v;
     v.load(src, row);
-    const double sum = with_cols<CI, true>(ci, slice, [&](auto cm, const int *base) {
+    const double sum = with_cols<CF, true>(ci, slice, [&](auto cm, const int *base) {
       constexpr int CM = decltype(cm)::value;
       double acc_row = 0.0;
 #pragma unroll
@@ -336,7 +336,7 @@ static void cg_spmv_dot(Ctx *c, const Level &L, const double *p, double *Ap) {
   const ColIdx ci = col_idx(c, L);
   const int64_t np = L.lay.npad;
   const ValSrc<double, double> src = val_src<double, double>(L);
-  with_forms<double>(L, ci, [&](auto CI, auto VF) {
+  with_forms<double>(L, ci, [&](auto CF, auto VF) {
     if constexpr (VF() != kValsStored) {
       if (run_rows(L, np)) {
         k_cg_spmv_dot_run<VF()><<<run_tiles(np), kBlock, 0, c->stream>>>(ci, src, p, Ap, np, c->partials,
@@ -344,7 +344,7 @@ static void cg_spmv_dot(Ctx *c, const Level &L, const double *p, double *Ap) {
         return;
       }
     }
-    k_cg_spmv_dot<CI(), VF()><<<tiles(np), kBlock, 0, c->stream>>>(ci, src, p, Ap, np, c->partials);
+    k_cg_spmv_dot<CF(), VF()><<<tiles(np), kBlock, 0, c->stream>>>(ci, src, p, Ap, np, c->partials);
   });
 }
 

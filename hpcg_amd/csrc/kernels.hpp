@@ -85,6 +85,13 @@ __device__ __forceinline__ int64_t tile_slot(unsigned tile, unsigned G) {
   return (int64_t)r * 8 + xcd;
 }
 
+// Where a launch takes its columns from.
+enum ColSource : int {
+  kColsStored = 0,  // the explicit 32-bit index of every entry
+  kColsSlice = 1,   // the compact form: the slice's record, and its deltas (ColForm)
+  kColsBlock = 2,   // the column is the row plus a distance that the slot has over the whole colour block
+};
+
 // Occupancy of the fp64 sparse kernels (SpMV, Gauss-Seidel steps,
 // restriction).  With explicit 32-bit column indices: at most two waves per
 // SIMD, so a wave holds the column, value and gather loads of all its slots
@@ -110,12 +117,12 @@ __device__ __forceinline__ int64_t tile_slot(unsigned tile, unsigned G) {
 #ifndef HPCGX_FP64_WAVES
 #define HPCGX_FP64_WAVES 2
 #endif
-template <class VT, bool CI = false, int SLOTS = 27>
+template <class VT, int CF = kColsStored, int SLOTS = 27>
 struct SparseOccupancy {
   static constexpr unsigned max_waves =
-      (sizeof(VT) == 8 && SLOTS >= 8) ? (CI ? HPCGX_CI_FP64_WAVES : HPCGX_FP64_WAVES) : 8;
+      (sizeof(VT) == 8 && SLOTS >= 8) ? (CF ? HPCGX_CI_FP64_WAVES : HPCGX_FP64_WAVES) : 8;
 };
-#define HPCGX_SPARSE_OCCUPANCY(VT, CI) __attribute__((amdgpu_waves_per_eu(1, SparseOccupancy<VT, CI>::max_waves)))
+#define HPCGX_SPARSE_OCCUPANCY(VT, CF) __attribute__((amdgpu_waves_per_eu(1, SparseOccupancy<VT, CF>::max_waves)))
 
 // Matrix loads.  NT (non-temporal): the fine level's matrix is streamed once
 // per pass and is far larger than any cache, so it is kept out of the way of
@@ -315,22 +322,40 @@ struct RowVals<kValsField, VT, ACC, NT, MASK> {
   __device__ __forceinline__ ACC diag(const ValSrc<VT, ACC> &, int64_t) const { return d; }
 };
 
-// Column index of (row, slot): the explicit 32-bit index, or the compact
-// form (ColForm) with a per-slice base.
+// Column index of (row, slot): the explicit 32-bit index, the compact form
+// (ColForm) with a per-slice base, or, in a launch over rows of one colour
+// block, the row plus the slot's distance.
 struct ColIdx {
   const int *cols;
   const int *cbase;     // null: explicit indices only
   const int8_t *cdelta;
   const uint8_t *cform;
+  const int *off;   // kColsBlock: the block's distances (null: the launch does not take this form)
+  int last;         // and the level's last row
 };
 
 // The columns a launch reads on a level: the compact form when the context
 // uses it and the level reads it (Level::read_compact), else the explicit
-// indices.
-inline ColIdx col_idx(const Ctx *c, const Level &L) {
-  if (L.cbase && ((c->col_format == kColsCompact && L.read_compact) || c->col_format == kColsCompactAlways))
-    return ColIdx{L.cols, L.cbase, L.cdelta, L.cform};
-  return ColIdx{L.cols, nullptr, nullptr, nullptr};
+// indices.  block >= 0: the launch takes rows of that colour block alone.
+//
+// Where a block's slots have one distance each (block_cols), a launch reads the
+// block's 27 distances, which stay in the caches, instead of a record for
+// every slice.  V-cycles, records -> distances: 192^3 fp32 581 -> 548 us, 192^3
+// kappa fp16 764 -> 709 (57 MB of records less), 64^3 245 -> 235.  Row runs keep the
+// records (k_gs_run: 104^3 to 1e-9 32.0 ms with them, 33.5 without).
+inline ColIdx col_idx(const Ctx *c, const Level &L, int block = -1) {
+  ColIdx ci;
+  ci.cols = L.cols;
+  ci.cbase = ci.off = nullptr;
+  if (!L.cbase || !((c->col_format == kColsCompact && L.read_compact) || c->col_format == kColsCompactAlways)) return ci;
+  ci.cbase = L.cbase;
+  ci.cdelta = L.cdelta;
+  ci.cform = L.cform;
+  if (block >= 0 && !L.bcols.empty()) {
+    ci.off = L.boffs + block * kMeta;
+    ci.last = (int)(L.lay.npad - 1);
+  }
+  return ci;
 }
 
 // The value source and form of a launch.  The forms other than the stored
@@ -360,16 +385,23 @@ inline int val_form(const Level &L, const ColIdx &ci) {
   else return L.vform;
 }
 
-// Runs f(CI, VF) with the column and value forms of a launch as constants.
-template <class VT, class F>
+// Runs f(CF, VF) with the column and value forms of a launch as constants.
+// BLOCKS: the launch takes the rows of one block (col_idx was given it).
+template <class VT, bool BLOCKS = false, class F>
 inline void with_forms(const Level &L, const ColIdx &ci, F &&f) {
-  if (!ci.cbase) return f(std::false_type{}, std::integral_constant<int, kValsStored>{});
+  if (!ci.cbase) return f(std::integral_constant<int, kColsStored>{}, std::integral_constant<int, kValsStored>{});
   const int vf = val_form<VT>(L, ci);
-  if constexpr (sizeof(VT) == 8) {
-    if (vf == kValsField) return f(std::true_type{}, std::integral_constant<int, kValsField>{});
+  auto with_vals = [&](auto CF) {
+    if constexpr (sizeof(VT) == 8) {
+      if (vf == kValsField) return f(CF, std::integral_constant<int, kValsField>{});
+    }
+    if (vf == kValsSlot) return f(CF, std::integral_constant<int, kValsSlot>{});
+    f(CF, std::integral_constant<int, kValsStored>{});
+  };
+  if constexpr (BLOCKS) {
+    if (ci.off) return with_vals(std::integral_constant<int, kColsBlock>{});
   }
-  if (vf == kValsSlot) return f(std::true_type{}, std::integral_constant<int, kValsSlot>{});
-  f(std::true_type{}, std::integral_constant<int, kValsStored>{});
+  with_vals(std::integral_constant<int, kColsSlice>{});
 }
 
 // Slice of a row.  UNI: the 64 lanes of the wave hold the 64 rows of one
@@ -382,7 +414,7 @@ __device__ __forceinline__ int slice_of(int64_t row) {
 }
 
 // Column of (row, slot s).  CM 0: the explicit 32-bit index; CM 1: base +
-// lane + int8 delta; CM 2: base + lane.  A launch picks one per slice
+// lane + int8 delta; CM 2: base + lane; CM 3: row + base (kColsBlock).  A launch picks one per slice
 // (with_cols), so each inner loop is straight-line code; base holds the
 // slice's 27 slot bases (with_cols provides them).
 template <int CM, bool NT>
@@ -394,8 +426,10 @@ __device__ __forceinline__ int col_at(const ColIdx &ci, int64_t row, const int *
     if constexpr (NT) d = __builtin_nontemporal_load(ci.cdelta + b + s * kSlice);
     else d = ci.cdelta[b + s * kSlice];
     return base[s] + (int)(row & 63) + (int)d;
-  } else {
+  } else if constexpr (CM == 2) {
     return base[s] + (int)(row & 63);
+  } else {
+    return min(max((int)row + base[s], 0), ci.last);  // a zero entry's row may lie outside the level
   }
 }
 
@@ -403,17 +437,22 @@ template <int V>
 using cmode = std::integral_constant<int, V>;
 
 // Runs f(cmode<CM>{}, base) with the column mode of the row's slice and its
-// slot bases.  CI: the launch reads compact indices.  UNI: the slice is the
+// slot bases (kColsBlock: the distances).  UNI: the slice is the
 // same for the whole wave: the bases and the form are read together from
 // the slice's record before the choice, scalar loads in one round trip
 // (small coarse steps are bound by their chain of dependent loads: reading
 // the form first and the bases after it cost one more), and the choice is a
 // scalar branch.  Otherwise each lane reads its slice's form from cform and
 // its bases from the record as the slots need them.
-template <bool CI, bool UNI, class F>
+template <int CF, bool UNI, class F>
 __device__ __forceinline__ auto with_cols(const ColIdx &ci, int slice, F &&f) {
-  if constexpr (!CI) {
+  if constexpr (CF == kColsStored) {
     return f(cmode<0>{}, (const int *)nullptr);
+  } else if constexpr (CF == kColsBlock) {
+    int off[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) off[s] = ci.off[s];
+    return f(cmode<3>{}, (const int *)off);
   } else if constexpr (UNI) {
     const int *rec = ci.cbase + (int64_t)slice * kMeta;
     int base[kSlots];
@@ -752,8 +791,8 @@ inline int block_tiles(const Level &L) {
 inline unsigned run_tiles(int64_t rows) { return (unsigned)((rows + 2 * kBlock - 1) / (2 * kBlock)); }
 
 // y = A x over rows [0, nrows); ComputeSPMV_ref.cpp:61-70
-template <class VT, class XT, class ACC, bool CI, int VF>
-__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_spmv(const ColIdx ci,
+template <class VT, class XT, class ACC, int CF, int VF>
+__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CF) void k_spmv(const ColIdx ci,
                                                  const ValSrc<VT, ACC> src,
                                                  const XT *__restrict__ x, XT *__restrict__ y,
                                                  int64_t nrows) {
@@ -763,7 +802,7 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_spmv(
   const int slice = slice_of<true>(row);
   RowVals<VF, VT, ACC, true, kAllSlots> v;
   v.load(src, row);
-  y[row] = (XT)with_cols<CI, true>(ci, slice, [&](auto cm, const int *base) {
+  y[row] = (XT)with_cols<CF, true>(ci, slice, [&](auto cm, const int *base) {
     constexpr int CM = decltype(cm)::value;
     ACC sum = 0;
 #pragma unroll
@@ -795,7 +834,7 @@ __device__ __forceinline__ void run_ax(const ColIdx &ci, const ValSrc<double, do
     const int64_t row = w.row + j * kSlice + lane;
     RowVals<VF, double, double, false, kAllSlots> v;
     v.load(src, row);
-    put(out, j, with_cols<true, true>(ci, slice_of<true>(row), [&](auto cm, const int *base) {
+    put(out, j, with_cols<kColsSlice, true>(ci, slice_of<true>(row), [&](auto cm, const int *base) {
       constexpr int CM = decltype(cm)::value;
       double sum = 0;
 #pragma unroll
@@ -870,7 +909,7 @@ static_assert(masks_keep_units(2) && masks_keep_units(4), "zero-start masks spli
 // GEN: general level, the diagonal's slot is dslot[row] (stencil: slot 13).
 // gs_value is a row's new value, from r_i; gs_row the update of one row, which
 // returns r_i * x_i (new) for the fused r.z.
-template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI, int VF, bool GEN, bool SAFE>
+template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, bool SAFE>
 __device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &src, ACC ri, const XT *x, int64_t row,
                                        const uint8_t *__restrict__ dslot) {
   constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
@@ -900,16 +939,16 @@ __device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &
     }
     return sum;
   };
-  ACC sum = with_cols<CI, true>(ci, slice, row_sum);
+  ACC sum = with_cols<CF, true>(ci, slice, row_sum);
   if (ZK < 0) sum += (ACC)x[row] * d;
   return (XT)(sum / d);
 }
 
-template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI, int VF, bool GEN, bool SAFE>
+template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, bool SAFE>
 __device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC> &src,
                                          const XT *__restrict__ r, XT *__restrict__ x, int64_t row,
                                          const uint8_t *__restrict__ dslot) {
-  const XT xn = gs_value<VT, XT, ACC, ZK, FINE, CI, VF, GEN, SAFE>(ci, src, (ACC)r[row], x, row, dslot);
+  const XT xn = gs_value<VT, XT, ACC, ZK, FINE, CF, VF, GEN, SAFE>(ci, src, (ACC)r[row], x, row, dslot);
   x[row] = xn;
   return (double)r[row] * (double)xn;
 }
@@ -918,30 +957,30 @@ __device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC>
 // post-smoother's last forward block and its backward steps); the block
 // also leaves its partial sum of r_i x_i in rz[blockIdx.x], so the solver's
 // r.z needs no pass of its own.
-template <class VT, class XT, class ACC, int ZK, bool FINE, bool CI = false, int VF = kValsStored, bool GEN = false,
+template <class VT, class XT, class ACC, int ZK, bool FINE, int CF = kColsStored, int VF = kValsStored, bool GEN = false,
           bool RZ = false, bool SAFE = false>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(1, SparseOccupancy<VT, CI, ZK < 0 ? kSlots : __builtin_popcount(swept_before_mask(ZK))>::max_waves)))
+__attribute__((amdgpu_waves_per_eu(1, SparseOccupancy<VT, CF, ZK < 0 ? kSlots : __builtin_popcount(swept_before_mask(ZK))>::max_waves)))
 void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
                                                const XT *__restrict__ r, XT *__restrict__ x,
                                                int64_t row0, int64_t nrows,
                                                const uint8_t *__restrict__ dslot, double *rz = nullptr) {
   static_assert(!GEN || ZK <= 0, "general levels: full rows, or the first block from x = 0 (diagonal only)");
   static_assert(!RZ || ZK < 0, "r.z is taken from the post-smoother");
-  static_assert(VF == kValsStored || (CI && !GEN), "value forms: stencil levels with compact columns");
+  static_assert(VF == kValsStored || (CF && !GEN), "value forms: stencil levels with compact columns");
   // blocks of 256 threads, or of 64 for the small coarse fp64 steps (one wave
   // per block spreads them over more CUs); the r.z form always takes 256
   const int64_t t = tile_id<HPCGX_FINE_ROT && FINE && sizeof(VT) == 8>() * (int64_t)blockDim.x + threadIdx.x;
   if constexpr (RZ) {
     // every thread reaches the block reduction; rows past the block add 0
     double acc = 0.0;
-    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CI, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
+    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
     const double v[1] = {acc};
     block_partials<1>(v, rz);
     return;
   }
   if (t >= nrows) return;
-  gs_row<VT, XT, ACC, ZK, FINE, CI, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
+  gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
 }
 
 // The partial sums of a value per row, as the one-row-per-lane launch leaves
@@ -1008,7 +1047,7 @@ __global__ __launch_bounds__(kBlock) void k_gs_run(const ColIdx ci, const ValSrc
   } else {
 #pragma unroll 1
     for (int j = 0; j < w.slices; ++j)
-      put(acc, j, gs_row<double, double, double, ZK, FINE, true, VF, false, SAFE>(ci, src, r, x, w.lane_row(j), nullptr));
+      put(acc, j, gs_row<double, double, double, ZK, FINE, kColsSlice, VF, false, SAFE>(ci, src, r, x, w.lane_row(j), nullptr));
   }
   if constexpr (RZ) run_partials<ROT>(w, acc, tile, (nrows + kBlock - 1) / kBlock, rz);
 }
@@ -1017,8 +1056,8 @@ __global__ __launch_bounds__(kBlock) void k_gs_run(const ColIdx ci, const ValSrc
 // ComputeRestriction_ref.cpp:51): rc[inj[t]] = r_f - (A x)_f for the t-th
 // injected row f = row0 + t (frow[t] when frow is given).  (A x)_f is summed
 // from 0 like SpMV, then subtracted.  SCALE: fp16 V-cycle, times sigma[t].
-template <class VT, class XT, class ACC, bool SCALE, bool CI, int VF>
-__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_restrict(const ColIdx ci, const ValSrc<VT, ACC> src,
+template <class VT, class XT, class ACC, bool SCALE, int CF, int VF>
+__global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CF) void k_restrict(const ColIdx ci, const ValSrc<VT, ACC> src,
                                                      const XT *__restrict__ r,
                                                      const XT *__restrict__ x,
                                                      XT *__restrict__ rc, const int *__restrict__ inj,
@@ -1043,10 +1082,10 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CI) void k_restr
   ACC ax;
   if (frow) {  // rows from a list: slices differ across the wave
     const int slice = slice_of<false>(row);
-    ax = with_cols<CI, false>(ci, slice, row_ax);
+    ax = with_cols<CF, false>(ci, slice, row_ax);
   } else {
     const int slice = slice_of<true>(row);
-    ax = with_cols<CI, true>(ci, slice, row_ax);
+    ax = with_cols<CF, true>(ci, slice, row_ax);
   }
   ACC res = (ACC)r[row] - ax;
   if (SCALE) res = res * (ACC)sigma[t];
@@ -1128,7 +1167,7 @@ struct TailArgs {
   int n, load_x;
 };
 
-template <class VT, class XT, class ACC, bool SCALE, bool CI, int VF, bool GEN>
+template <class VT, class XT, class ACC, bool SCALE, int CF, int VF, bool GEN>
 __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, ACC> a) {
   extern __shared__ double tail_shared[];
   XT *lds = reinterpret_cast<XT *>(tail_shared);
@@ -1141,7 +1180,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
       const int end = L.start[k + 1] >> 6;
       for (int slice = (L.start[k] >> 6) + wave; slice < end; slice += nw) {
         const int row = slice * kSlice + lane;
-        x[row] = gs_value<VT, XT, ACC, -1, false, CI, VF, GEN, false>(L.ci, L.src, (ACC)lds[L.roff + row], x, row, L.dslot);
+        x[row] = gs_value<VT, XT, ACC, -1, false, CF, VF, GEN, false>(L.ci, L.src, (ACC)lds[L.roff + row], x, row, L.dslot);
       }
       __syncthreads();
     }
@@ -1178,8 +1217,8 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
         return ax;
       };
       ACC ax;
-      if constexpr (GEN) ax = with_cols<CI, false>(L.ci, slice_of<false>(row), row_ax);  // rows from a list
-      else ax = with_cols<CI, true>(L.ci, slice_of<true>(row), row_ax);
+      if constexpr (GEN) ax = with_cols<CF, false>(L.ci, slice_of<false>(row), row_ax);  // rows from a list
+      else ax = with_cols<CF, true>(L.ci, slice_of<true>(row), row_ax);
       ACC res = (ACC)lds[L.roff + row] - ax;
       if (SCALE) res = res * (ACC)L.sigma[t];
       lds[a.lv[l + 1].roff + L.inj[t]] = (XT)res;

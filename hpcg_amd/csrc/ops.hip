@@ -18,7 +18,7 @@ template <class VT, class XT, class ACC, int ZK, bool FINE, bool SAFE = false>
 static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *rz = nullptr) {
   const int64_t r0 = L.lay.start[k], nr = L.lay.start[k + 1] - r0;
   if (nr <= 0) return;
-  const ColIdx ci = col_idx(c, L);
+  const ColIdx ci = col_idx(c, L, k);
   // Coarse fp64 steps of blocks under HPCGX_ONE_WAVE_ROWS (2^20) rows launch
   // as one-wave blocks, which spreads them over more CUs: with explicit
   // columns at two waves per SIMD a 192^3 set measured 2-6 % faster, 512^3
@@ -38,14 +38,14 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
   if constexpr (ZK < 0 && sizeof(VT) == 8 && sizeof(XT) == 8) {
     if (rz) {
       // 256-thread blocks: the partials are per block of 4 waves, tiles(nr) of them
-      with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+      with_forms<VT, true>(L, ci, [&](auto CF, auto VF) {
         if constexpr (VF() != kValsStored) {
           if (run_rows(L, nr)) {
             k_gs_run<-1, FINE, VF(), true><<<run_tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, rz);
             return;
           }
         }
-        k_gs<VT, XT, ACC, -1, FINE, CI(), VF(), false, true><<<tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, nullptr, rz);
+        k_gs<VT, XT, ACC, -1, FINE, CF(), VF(), false, true><<<tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr, nullptr, rz);
       });
       return;
     }
@@ -53,20 +53,20 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
   if constexpr (ZK <= 0) {  // general levels: full rows, or the first block from x = 0
     if (L.dslot) {
       if (ci.cbase)
-        k_gs<VT, XT, ACC, ZK, FINE, true, kValsStored, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
+        k_gs<VT, XT, ACC, ZK, FINE, kColsSlice, kValsStored, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
       else
-        k_gs<VT, XT, ACC, ZK, FINE, false, kValsStored, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
+        k_gs<VT, XT, ACC, ZK, FINE, kColsStored, kValsStored, true><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, L.dslot);
       return;
     }
   }
-  with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+  with_forms<VT, true>(L, ci, [&](auto CF, auto VF) {
     if constexpr (VF() != kValsStored && sizeof(XT) == 8) {
       if (run_rows(L, nr)) {
         k_gs_run<ZK, FINE, VF(), false, SAFE><<<run_tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr);
         return;
       }
     }
-    k_gs<VT, XT, ACC, ZK, FINE, CI(), VF(), false, false, SAFE><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
+    k_gs<VT, XT, ACC, ZK, FINE, CF(), VF(), false, false, SAFE><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
   });
 }
 
@@ -186,8 +186,8 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
   }
   const unsigned lds = (unsigned)(off * sizeof(XT));
   const unsigned bs = (unsigned)std::min(waves, kTailThreads / kSlice) * kSlice;
-  auto go = [&](auto CI, auto VF, auto GEN) {
-    const auto kernel = k_tail<VT, XT, ACC, SCALE, CI(), VF(), GEN()>;
+  auto go = [&](auto CF, auto VF, auto GEN) {
+    const auto kernel = k_tail<VT, XT, ACC, SCALE, CF(), VF(), GEN()>;
     static std::atomic<uint64_t> raised{0};  // devices on which the kernel may take all of a CU's LDS
     const uint64_t bit = (uint64_t)1 << (c->device & 63);
     if (!(raised.load() & bit)) {
@@ -198,13 +198,13 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
   };
   if (F.dslot) {
     constexpr std::integral_constant<int, kValsStored> stored{};
-    if (ci.cbase) go(std::true_type{}, stored, std::true_type{});
-    else go(std::false_type{}, stored, std::true_type{});
+    if (ci.cbase) go(std::integral_constant<int, kColsSlice>{}, stored, std::true_type{});
+    else go(std::integral_constant<int, kColsStored>{}, stored, std::true_type{});
   } else {
     // a kappa level reads its stored values here: the field's 27 gathers would
     // not come from LDS (20^3 fp64, 2 levels: 143 us against 93)
-    with_forms<VT>(F, ci, [&](auto CI, auto VF) {
-      go(CI, std::integral_constant<int, VF() == kValsSlot ? kValsSlot : kValsStored>{}, std::false_type{});
+    with_forms<VT>(F, ci, [&](auto CF, auto VF) {
+      go(CF, std::integral_constant<int, VF() == kValsSlot ? kValsSlot : kValsStored>{}, std::false_type{});
     });
   }
   return true;
@@ -266,15 +266,15 @@ static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64
     xc_v = reinterpret_cast<XT *>(C.x32);
   }
   const int64_t nc = L.ninj, r0 = L.lay.start[L.lay.inj];
-  const ColIdx ci = col_idx(c, L);
-  with_forms<VT>(L, ci, [&](auto CI, auto VF) {
+  const ColIdx ci = col_idx(c, L, L.frow ? -1 : L.lay.inj);
+  with_forms<VT, true>(L, ci, [&](auto CF, auto VF) {
     if constexpr (VF() != kValsStored && sizeof(XT) == 8) {
       if (!L.frow && run_rows(L, nc)) {
         k_restrict_run<VF()><<<run_tiles(nc), kBlock, 0, c->stream>>>(ci, val_src<VT, ACC>(L), r, x, rc_v, L.inj, r0, nc);
         return;
       }
     }
-    k_restrict<VT, XT, ACC, SCALE, CI(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
+    k_restrict<VT, XT, ACC, SCALE, CF(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
         ci, val_src<VT, ACC>(L), r, x, rc_v, L.inj, L.sigma, r0, nc, L.frow);
   });
   HPCGX_CHECK_LAUNCH(c);
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(kBlock) void k_to_double(const float *__restrict__ 
 int spmv_fp64(Ctx *c, int level, const double *x, double *y) {
   const Level &L = c->levels[level];
   const ColIdx ci = col_idx(c, L);
-  with_forms<double>(L, ci, [&](auto CI, auto VF) {
+  with_forms<double>(L, ci, [&](auto CF, auto VF) {
     if constexpr (VF() != kValsStored) {
       if (run_rows(L, L.lay.npad)) {
         k_spmv_run<VF()><<<run_tiles(L.lay.npad), kBlock, 0, c->stream>>>(ci, val_src<double, double>(L), x, y, L.lay.npad,
@@ -412,7 +412,7 @@ int spmv_fp64(Ctx *c, int level, const double *x, double *y) {
         return;
       }
     }
-    k_spmv<double, double, double, CI(), VF()><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(
+    k_spmv<double, double, double, CF(), VF()><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(
         ci, val_src<double, double>(L), x, y, L.lay.npad);
   });
   HPCGX_CHECK_LAUNCH(c);
@@ -517,8 +517,8 @@ int hpcgx_restrict(hpcgx_ctx *c, int level, const double *r, const double *x, do
     return rc;
   const Level &L = c->levels[level];
   const int64_t nc = L.ninj;
-  const ColIdx ci = col_idx(c, L);
-  with_forms<double>(L, ci, [&](auto CI, auto VF) {
+  const ColIdx ci = col_idx(c, L, L.frow ? -1 : L.lay.inj);
+  with_forms<double, true>(L, ci, [&](auto CF, auto VF) {
     if constexpr (VF() != kValsStored) {
       if (!L.frow && run_rows(L, nc)) {
         k_restrict_run<VF()><<<run_tiles(nc), kBlock, 0, c->stream>>>(ci, val_src<double, double>(L), r, x, rc_out, L.inj,
@@ -526,7 +526,7 @@ int hpcgx_restrict(hpcgx_ctx *c, int level, const double *r, const double *x, do
         return;
       }
     }
-    k_restrict<double, double, double, false, CI(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
+    k_restrict<double, double, double, false, CF(), VF()><<<tiles(nc), kBlock, 0, c->stream>>>(
         ci, val_src<double, double>(L), r, x, rc_out, L.inj, nullptr, L.lay.start[L.lay.inj], nc, L.frow);
   });
   HPCGX_CHECK_LAUNCH(c);

@@ -176,11 +176,12 @@ int ensure_stage(Ctx *c, int64_t n) {
 
 // One allocation per level for the forms: the slot values (27 in fp64, 27
 // each for the fp32 and fp16 copies as fp32), each block's usual distance from
-// a row to its slots' columns (kBlockOffs), the row masks and the slices'
+// a row to its slots' columns, the exact ones (BlockCols), the row masks and the slices'
 // column forms.
-constexpr size_t kOffsAt = 512;
-constexpr size_t kSlotvBytes = 1536;
-static_assert(kOffsAt >= kSlots * 16 && kSlotvBytes >= kOffsAt + kColours * kSlots * sizeof(int), "");
+constexpr size_t kOffsAt = 512, kBoffsAt = 1536;
+constexpr size_t kSlotvBytes = kBoffsAt + kColours * sizeof(BlockCols);
+static_assert(kOffsAt >= kSlots * 16 && kBoffsAt >= kOffsAt + kColours * kSlots * sizeof(int), "");
+static_assert(sizeof(BlockCols) == kMeta * sizeof(int), "");
 constexpr int kNoOffset = INT_MIN;
 static int *level_offs(const Level &L) { return reinterpret_cast<int *>(reinterpret_cast<char *>(L.slotv) + kOffsAt); }
 static size_t form_bytes(const Level &L) {
@@ -1166,18 +1167,17 @@ __global__ __launch_bounds__(kBlock) void k_compact_cols(const int *__restrict__
   const int form = any_wide ? kFormWide : all_uniform ? kFormUniform : kFormDelta;
   if (lane == 0) cform[slice] = (uint8_t)form;
   if (lane < kMeta - kSlots) cbase[slice * kMeta + kSlots + lane] = lane == 0 ? form : 0;  // the form, then padding
-  if (lane == 0 && form == kFormWide) atomicAdd(&flags[kWideSlices], 1);
   if (!vmask) return;
   const bool real = iperm[row] >= 0;
   if (real) mask |= 1u << kDiagSlot;
   vmask[row] = mask;
   const bool bad_diag = diag_differs(vals[val_pos<2>(row, kDiagSlot)], real, slotv[kDiagSlot]);
   const bool bs = __any(bad_slot), bd = __any(bad_diag), bf = !field || __any(bad_field);
-  // a flag already up is not raised again: on a level without the form every wave would queue on it
+  // stores, not read-modify-writes: on a level without the form every wave raises its flag
   if (lane == 0) {
-    if (bs && !__hip_atomic_load(&flags[kBadSlot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&flags[kBadSlot], 1);
-    if (bd && !__hip_atomic_load(&flags[kBadDiag], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&flags[kBadDiag], 1);
-    if (bf && !__hip_atomic_load(&flags[kBadField], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&flags[kBadField], 1);
+    if (bs) flags[kBadSlot] = 1;
+    if (bd) flags[kBadDiag] = 1;
+    if (bf) flags[kBadField] = 1;
   }
 }
 
@@ -1186,7 +1186,7 @@ __global__ __launch_bounds__(kBlock) void k_check_diag(const double *__restrict_
                                                        const double *__restrict__ slotv, int64_t npad, int *flags) {
   const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   const bool bad = p < npad && diag_differs(vals[val_pos<2>(p, kDiagSlot)], (vmask[p] >> kDiagSlot) & 1u, slotv[kDiagSlot]);
-  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(&flags[kBadDiag], 1);
+  if (__any(bad) && (threadIdx.x & 63) == 0) flags[kBadDiag] = 1;
 }
 
 // The candidate value of each slot: the first stored entry met in that slot
@@ -1240,7 +1240,7 @@ __global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(LayoutDe
   lo[kSlots + t] = __half2float(__float2half_rn((float)(t == kDiagSlot ? 1.0 : a * di * di)));
 }
 // Whether each slice continues in the next one: both are uniform and each
-// slot's base is 64 rows further.  Counts those that do.
+// slot's base is 64 rows further.  Counts those that do, and the wide ones.
 __global__ __launch_bounds__(kBlock) void k_slice_runs(int *__restrict__ cbase, int64_t nslices, int *flags) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   bool on = i + 1 < nslices;
@@ -1252,11 +1252,39 @@ __global__ __launch_bounds__(kBlock) void k_slice_runs(int *__restrict__ cbase, 
   }
   if (i < nslices) cbase[i * kMeta + kRunAt] = on;
   const int n = __popcll(__ballot(on));
-  if (n && (threadIdx.x & 63) == 0) atomicAdd(&flags[kRunSlices], n);
+  const int wide = __popcll(__ballot(i < nslices && cbase[i * kMeta + kSlots] == kFormWide));
+  if ((threadIdx.x & 63) == 0) {
+    if (n) atomicAdd(&flags[kRunSlices], n);
+    if (wide) atomicAdd(&flags[kWideSlices], wide);
+  }
 }
 
 __global__ void k_clear_flags(int *flags) {
   if (threadIdx.x < kFormFlags) flags[threadIdx.x] = 0;
+}
+
+// The distances of the slots' columns from the rows of each block, where they
+// are one over the block: a stencil level with even extents in x and y and its
+// rows in natural order numbers the rows of all its blocks alike (block_index).
+static std::vector<BlockCols> block_cols(const Layout &a) {
+  if (a.general || a.strip || a.nx % 2 || a.ny % 2 || a.npad >= ((int64_t)1 << 30)) return {};
+  std::vector<BlockCols> out(kColours);
+  const int64_t NX = a.nx / 2, NY = a.ny / 2;
+  for (int k = 0; k < kColours; ++k) {
+    BlockCols &b = out[k];
+    for (int s = 0; s < kSlots; ++s) {
+      const int d[3] = {s % 3 - 1, s / 3 % 3 - 1, s / 9 - 1};
+      int64_t step[3];  // in the blocks' coordinates: row X of class bit c lies at 2 X + c
+      int cls = 0;
+      for (int ax = 0; ax < 3; ++ax) {
+        const int from = (a.cls[k] >> ax) & 1, to = (from + d[ax]) & 1;
+        cls |= to << ax;
+        step[ax] = (from + d[ax] - to) / 2;
+      }
+      b.off[s] = (int)(a.start[a.pos[cls]] - a.start[k] + (step[2] * NY + step[1]) * NX + step[0]);
+    }
+  }
+  return out;
 }
 
 // Launches the building of a level's compact columns and value forms; the
@@ -1264,11 +1292,16 @@ __global__ void k_clear_flags(int *flags) {
 static int build_compact_cols(Ctx *c, Level &L, int *flags) {
   const int64_t ns = L.lay.npad / kSlice;
   int rc;
+  L.bcols = block_cols(L.lay);
   if ((rc = dalloc(c, (void **)&L.cbase, (size_t)ns * kMeta * sizeof(int), false))) return rc;
   if ((rc = dalloc(c, (void **)&L.cdelta, (size_t)L.lay.npad * kSlots * sizeof(int8_t), false))) return rc;
   if ((rc = dalloc(c, (void **)&L.slotv, form_bytes(L), false))) return rc;
   uint32_t *mask = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(L.slotv) + kSlotvBytes);
   L.cform = reinterpret_cast<uint8_t *>(mask + L.lay.npad);
+  if (!L.bcols.empty()) {
+    L.boffs = reinterpret_cast<int *>(reinterpret_cast<char *>(L.slotv) + kBoffsAt);
+    HPCGX_HIP(c, hipMemcpyAsync(L.boffs, L.bcols.data(), kColours * sizeof(BlockCols), hipMemcpyHostToDevice, c->stream));
+  }
   if (!L.lay.general) {
     L.vmask = mask;
     k_slot_values<<<1, kColours * kSampleRows, 0, c->stream>>>(L.ldev, L.vals, L.cols, L.slotv, level_offs(L), flags);
@@ -1280,7 +1313,7 @@ static int build_compact_cols(Ctx *c, Level &L, int *flags) {
   k_compact_cols<<<grid, kBlock, 0, c->stream>>>(L.cols, L.vals, L.dslot, L.cbase, L.cdelta, L.cform, ns,
                                                  L.lay.npad, L.iperm, L.slotv, L.field, L.vmask, level_offs(L), L.ldev,
                                                  flags);
-  if (L.vmask) k_slice_runs<<<nblk(ns), kBlock, 0, c->stream>>>(L.cbase, ns, flags);
+  k_slice_runs<<<nblk(ns), kBlock, 0, c->stream>>>(L.cbase, ns, flags);
   HPCGX_CHECK_LAUNCH(c);
   return HPCGX_OK;
 }
