@@ -364,17 +364,70 @@ static int ensure_hist(Ctx *c, int max_iter) {
   return HPCGX_OK;
 }
 
-static int read_scalar(Ctx *c, int which, double *out) {
-  HPCGX_HIP(c, hipMemcpyAsync(c->hbuf, c->scal + which, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HPCGX_HIP(c, hipStreamSynchronize(c->stream));
-  *out = c->hbuf[0];
+// The solvers' V-cycle z = M^-1 r on their own vectors.
+static int solver_mg_launches(Ctx *c, int variant, int64_t *nrz) {
+  if (variant == HPCGX_CG_MIXED_FP16) return mg_fp16_scaled(c, c->levels[0].r16, c->cg_z32);
+  if (variant == HPCGX_CG_MIXED_FP32) return mg_fp32(c, 0, c->cg_r32, c->cg_z32);
+  return mg_fp64(c, 0, c->cg_r, c->cg_z, nrz ? c->partials : nullptr, nrz);
+}
+
+// Level-0 rows up to which the host is what a solve waits for: a V-cycle is up
+// to 95 launches, which cost the host 4 us each, 7 after it has waited for the
+// GPU.  On larger levels the GPU is behind the host anyway, and a replay (or a
+// V-cycle launched ahead) was 1 to 2 % slower (kappa 256x192x144, FP16 MG: 117
+// against 120 ms).
+constexpr int64_t kHostBoundRows = (int64_t)1 << 22;
+
+// solver_mg_launches, from a graph once it has been recorded: one launch, and
+// the GPU starts each kernel sooner after the last.  Solves, launches -> graph
+// and V-cycles ahead (run_ahead): 64^3 to 1e-9 14.4 -> 11.4 ms, 96^3 FP16 MG 27.5 ->
+// 23.3, 104^3 33.5 -> 30.4, 50 iterations at 64^3 14.4 -> 13.3.  Not where the whole
+// V-cycle is two launches (k_tail).
+//
+// Recorded in a solve's second iteration (the first has then been through every
+// kernel) on the context's own stream, 0.2 ms; it holds the context's own vectors
+// alone, is kept between solves, and is dropped when a level, a copy or the
+// format changes (drop_graphs).  If it cannot be recorded the launches stay.
+static int solver_mg(Ctx *c, int variant, int64_t *nrz, bool record) {
+  const int64_t np = c->levels[0].lay.npad;
+  hipGraphExec_t &exec = c->mg_graph[variant];
+  if (!exec && record && !c->graphs_off && np > kTailRows && np <= kHostBoundRows) {
+    const hipStream_t stream = c->stream;
+    hipGraph_t graph = nullptr;
+    int rc = HPCGX_EHIP;
+    if (hipStreamBeginCapture(c->own_stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+      c->stream = c->own_stream;
+      rc = solver_mg_launches(c, variant, nrz);
+      c->stream = stream;
+      if (hipStreamEndCapture(c->own_stream, &graph) != hipSuccess) rc = HPCGX_EHIP;
+    }
+    if (rc == HPCGX_OK && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) exec = nullptr;
+    if (graph) (void)hipGraphDestroy(graph);
+    if (exec && nrz) c->mg_nrz = *nrz;
+    if (!exec) {
+      c->graphs_off = true;
+      (void)hipGetLastError();
+    }
+  }
+  if (!exec) return solver_mg_launches(c, variant, nrz);
+  if (nrz) *nrz = c->mg_nrz;
+  HPCGX_HIP(c, hipGraphLaunch(exec, c->stream));
   return HPCGX_OK;
+}
+
+// Whether the next V-cycle is launched before the norm of this iteration is
+// known: on levels where the host is slow to restart, and while the last norm is
+// well above the tolerance, so that one iteration does not reach it.  (If it
+// does, the V-cycle was for nothing: it writes z alone.)
+static bool run_ahead(const Ctx *c, double normr, double normr0, double tol) {
+  return c->levels[0].lay.npad <= kHostBoundRows && normr / normr0 > 8.0 * tol;
 }
 
 // Per-phase timing with events recorded between the phases of an iteration
 // (times[1] dot, [2] WAXPBY, [3] SpMV, [5] MG; the fused update kernel is
-// counted as WAXPBY).  `ev` is the iteration's 6 events: c->ev when the
-// host waits for every iteration, a run of c->evpool in a deferred batch.
+// counted as WAXPBY).  `ev` is the iteration's 6 events of c->evpool: two sets in
+// turn when the host waits for every iteration (the next V-cycle may be under
+// way by then), one set per iteration in a deferred batch.
 struct PhaseTimer {
   Ctx *c;
   bool on;
@@ -383,8 +436,8 @@ struct PhaseTimer {
   void mark(int i) {
     if (on) (void)hipEventRecord(ev[i], c->stream);
   }
-  void collect(const hipEvent_t *e) {  // after a stream sync: e0..e5 = MG | rz | p | spmv | update
-    if (!on) return;
+  void collect(const hipEvent_t *e) {  // e0..e5 = MG | rz | p | spmv | update
+    if (!on || hipEventSynchronize(e[5]) != hipSuccess) return;
     float ms;
     static const int slot[5] = {5, 1, 2, 3, 2};
     for (int i = 0; i < 5; ++i)
@@ -419,9 +472,9 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
   if ((rc = spmv_fp64(c, 0, x, Ap))) return rc;
   k_cg_residual<false><<<G, kBlock, 0, c->stream>>>(np, b, Ap, r, nullptr, c->partials);
   HPCGX_CHECK_LAUNCH(c);
-  if ((rc = finish(c, 1, G, F_NORMR2))) return rc;
+  if ((rc = finish(c, 1, G, F_NORMR2, nullptr, c->hsum))) return rc;
   double n2;
-  if ((rc = read_scalar(c, S_NORMR2, &n2))) return rc;
+  if ((rc = wait_host(c, c->hsum, &n2))) return rc;
   double normr = std::sqrt(n2);
   const double normr0 = normr;
   if (hist) hist[0] = normr;
@@ -435,24 +488,29 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
   // the few old entries it does read (times a zero matrix entry) must be
   // finite, which a solve that ended on a NaN may not have left.
   if (precond && (rc = zero_vec(c, z, np))) return rc;
-  if (deferred && ((rc = ensure_hist(c, kDeferBatch)) || (rc = ensure_evpool(c, times ? 6 * kDeferBatch : 0))))
-    return rc;
+  if (deferred && (rc = ensure_hist(c, kDeferBatch))) return rc;
+  if (times && (rc = ensure_evpool(c, 6 * (deferred ? kDeferBatch : 2)))) return rc;
+  const auto events = [&](int j) { return !times ? nullptr : &c->evpool[6 * (deferred ? (j - 1) % kDeferBatch : j & 1)]; };
+  int64_t nrz = 0;
+  const auto precondition = [&](int j) -> int {  // of iteration j
+    tm.ev = events(j);
+    tm.mark(0);
+    int e = precond ? solver_mg(c, HPCGX_CG_FP64, fuse_rz ? &nrz : nullptr, j > 1) : HPCGX_OK;
+    tm.mark(1);
+    return e;
+  };
+  bool ahead = false;  // the coming iteration's V-cycle has been launched
   const bool pairs_ok = np % 2 == 0 && ((reinterpret_cast<uintptr_t>(z) | reinterpret_cast<uintptr_t>(p) |
                                           reinterpret_cast<uintptr_t>(x)) & 15) == 0;
   int k = 1;
   while (k <= max_iter && normr / normr0 > tol) {
     const int kend = deferred ? std::min(max_iter, k + kDeferBatch - 1) : k;
     for (int j = k; j <= kend; ++j) {
-      tm.ev = !times ? nullptr : deferred ? &c->evpool[6 * (j - k)] : c->ev;
-      tm.mark(0);
+      if (!ahead && (rc = precondition(j))) return rc;
+      ahead = false;
       if (fuse_rz) {  // r.z partials from the V-cycle's post-smoother
-        int64_t nrz = 0;
-        if ((rc = mg_fp64(c, 0, r, z, c->partials, &nrz))) return rc;
-        tm.mark(1);
         if ((rc = finish(c, 1, nrz, j == 1 ? F_RZ_FIRST : F_RZ))) return rc;
       } else {
-        if (precond && (rc = mg_fp64(c, 0, r, z))) return rc;
-        tm.mark(1);
         k_cg_rz<double><<<G, kBlock, 0, c->stream>>>(np, r, z, c->partials);
         if ((rc = finish(c, 1, G, j == 1 ? F_RZ_FIRST : F_RZ))) return rc;
       }
@@ -466,7 +524,7 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
       if ((rc = finish(c, 1, T, F_PAP))) return rc;
       tm.mark(4);
       k_cg_update_r<<<G, kBlock, 0, c->stream>>>(np, r, Ap, c->partials, c->scal);
-      if ((rc = finish(c, 1, G, F_NORMR2, deferred ? c->hist + (j - k) : nullptr))) return rc;
+      if ((rc = finish(c, 1, G, F_NORMR2, deferred ? c->hist + (j - k) : nullptr, deferred ? nullptr : c->hsum))) return rc;
       tm.mark(5);
       HPCGX_CHECK_LAUNCH(c);
     }
@@ -474,12 +532,16 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
       HPCGX_HIP(c, hipMemcpyAsync(c->hbuf, c->hist, (size_t)(kend - k + 1) * sizeof(double), hipMemcpyDeviceToHost,
                                   c->stream));
       HPCGX_HIP(c, hipStreamSynchronize(c->stream));
-    } else if ((rc = read_scalar(c, S_NORMR2, &n2))) {
-      return rc;
+    } else {
+      if (precond && k < max_iter && run_ahead(c, normr, normr0, tol)) {
+        if ((rc = precondition(k + 1))) return rc;
+        ahead = true;
+      }
+      if ((rc = wait_host(c, c->hsum, &n2))) return rc;
     }
     // the reference's stopping test, iteration by iteration (CG.cpp:100)
     for (int j = k; j <= kend; ++j) {
-      if (times) tm.collect(deferred ? &c->evpool[6 * (j - k)] : c->ev);
+      if (times) tm.collect(events(j));
       normr = std::sqrt(deferred ? c->hbuf[j - k] : n2);
       if (hist) hist[j] = normr;
       *niters = j;
@@ -516,14 +578,24 @@ static int cg_mixed(Ctx *c, int variant, const double *b, double *x, int max_ite
   const float *dscale = f16 ? L0.dinv : nullptr;
   int rc;
   PhaseTimer tm{c, times != nullptr};
-  tm.ev = c->ev;
+  if (times && (rc = ensure_evpool(c, 12))) return rc;
+  const auto events = [&](int k) { return times ? &c->evpool[6 * (k & 1)] : nullptr; };
+  int cycles = 0;
+  const auto precondition = [&](int k) -> int {  // of iteration k
+    tm.ev = events(k);
+    tm.mark(0);
+    int e = solver_mg(c, variant, nullptr, cycles++ > 0);
+    tm.mark(1);
+    return e;
+  };
+  bool ahead = false;  // the coming iteration's V-cycle has been launched
   auto true_residual = [&](double *n2) -> int {
     int e = spmv_fp64(c, 0, x, Ap);
     if (e) return e;
     k_cg_residual<true><<<G, kBlock, 0, c->stream>>>(np, b, Ap, r, r32, c->partials, dscale);
     HPCGX_CHECK_LAUNCH(c);
-    if ((e = finish(c, 1, G, F_NORMR2))) return e;
-    return read_scalar(c, S_NORMR2, n2);
+    if ((e = finish(c, 1, G, F_NORMR2, nullptr, c->hsum))) return e;
+    return wait_host(c, c->hsum, n2);
   };
   double n2;
   if ((rc = true_residual(&n2))) return rc;
@@ -540,12 +612,11 @@ static int cg_mixed(Ctx *c, int variant, const double *b, double *x, int max_ite
       normr = std::sqrt(n2);
       if (!(normr / normr0 > tol)) break;
       restart = true;
+      ahead = false;  // r is the true residual now
     }
     ++k;
-    tm.mark(0);
-    rc = f16 ? mg_fp16_scaled(c, r32, z32) : mg_fp32(c, 0, r32, z32);
-    if (rc) return rc;
-    tm.mark(1);
+    if (!ahead && (rc = precondition(k))) return rc;
+    ahead = false;
     k_fcg_rz<<<G, kBlock, 0, c->stream>>>(np, r, z32, Ap, c->partials, restart ? 1 : 0, dscale);
     if ((rc = finish(c, 2, G, restart ? F_RZ_FIRST : F_FCG))) return rc;
     tm.mark(2);
@@ -559,15 +630,20 @@ static int cg_mixed(Ctx *c, int variant, const double *b, double *x, int max_ite
     if ((rc = finish(c, 1, T, F_PAP))) return rc;
     tm.mark(4);
     k_cg_update<true><<<G, kBlock, 0, c->stream>>>(np, x, p, r, Ap, r32, c->partials, c->scal, dscale);
-    if ((rc = finish(c, 1, G, F_NORMR2))) return rc;
+    if ((rc = finish(c, 1, G, F_NORMR2, nullptr, c->hsum))) return rc;
     tm.mark(5);
     HPCGX_CHECK_LAUNCH(c);
-    if ((rc = read_scalar(c, S_NORMR2, &n2))) return rc;
-    tm.collect(c->ev);
+    if (k < max_iter && run_ahead(c, normr, normr0, tol)) {
+      if ((rc = precondition(k + 1))) return rc;
+      ahead = true;
+    }
+    if ((rc = wait_host(c, c->hsum, &n2))) return rc;
+    tm.collect(events(k));
     normr = std::sqrt(n2);
     if (hist) hist[k] = normr;
     *niters = k;
   }
+  HPCGX_HIP(c, hipStreamSynchronize(c->stream));
   *normr_out = normr;
   *normr0_out = normr0;
   if (times) {

@@ -344,7 +344,8 @@ struct Ctx {
   double *hist = nullptr;      // device norms of a deferred-stop batch
   int hist_cap = 0;
   std::vector<hipEvent_t> evpool;  // phase events of a deferred-stop batch (6 per iteration)
-  double *hbuf = nullptr;      // pinned host scratch
+  double *hbuf = nullptr;      // pinned host scratch [64]
+  double *hsum = nullptr;      // pinned total of a finishing kernel (wait_host)
   // solver buffers (level-0 length)
   double *cg_r = nullptr, *cg_z = nullptr, *cg_p = nullptr, *cg_Ap = nullptr;
   float *cg_r32 = nullptr, *cg_z32 = nullptr;
@@ -361,6 +362,10 @@ struct Ctx {
   int prepared = 0;  // bit 1: fp32 copies, bit 2: fp16 copies
   int col_format = kColsCompact;  // column indices the kernels read (ColFormat)
   hipEvent_t ev[8] = {};
+  // the solvers' V-cycles (by HPCGX_CG_*), recorded as graphs (solver_mg)
+  hipGraphExec_t mg_graph[3] = {};
+  int64_t mg_nrz = 0;       // r.z partials that the recorded fp64 one leaves
+  bool graphs_off = false;  // recording failed on this context
 };
 
 // error handling ------------------------------------------------------------
@@ -396,8 +401,13 @@ int symgs_fp64(Ctx *c, int level, const double *r, double *x);
 int zero_vec(Ctx *c, double *x, int64_t n);
 int zero_vec(Ctx *c, float *x, int64_t n);
 int ensure_reduce(Ctx *c, int64_t grid);
-// slot (F_NORMR2 only): record the norm there and run the deferred stop test
-int finish(Ctx *c, int nv, int64_t grid, int op, double *slot = nullptr);
+// slot (F_NORMR2 only): record the norm there and run the deferred stop test.
+// host: pinned memory that receives the total too (F_DOT, F_NORMR2); wait_host
+// waits until it is there and returns it.
+int wait_host(Ctx *c, const double *host, double *out);
+int finish(Ctx *c, int nv, int64_t grid, int op, double *slot = nullptr, double *host = nullptr);
+// Drops the recorded V-cycles: whatever they point at is about to change.
+void drop_graphs(Ctx *c);
 constexpr unsigned chunk_blocks(int64_t n) { return (unsigned)((n + 4 * 256 - 1) / (4 * 256)); }
 // Looks up the static scratch of hpcgx_dot_noalloc on `device` (current).
 int noalloc_scratch_init(int device);

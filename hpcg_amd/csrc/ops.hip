@@ -601,11 +601,8 @@ int hpcgx_dot(hpcgx_ctx *c, int64_t n, const double *x, const double *y, double 
   if ((rc = check_vecs(c, m, "dot", {x, y}))) return rc;
   k_dot<<<chunk_blocks(m), kBlock, 0, c->stream>>>(m, x, y, c->partials);
   HPCGX_CHECK_LAUNCH(c);
-  if ((rc = finish(c, 1, chunk_blocks(m), F_DOT))) return rc;
-  HPCGX_HIP(c, hipMemcpyAsync(c->hbuf, c->scal + S_DOT, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HPCGX_HIP(c, hipStreamSynchronize(c->stream));
-  *result = c->hbuf[0];
-  return HPCGX_OK;
+  if ((rc = finish(c, 1, chunk_blocks(m), F_DOT, nullptr, c->hsum))) return rc;
+  return wait_host(c, c->hsum, result);
 }
 
 int hpcgx_waxpby(hpcgx_ctx *c, int64_t n, double alpha, const double *x, double beta, const double *y,
@@ -628,11 +625,8 @@ int hpcgx_waxpby_dot(hpcgx_ctx *c, int64_t n, double alpha, const double *x, dou
   if ((rc = check_vecs(c, m, "waxpby_dot", {x, y, w}))) return rc;
   k_waxpby_dot<<<chunk_blocks(m), kBlock, 0, c->stream>>>(m, alpha, x, beta, y, w, c->partials);
   HPCGX_CHECK_LAUNCH(c);
-  if ((rc = finish(c, 1, chunk_blocks(m), F_DOT))) return rc;
-  HPCGX_HIP(c, hipMemcpyAsync(c->hbuf, c->scal + S_DOT, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HPCGX_HIP(c, hipStreamSynchronize(c->stream));
-  *result = c->hbuf[0];
-  return HPCGX_OK;
+  if ((rc = finish(c, 1, chunk_blocks(m), F_DOT, nullptr, c->hsum))) return rc;
+  return wait_host(c, c->hsum, result);
 }
 
 // hpcgx_dot with its partial sums in the static scratch instead of the
@@ -666,9 +660,8 @@ int hpcgx_dot_noalloc(hpcgx_ctx *c, int64_t n, const double *x, const double *y,
     src = s + kNaFolded;
     grid = g2;
   }
-  k_finish<1><<<1, kFinishThreads, 0, c->stream>>>(src, grid, s + kNaScal, F_DOT, nullptr);
+  k_finish<1><<<1, kFinishThreads, 0, c->stream>>>(src, grid, s + kNaScal, F_DOT, nullptr, c->hbuf);
   HPCGX_CHECK_LAUNCH(c);
-  HPCGX_HIP(c, hipMemcpyAsync(c->hbuf, s + kNaScal + S_DOT, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HPCGX_HIP(c, hipStreamSynchronize(c->stream));
   *result = c->hbuf[0];
   return HPCGX_OK;

@@ -143,9 +143,34 @@ int ensure_reduce(Ctx *c, int64_t grid) {
   return HPCGX_OK;
 }
 
+// What pinned memory holds until a finishing kernel has written its total: a
+// signalling NaN, which no sum is.
+constexpr uint64_t kNoTotal = 0x7ff4c0ffee00d15cull;
+
+int wait_host(Ctx *c, const double *host, double *out) {
+  const volatile uint64_t *p = reinterpret_cast<const volatile uint64_t *>(host);
+  for (uint64_t n = 1; *p == kNoTotal; ++n) {
+    if (n % 4096) {
+#if defined(__x86_64__)
+      __builtin_ia32_pause();
+#endif
+      continue;
+    }
+    // a stream that has stopped, or is done, does not write any more
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipErrorNotReady) continue;
+    if (e != hipSuccess) return set_err(c, HPCGX_EHIP, std::string("waiting for a total : ") + hipGetErrorString(e));
+    if (*p == kNoTotal) return set_err(c, HPCGX_EHIP, "a total was not written");
+  }
+  const uint64_t bits = *p;
+  std::memcpy(out, &bits, sizeof *out);
+  return HPCGX_OK;
+}
+
 // One-block finishing kernel of a reduction over `grid` producer blocks.
-int finish(Ctx *c, int nv, int64_t grid, int op, double *slot) {
+int finish(Ctx *c, int nv, int64_t grid, int op, double *slot, double *host) {
   const double *src = c->partials;
+  if (host) *reinterpret_cast<volatile uint64_t *>(host) = kNoTotal;
   if (grid > kFoldAbove) {
     const int64_t g2 = (grid + kFold - 1) / kFold;
     if (nv == 1)
@@ -156,9 +181,9 @@ int finish(Ctx *c, int nv, int64_t grid, int op, double *slot) {
     grid = g2;
   }
   if (nv == 1)
-    k_finish<1><<<1, kFinishThreads, 0, c->stream>>>(src, grid, c->scal, op, slot);
+    k_finish<1><<<1, kFinishThreads, 0, c->stream>>>(src, grid, c->scal, op, slot, host);
   else
-    k_finish<2><<<1, kFinishThreads, 0, c->stream>>>(src, grid, c->scal, op, slot);
+    k_finish<2><<<1, kFinishThreads, 0, c->stream>>>(src, grid, c->scal, op, slot, host);
   HPCGX_CHECK_LAUNCH(c);
   return HPCGX_OK;
 }
@@ -188,7 +213,17 @@ static size_t form_bytes(const Level &L) {
   return kSlotvBytes + L.lay.npad * sizeof(uint32_t) + (size_t)(L.lay.npad / kSlice);
 }
 
+void drop_graphs(Ctx *c) {
+  for (hipGraphExec_t &g : c->mg_graph) {
+    if (!g) continue;
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipGraphExecDestroy(g);
+    g = nullptr;
+  }
+}
+
 static void free_level(Ctx *c, Level &L) {
+  drop_graphs(c);
   const size_t m = (size_t)L.lay.npad * kSlots;
   dfree(c, L.cols, m * sizeof(int));
   dfree(c, L.vals, m * sizeof(double));
@@ -927,6 +962,7 @@ static int build_compact_all(Ctx *c);
 
 int ensure_ready(Ctx *c) {
   if (c->ready) return HPCGX_OK;
+  drop_graphs(c);
   if (c->levels.empty()) return set_err(c, HPCGX_ESTATE, "no problem: upload or generate levels first");
   const int nl = (int)c->levels.size();
   int rc;
@@ -1351,6 +1387,7 @@ static int build_compact_all(Ctx *c) {
 static int build_precision(Ctx *c, int prec) {
   int rc = ensure_ready(c);
   if (rc) return rc;
+  drop_graphs(c);
   const int nl = (int)c->levels.size();
   for (int l = 0; l < nl; ++l) {
     Level &L = c->levels[l];
@@ -1448,10 +1485,11 @@ int hpcgx_create(int device, hpcgx_ctx **out) {
     hpcgx_destroy(c);
     return rc;
   }
-  if (hipHostMalloc((void **)&c->hbuf, 64 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc((void **)&c->hbuf, 72 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
     hpcgx_destroy(c);
     return HPCGX_ENOMEM;
   }
+  c->hsum = c->hbuf + 64;
   for (auto &ev : c->ev) (void)hipEventCreate(&ev);
   if (hipStreamSynchronize(c->stream) != hipSuccess) {
     hpcgx_destroy(c);
@@ -1465,6 +1503,7 @@ int hpcgx_destroy(hpcgx_ctx *c) {
   if (!c) return HPCGX_EINVAL;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
+  drop_graphs(c);
   for (auto &L : c->levels) free_level(c, L);
   for (auto &kv : c->user_vecs) (void)hipFree(const_cast<void *>(kv.first));
   (void)hipFree(c->cg_r);
@@ -1664,6 +1703,7 @@ int hpcgx_level_colouring(const hpcgx_ctx *c, int level, int *ncolours, int *gen
 int hpcgx_level_set_diagonal(hpcgx_ctx *c, int level, const double *diag) {
   if (!c || !diag || level < 0 || level >= (int)c->levels.size()) return set_err(c, HPCGX_EINVAL, "set_diagonal: bad argument");
   HPCGX_HIP(c, hipSetDevice(c->device));
+  drop_graphs(c);
   Level &L = c->levels[level];
   int rc = ensure_stage(c, L.lay.n);
   if (rc) return rc;
@@ -1714,6 +1754,7 @@ int hpcgx_set_column_format(hpcgx_ctx *c, int format) {
     return set_err(c, HPCGX_EINVAL,
                    "set_column_format: HPCGX_COLS_EXPLICIT, HPCGX_COLS_COMPACT or HPCGX_COLS_COMPACT_ALWAYS");
   HPCGX_HIP(c, hipSetDevice(c->device));
+  drop_graphs(c);
   c->col_format = format == HPCGX_COLS_COMPACT ? kColsCompact
                  : format == HPCGX_COLS_COMPACT_ALWAYS ? kColsCompactAlways : kColsExplicit;
   if (c->ready) {
