@@ -725,8 +725,8 @@ struct RunVals {
 
 // sum[j] += (SUB: -=) a x over the slots in MASK, ascending.  base: the
 // first slice's slot bases (scalars); e0: the lane's first row, from the
-// run's start; xd: x of the rows themselves.  SAFE as in gs_row.
-template <int VF, uint32_t MASK, bool SUB, bool SAFE>
+// run's start; xd: x of the rows themselves.  GUARD as in gs_value.
+template <int VF, uint32_t MASK, bool SUB, uint32_t GUARD>
 __device__ __forceinline__ void run_sum(const int (&base)[kSlots], unsigned e0, const ValSrc<double, double> &src,
                                         const RunVals<VF> &v, const double *__restrict__ x, const double (&xd)[2],
                                         double (&sum)[2]) {
@@ -744,7 +744,7 @@ __device__ __forceinline__ void run_sum(const int (&base)[kSlots], unsigned e0, 
       if (s == kDiagSlot) a = v.d[j];
       else if constexpr (VF == kValsField) a = bit_select(v.m[j], s, -((v.ki[j] + kv[j]) * 0.5));
       else a = bit_select(v.m[j], s, src.slotv[s]);
-      const double t = a * (SAFE && a == 0.0 ? 0.0 : xv[j]);
+      const double t = a * (((GUARD >> s) & 1u) && a == 0.0 ? 0.0 : xv[j]);
       if constexpr (SUB) sum[j] -= t;
       else sum[j] += t;
     }
@@ -762,7 +762,10 @@ struct RunWave {
   int base[kSlots];
   __device__ __forceinline__ void init(const ColIdx &ci, int64_t row0, int64_t nrows, int64_t tile) {
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int64_t g = (tile * (int64_t)(kBlock / kSlice) + w) * 2;
+    take(ci, row0, nrows, (tile * (int64_t)(kBlock / kSlice) + w) * 2);
+  }
+  // slices g and g + 1 of the launch
+  __device__ __forceinline__ void take(const ColIdx &ci, int64_t row0, int64_t nrows, int64_t g) {
     const int64_t left = (nrows >> 6) - g;
     row = row0 + g * kSlice;
     slices = left <= 0 ? 0 : left < 2 ? 1 : 2;
@@ -833,7 +836,7 @@ __device__ __forceinline__ void run_ax(const ColIdx &ci, const ValSrc<double, do
     v.load(src, w.row + 2 * lane);
     double xd[2];
     ld_pair(x + w.row + 2 * lane, xd);
-    run_sum<VF, kAllSlots, false, false>(w.base, 2 * lane, src, v, x, xd, out);
+    run_sum<VF, kAllSlots, false, 0>(w.base, 2 * lane, src, v, x, xd, out);
     return;
   }
 #pragma unroll 1
@@ -914,9 +917,18 @@ static_assert(masks_keep_units(2) && masks_keep_units(4), "zero-start masks spli
 // ZK == 0 reads no neighbour at all (x_i = r_i / a_ii), which holds for the
 // first block of any order, general levels included.
 // GEN: general level, the diagonal's slot is dslot[row] (stencil: slot 13).
+// GUARD: slots in which a zero entry (a neighbour outside the grid) contributes
+// 0 * 0, as the reference's zeroed x gives, whatever the row it points at
+// holds.  SAFE guards them all, in a step from x = 0 into a vector that may hold
+// anything: such an entry may point at a row not written yet in this sweep.
+// The solvers clear their level-0 buffer when a solve begins, so their level-0
+// sweeps skip the select.
+template <int ZK, bool SAFE>
+constexpr uint32_t gs_guard = ZK >= 0 && SAFE ? kAllSlots : 0;
+
 // gs_value is a row's new value, from r_i; gs_row the update of one row, which
 // returns r_i * x_i (new) for the fused r.z.
-template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, bool SAFE>
+template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, uint32_t GUARD>
 __device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &src, ACC ri, const XT *x, int64_t row,
                                        const uint8_t *__restrict__ dslot) {
   constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
@@ -936,12 +948,7 @@ __device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &
       const int c = col_at<CM, FINE>(ci, row, base, b, s);
       const ACC v = vr.at(s, c);
       const ACC xc = (ACC)x[c];
-      // SAFE (from x = 0 into a vector that may hold anything): a zero entry (a neighbour
-      // outside the grid) may point at a row not written yet in this sweep,
-      // whose old value is not trusted: it contributes 0 * 0, as the
-      // reference's zeroed x gives.  The solvers clear their level-0
-      // buffer when a solve begins, so their level-0 sweeps skip the select.
-      if constexpr (ZK >= 0 && SAFE) sum -= v * (v != (ACC)0 ? xc : (ACC)0);
+      if ((GUARD >> s) & 1u) sum -= v * (v != (ACC)0 ? xc : (ACC)0);
       else sum -= v * xc;
     }
     return sum;
@@ -951,11 +958,11 @@ __device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &
   return (XT)(sum / d);
 }
 
-template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, bool SAFE>
+template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, uint32_t GUARD>
 __device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC> &src,
                                          const XT *__restrict__ r, XT *__restrict__ x, int64_t row,
                                          const uint8_t *__restrict__ dslot) {
-  const XT xn = gs_value<VT, XT, ACC, ZK, FINE, CF, VF, GEN, SAFE>(ci, src, (ACC)r[row], x, row, dslot);
+  const XT xn = gs_value<VT, XT, ACC, ZK, FINE, CF, VF, GEN, GUARD>(ci, src, (ACC)r[row], x, row, dslot);
   x[row] = xn;
   return (double)r[row] * (double)xn;
 }
@@ -981,13 +988,13 @@ void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
   if constexpr (RZ) {
     // every thread reaches the block reduction; rows past the block add 0
     double acc = 0.0;
-    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
+    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, gs_guard<ZK, SAFE>>(ci, src, r, x, row0 + t, dslot);
     const double v[1] = {acc};
     block_partials<1>(v, rz);
     return;
   }
   if (t >= nrows) return;
-  gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, SAFE>(ci, src, r, x, row0 + t, dslot);
+  gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, gs_guard<ZK, SAFE>>(ci, src, r, x, row0 + t, dslot);
 }
 
 // The partial sums of a value per row, as the one-row-per-lane launch leaves
@@ -1022,41 +1029,118 @@ __device__ __forceinline__ void run_partials(const RunWave &w, double (&v)[2], i
   }
 }
 
+// One Gauss-Seidel step on a wave's two slices; acc[j]: r_i x_i of lane_row(j).
+template <int ZK, bool FINE, int VF, uint32_t GUARD>
+__device__ __forceinline__ void gs_run_rows(const ColIdx &ci, const ValSrc<double, double> &src, const RunWave &w,
+                                            const double *__restrict__ r, double *x, double (&acc)[2]) {
+  constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
+  acc[0] = acc[1] = 0.0;
+  if (w.run) {
+    if (!w.active) return;
+    const int64_t row = w.lane_row(0);
+    RunVals<VF> v;
+    v.load(src, row);
+    double rv[2], xd[2] = {0.0, 0.0}, xn[2];
+    ld_pair(r + row, rv);
+    if constexpr (ZK < 0) ld_pair(x + row, xd);
+    double sum[2] = {rv[0], rv[1]};
+    run_sum<VF, mask, true, GUARD>(w.base, 2 * (threadIdx.x & 63), src, v, x, xd, sum);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if constexpr (ZK < 0) sum[j] += xd[j] * v.d[j];
+      xn[j] = sum[j] / v.d[j];
+      acc[j] = rv[j] * xn[j];
+    }
+    st_pair(x + row, xn);
+    return;
+  }
+#pragma unroll 1
+  for (int j = 0; j < w.slices; ++j)
+    put(acc, j, gs_row<double, double, double, ZK, FINE, kColsSlice, VF, false, GUARD>(ci, src, r, x, w.lane_row(j), nullptr));
+}
+
 // One Gauss-Seidel step by row runs (k_gs on kValsSlot and kValsField levels).
 template <int ZK, bool FINE, int VF, bool RZ = false, bool SAFE = false>
 __global__ __launch_bounds__(kBlock) void k_gs_run(const ColIdx ci, const ValSrc<double, double> src,
                                                    const double *__restrict__ r, double *__restrict__ x,
                                                    int64_t row0, int64_t nrows, double *rz = nullptr) {
-  constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
   constexpr bool ROT = HPCGX_FINE_ROT && FINE;
   const int64_t tile = tile_id<ROT>();
   RunWave w;
   w.init(ci, row0, nrows, tile);
-  double acc[2] = {0.0, 0.0};
-  if (w.run) {
-    if (w.active) {
-      const int64_t row = w.lane_row(0);
-      RunVals<VF> v;
-      v.load(src, row);
-      double rv[2], xd[2] = {0.0, 0.0}, xn[2];
-      ld_pair(r + row, rv);
-      if constexpr (ZK < 0) ld_pair(x + row, xd);
-      double sum[2] = {rv[0], rv[1]};
-      run_sum<VF, mask, true, ZK >= 0 && SAFE>(w.base, 2 * (threadIdx.x & 63), src, v, x, xd, sum);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if constexpr (ZK < 0) sum[j] += xd[j] * v.d[j];
-        xn[j] = sum[j] / v.d[j];
-        acc[j] = rv[j] * xn[j];
-      }
-      st_pair(x + row, xn);
-    }
-  } else {
-#pragma unroll 1
-    for (int j = 0; j < w.slices; ++j)
-      put(acc, j, gs_row<double, double, double, ZK, FINE, kColsSlice, VF, false, SAFE>(ci, src, r, x, w.lane_row(j), nullptr));
-  }
+  double acc[2];
+  gs_run_rows<ZK, FINE, VF, gs_guard<ZK, SAFE>>(ci, src, w, r, x, acc);
   if constexpr (RZ) run_partials<ROT>(w, acc, tile, (nrows + kBlock - 1) / kBlock, rz);
+}
+
+// Colour steps that follow one another on two classes that differ in x alone (4
+// then 5, and 1, 0, 1 around the turn of the sweep), in one launch.
+//
+// Rows of the two classes couple only along their own grid line: a launch in
+// which each workgroup takes whole lines of both blocks, with a barrier in
+// place of the launch between the steps, updates every row from the values that
+// the separate steps would read.  A launch less is 3 to 4 us less where a step
+// is bound by its own latency; see lines_pay for where that ends.  V-cycles,
+// steps apart -> these pairs -> and those in z (k_gs_columns): 64^3 fp64 234 -> 208 ->
+// 199 us, 104^3 371 -> 326 -> 324, 128^3 fp32 376 -> 325 -> 302, kappa 104^3 fp16 342 ->
+// 299 -> 293.
+//
+// Past the end of a line, the slots along it point at another line of the
+// other block, which another workgroup may be updating: they are guarded.
+// SAFE: so are the others, in the third step too (a zero entry's row may run on
+// from its block's end into the blocks that this launch writes first).
+//
+// A row per lane, columns by the blocks' distances; a workgroup takes `rows`
+// rows (whole lines) of each block.  STEPS 3: the first block again.  ZA, ZB: the
+// steps' places in a sweep from x = 0 (ZK of k_gs), or -1.
+constexpr uint32_t kLineSlots = 1u << (kDiagSlot - 1) | 1u << (kDiagSlot + 1);
+
+template <class VT, class XT, class ACC, int ZA, int ZB, int STEPS, bool FINE, int VF, bool SAFE>
+__global__ __launch_bounds__(kBlock) void k_gs_lines(const ColIdx cia, const ColIdx cib, const ValSrc<VT, ACC> src,
+                                                     const XT *__restrict__ r, XT *x, int64_t rowa, int64_t rowb,
+                                                     int64_t nrows, int rows) {
+  constexpr uint32_t guard = SAFE ? kAllSlots : kLineSlots;
+  const int64_t i = tile_id() * rows + threadIdx.x;
+  const bool in = (int)threadIdx.x < rows && i < nrows;
+  auto step = [&](auto zk, const ColIdx &ci, int64_t row) {
+    if (in)
+      x[row] = gs_value<VT, XT, ACC, decltype(zk)::value, FINE, kColsBlock, VF, false, guard>(ci, src, (ACC)r[row], x, row, nullptr);
+  };
+  step(std::integral_constant<int, ZA>{}, cia, rowa + i);
+  __syncthreads();
+  step(std::integral_constant<int, ZB>{}, cib, rowb + i);
+  if constexpr (STEPS == 3) {
+    __syncthreads();
+    step(std::integral_constant<int, -1>{}, cia, rowa + i);
+  }
+}
+
+// The same for two classes that differ in z alone (7 then 3, 2 then 6, and
+// back): their rows couple only along z, and a workgroup takes `cols` columns of
+// both blocks through all nz planes of `plane` rows; one more takes the rows that
+// pad the blocks.  Workgroups of 512 threads were slower (64^3 223 us).
+constexpr uint32_t kColumnSlots = 1u << (kDiagSlot - 9) | 1u << (kDiagSlot + 9);
+template <class VT, class XT, class ACC, int ZA, int ZB, bool FINE, int VF, bool SAFE>
+__global__ __launch_bounds__(kBlock) void k_gs_columns(const ColIdx cia, const ColIdx cib, const ValSrc<VT, ACC> src,
+                                                       const XT *__restrict__ r, XT *x, int64_t rowa, int64_t rowb,
+                                                       int64_t nrows, int plane, int nz, int cols) {
+  constexpr uint32_t guard = SAFE ? kAllSlots : kColumnSlots;
+  const int64_t tile = tile_id();
+  const int z = (int)threadIdx.x / cols;
+  const int64_t q = tile * cols + ((int)threadIdx.x - z * cols);
+  bool in = z < nz && q < plane;
+  int64_t i = (int64_t)z * plane + q;
+  if (tile * cols >= plane) {
+    i = (int64_t)nz * plane + threadIdx.x;
+    in = i < nrows;
+  }
+  auto step = [&](auto zk, const ColIdx &ci, int64_t row) {
+    if (in)
+      x[row] = gs_value<VT, XT, ACC, decltype(zk)::value, FINE, kColsBlock, VF, false, guard>(ci, src, (ACC)r[row], x, row, nullptr);
+  };
+  step(std::integral_constant<int, ZA>{}, cia, rowa + i);
+  __syncthreads();
+  step(std::integral_constant<int, ZB>{}, cib, rowb + i);
 }
 
 // Residual at the injected rows and restriction, fused (ComputeMG_ref.cpp:49-51 +
@@ -1187,7 +1271,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
       const int end = L.start[k + 1] >> 6;
       for (int slice = (L.start[k] >> 6) + wave; slice < end; slice += nw) {
         const int row = slice * kSlice + lane;
-        x[row] = gs_value<VT, XT, ACC, -1, false, CF, VF, GEN, false>(L.ci, L.src, (ACC)lds[L.roff + row], x, row, L.dslot);
+        x[row] = gs_value<VT, XT, ACC, -1, false, CF, VF, GEN, 0>(L.ci, L.src, (ACC)lds[L.roff + row], x, row, L.dslot);
       }
       __syncthreads();
     }

@@ -70,18 +70,79 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
   });
 }
 
+// Whether steps on blocks whose classes differ in x alone share a launch
+// (k_gs_lines).  They must lie at one distance per slot (block_cols: even extents
+// in x and y, so the lines of the two blocks are alike).  Blocks of up to
+// 2^18 rows: the pairs of a 104^3 and a 128^3 fine level (140608 and 262144 rows)
+// gain 23 and 15 us a V-cycle, those of 192^3 (884736) lose 90.
+static bool lines_pay(const Ctx *c, const Level &L) {
+  return !L.bcols.empty() && col_idx(c, L, 0).off && L.lay.start[1] <= (1 << 18) && L.lay.nx / 2 <= kBlock;
+}
+
+// Whether steps on blocks whose classes differ in z alone do (k_gs_columns): an even
+// extent in z, so the blocks have the same planes, and at least 4 columns of
+// them in a workgroup.  Blocks of up to 2^16 rows: 32768 rows gain 3 us a pair,
+// 110592 lose 3 (a workgroup's columns are then a few short pieces of lines).
+static bool columns_pay(const Ctx *c, const Level &L) {
+  return !L.bcols.empty() && col_idx(c, L, 0).off && L.lay.start[1] <= (1 << 16) && L.lay.nz % 2 == 0 &&
+         L.lay.nz / 2 <= kBlock / 4;
+}
+
+// Steps of blocks a, b (STEPS 3: and a again), whose classes differ in x alone.
+template <class VT, class XT, class ACC, int ZA, int ZB, int STEPS, bool FINE, bool SAFE = false>
+static void gs_lines(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b) {
+  if (!lines_pay(c, L)) {
+    gs_block<VT, XT, ACC, ZA, FINE, SAFE>(c, L, r, x, a);
+    gs_block<VT, XT, ACC, ZB, FINE, SAFE>(c, L, r, x, b);
+    if constexpr (STEPS == 3) gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, a);
+    return;
+  }
+  const int64_t ra = L.lay.start[a], rb = L.lay.start[b], nr = L.lay.start[a + 1] - ra;
+  const int line = L.lay.nx / 2, rows = line <= kSlice ? kSlice / line * line : line;
+  const unsigned grid = (unsigned)((nr + rows - 1) / rows), bs = (unsigned)(rows + kSlice - 1) / kSlice * kSlice;
+  const ColIdx cia = col_idx(c, L, a), cib = col_idx(c, L, b);
+  with_forms<VT>(L, cia, [&](auto CF, auto VF) {
+    if constexpr (CF() != kColsStored)
+      k_gs_lines<VT, XT, ACC, ZA, ZB, STEPS, FINE, VF(), SAFE>
+          <<<grid, bs, 0, c->stream>>>(cia, cib, val_src<VT, ACC>(L), r, x, ra, rb, nr, rows);
+  });
+}
+
+// Steps of blocks a, b, whose classes differ in z alone.
+template <class VT, class XT, class ACC, int ZA, int ZB, bool FINE, bool SAFE = false>
+static void gs_columns(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b) {
+  if (!columns_pay(c, L)) {
+    gs_block<VT, XT, ACC, ZA, FINE, SAFE>(c, L, r, x, a);
+    gs_block<VT, XT, ACC, ZB, FINE, SAFE>(c, L, r, x, b);
+    return;
+  }
+  const int64_t ra = L.lay.start[a], rb = L.lay.start[b], nr = L.lay.start[a + 1] - ra;
+  const int plane = L.lay.nx / 2 * (L.lay.ny / 2), nz = L.lay.nz / 2, cols = kBlock / nz;
+  const unsigned grid = (unsigned)((plane + cols - 1) / cols) + (nr > (int64_t)plane * nz ? 1 : 0);
+  const ColIdx cia = col_idx(c, L, a), cib = col_idx(c, L, b);
+  with_forms<VT>(L, cia, [&](auto CF, auto VF) {
+    if constexpr (CF() != kColsStored)
+      k_gs_columns<VT, XT, ACC, ZA, ZB, FINE, VF(), SAFE>
+          <<<grid, kBlock, 0, c->stream>>>(cia, cib, val_src<VT, ACC>(L), r, x, ra, rb, nr, plane, nz, cols);
+  });
+}
+
 // The zero-start forward sweep of the default order: block k reads only the
-// blocks swept before it.
+// blocks swept before it.  The backward step of block 6 comes with it.
 template <class VT, class XT, class ACC, bool FINE, bool SAFE>
 static void zero_start_forward(Ctx *c, const Level &L, const XT *r, XT *x) {
-  gs_block<VT, XT, ACC, 0, FINE, SAFE>(c, L, r, x, 0);
-  gs_block<VT, XT, ACC, 1, FINE, SAFE>(c, L, r, x, 1);
-  gs_block<VT, XT, ACC, 2, FINE, SAFE>(c, L, r, x, 2);
-  gs_block<VT, XT, ACC, 3, FINE, SAFE>(c, L, r, x, 3);
-  gs_block<VT, XT, ACC, 4, FINE, SAFE>(c, L, r, x, 4);
-  gs_block<VT, XT, ACC, 5, FINE, SAFE>(c, L, r, x, 5);
-  gs_block<VT, XT, ACC, 6, FINE, SAFE>(c, L, r, x, 6);
-  gs_block<VT, XT, ACC, 7, FINE, SAFE>(c, L, r, x, 7);
+  gs_columns<VT, XT, ACC, 0, 1, FINE, SAFE>(c, L, r, x, 0, 1);
+  gs_lines<VT, XT, ACC, 2, 3, 2, FINE, SAFE>(c, L, r, x, 2, 3);
+  gs_columns<VT, XT, ACC, 4, 5, FINE, SAFE>(c, L, r, x, 4, 5);
+  gs_lines<VT, XT, ACC, 6, 7, 3, FINE, SAFE>(c, L, r, x, 6, 7);
+}
+
+// The remaining backward steps of the default order, from block 5.
+template <class VT, class XT, class ACC, bool FINE>
+static void backward_from_5(Ctx *c, const Level &L, const XT *r, XT *x) {
+  gs_columns<VT, XT, ACC, -1, -1, FINE>(c, L, r, x, 5, 4);
+  gs_lines<VT, XT, ACC, -1, -1, 2, FINE>(c, L, r, x, 3, 2);
+  gs_columns<VT, XT, ACC, -1, -1, FINE>(c, L, r, x, 1, 0);
 }
 
 template <class XT>
@@ -95,6 +156,36 @@ static bool default_order(const Level &L) {
   for (int k = 0; k < kColours; ++k)
     if (L.lay.cls[k] != kDefaultOrder[k]) return false;
   return true;
+}
+
+// r.x partials of a level as its post-smoother's steps leave them (k_gs with
+// RZ): the tiles of the last block, then of the blocks down to the first, each
+// block's in the order of its launch.
+struct RzBlocks {
+  int start[kTailColours + 1];
+  int ncol;
+};
+__global__ __launch_bounds__(kBlock) void k_rz(const RzBlocks L, const double *__restrict__ r,
+                                               const double *__restrict__ x, double *rz) {
+  int k = L.ncol - 1, first = 0, n = 0;
+  for (;; --k) {
+    n = (L.start[k + 1] - L.start[k] + kBlock - 1) / kBlock;
+    if ((int)blockIdx.x < first + n) break;
+    first += n;
+  }
+  const int64_t row = L.start[k] + tile_at<HPCGX_FINE_ROT != 0>((int)blockIdx.x - first, n) * kBlock + threadIdx.x;
+  const double v[1] = {row < L.start[k + 1] ? r[row] * x[row] : 0.0};
+  block_partials<1>(v, rz);
+}
+// Returns the number of partials.
+static int64_t rz_pass(Ctx *c, const Level &L, const double *r, const double *x, double *rz) {
+  RzBlocks b;
+  b.ncol = L.lay.ncol;
+  int64_t n = 0;
+  for (int k = 0; k <= b.ncol; ++k) b.start[k] = (int)L.lay.start[k];
+  for (int k = 0; k < b.ncol; ++k) n += tiles(b.start[k + 1] - b.start[k]);
+  k_rz<<<(unsigned)n, kBlock, 0, c->stream>>>(b, r, x, rz);
+  return n;
 }
 
 // One symmetric Gauss-Seidel step over the colour blocks.  Forward sweep
@@ -120,6 +211,19 @@ static void sweep(Ctx *c, const Level &L, const XT *r, XT *x, bool zero_start, d
   } else if (zero_start) {
     if (untrusted_x) zero_start_forward<VT, XT, ACC, FINE, true>(c, L, r, x);
     else zero_start_forward<VT, XT, ACC, FINE, false>(c, L, r, x);
+    backward_from_5<VT, XT, ACC, FINE>(c, L, r, x);
+    return;
+  } else if (default_order(L) && (!rz || lines_pay(c, L))) {
+    gs_columns<VT, XT, ACC, -1, -1, FINE>(c, L, r, x, 0, 1);
+    gs_lines<VT, XT, ACC, -1, -1, 2, FINE>(c, L, r, x, 2, 3);
+    gs_columns<VT, XT, ACC, -1, -1, FINE>(c, L, r, x, 4, 5);
+    gs_lines<VT, XT, ACC, -1, -1, 3, FINE>(c, L, r, x, 6, 7);
+    backward_from_5<VT, XT, ACC, FINE>(c, L, r, x);
+    // a pass of its own for r.x costs less than the launches that the pairs save
+    if constexpr (sizeof(XT) == 8) {
+      if (rz) *nrz = rz_pass(c, L, r, x, rz);
+    }
+    return;
   } else {
     for (int k = 0; k + 1 < L.lay.ncol; ++k) gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, k);
     const int last = L.lay.ncol - 1;
@@ -210,26 +314,6 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
   return true;
 }
 
-// r.x partials of a level that the tail solved, as its post-smoother's steps
-// leave them (k_gs with RZ): the tiles of the last block, then of the blocks
-// down to the first, each block's in the order of its launch.
-struct TailBlocks {
-  int start[kTailColours + 1];
-  int ncol;
-};
-__global__ __launch_bounds__(kBlock) void k_tail_rz(const TailBlocks L, const double *__restrict__ r,
-                                                    const double *__restrict__ x, double *rz) {
-  int k = L.ncol - 1, first = 0, n = 0;
-  for (;; --k) {
-    n = (L.start[k + 1] - L.start[k] + kBlock - 1) / kBlock;
-    if ((int)blockIdx.x < first + n) break;
-    first += n;
-  }
-  const int64_t row = L.start[k] + tile_at<HPCGX_FINE_ROT != 0>((int)blockIdx.x - first, n) * kBlock + threadIdx.x;
-  const double v[1] = {row < L.start[k + 1] ? r[row] * x[row] : 0.0};
-  block_partials<1>(v, rz);
-}
-
 // V-cycle of ComputeMG_ref.cpp:39-63: x = 0; pre-smooth; residual + restrict;
 // recurse; prolong; post-smooth.  The coarsest level gets one smoothing step.
 // rz / nrz: r.x partials of the result from the post-smoother (see sweep);
@@ -242,14 +326,7 @@ static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64
   const Level &L = c->levels[l];
   if (tail<VT, XT, ACC, SCALE>(c, l, r, x)) {
     if constexpr (sizeof(VT) == 8) {
-      if (rz) {
-        TailBlocks b;
-        b.ncol = L.lay.ncol;
-        *nrz = 0;
-        for (int k = 0; k <= b.ncol; ++k) b.start[k] = (int)L.lay.start[k];
-        for (int k = 0; k < b.ncol; ++k) *nrz += tiles(b.start[k + 1] - b.start[k]);
-        k_tail_rz<<<(unsigned)*nrz, kBlock, 0, c->stream>>>(b, r, x, rz);
-      }
+      if (rz) *nrz = rz_pass(c, L, r, x, rz);
     }
     HPCGX_CHECK_LAUNCH(c);
     return HPCGX_OK;
