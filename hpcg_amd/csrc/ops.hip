@@ -277,12 +277,16 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
     t.inj = L.inj;
     t.frow = L.frow;
     t.sigma = L.sigma;
+    t.boffs = !L.bcols.empty() && L.diag_one ? L.boffs : nullptr;
     t.ninj = (int)L.ninj;
     t.row0 = (int)L.lay.start[L.lay.inj];
     t.npad = (int)L.lay.npad;
     t.ncol = L.lay.ncol;
     for (int j = 0; j <= L.lay.ncol; ++j) t.start[j] = (int)L.lay.start[j];
-    for (int j = 0; j < L.lay.ncol; ++j) waves = std::max(waves, (t.start[j + 1] - t.start[j]) >> 6);
+    int slices = 1;
+    for (int j = 0; j < L.lay.ncol; ++j) slices = std::max(slices, (t.start[j + 1] - t.start[j]) >> 6);
+    if (slices > kTailThreads / kSlice) t.boffs = nullptr;
+    waves = std::max(waves, slices);
     t.xoff = (int)off;
     t.roff = (int)(off + L.lay.npad);
     off += 2 * L.lay.npad;
