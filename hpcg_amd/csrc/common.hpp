@@ -263,11 +263,6 @@ __host__ __device__ inline int64_t perm_of(const LayoutDev &L, int ix, int iy, i
   return L.start[k] + block_index(L, k, ix >> 1, iy >> 1, iz >> 1);
 }
 
-// How far the column of each slot lies from the row, over a colour block.
-struct BlockCols {
-  int off[kMeta];  // padded like a slice's record
-};
-
 struct Level {
   Layout lay;
   LayoutDev ldev;
@@ -298,8 +293,9 @@ struct Level {
   // slices are wide (on a level of mostly wide slices the explicit indices
   // ran faster: a renumbered 128^3 hierarchy, 779 against 747 GFLOP/s)
   bool read_compact = false;
-  std::vector<BlockCols> bcols;  // per block, where every slot has one distance (block_cols), else empty
-  int *boffs = nullptr;          // the same on the device, kMeta ints per block
+  // kMeta ints per block: how far the column of each slot lies from the row,
+  // where that is one distance over the block (has_block_offs), else null
+  int *boffs = nullptr;
   // Value form of the fp64 matrix (ValForm).  vmask: bit s set where slot s
   // of the row stores an entry (bit 13: a row of the level, clear on
   // padding); slotv: the 27 slot values of kValsSlot, then the same for the

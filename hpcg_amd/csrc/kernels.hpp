@@ -338,7 +338,7 @@ struct ColIdx {
 // uses it and the level reads it (Level::read_compact), else the explicit
 // indices.  block >= 0: the launch takes rows of that colour block alone.
 //
-// Where a block's slots have one distance each (block_cols), a launch reads the
+// Where a block's slots have one distance each (has_block_offs), a launch reads the
 // block's 27 distances, which stay in the caches, instead of a record for
 // every slice.  V-cycles, records -> distances: 192^3 fp32 581 -> 548 us, 192^3
 // kappa fp16 764 -> 709 (57 MB of records less), 64^3 245 -> 235.  Row runs keep the
@@ -351,7 +351,7 @@ inline ColIdx col_idx(const Ctx *c, const Level &L, int block = -1) {
   ci.cbase = L.cbase;
   ci.cdelta = L.cdelta;
   ci.cform = L.cform;
-  if (block >= 0 && !L.bcols.empty()) {
+  if (block >= 0 && L.boffs) {
     ci.off = L.boffs + block * kMeta;
     ci.last = (int)(L.lay.npad - 1);
   }
@@ -1245,7 +1245,7 @@ struct TailLevel {
   const int *frow;
   const float *sigma;
   int ninj, row0;
-  const int *boffs;  // the blocks' distances (block_cols) where sweep_slot takes the level, else null
+  const int *boffs;  // the blocks' distances (has_block_offs) where sweep_slot takes the level, else null
   int npad, ncol;
   int xoff, roff;    // x and r in LDS, in elements
   int start[kTailColours + 1];

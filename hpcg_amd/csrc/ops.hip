@@ -71,12 +71,12 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
 }
 
 // Whether steps on blocks whose classes differ in x alone share a launch
-// (k_gs_lines).  They must lie at one distance per slot (block_cols: even extents
+// (k_gs_lines).  They must lie at one distance per slot (has_block_offs: even extents
 // in x and y, so the lines of the two blocks are alike).  Blocks of up to
 // 2^18 rows: the pairs of a 104^3 and a 128^3 fine level (140608 and 262144 rows)
 // gain 23 and 15 us a V-cycle, those of 192^3 (884736) lose 90.
 static bool lines_pay(const Ctx *c, const Level &L) {
-  return !L.bcols.empty() && col_idx(c, L, 0).off && L.lay.start[1] <= (1 << 18) && L.lay.nx / 2 <= kBlock;
+  return L.boffs && col_idx(c, L, 0).off && L.lay.start[1] <= (1 << 18) && L.lay.nx / 2 <= kBlock;
 }
 
 // Whether steps on blocks whose classes differ in z alone do (k_gs_columns): an even
@@ -84,7 +84,7 @@ static bool lines_pay(const Ctx *c, const Level &L) {
 // them in a workgroup.  Blocks of up to 2^16 rows: 32768 rows gain 3 us a pair,
 // 110592 lose 3 (a workgroup's columns are then a few short pieces of lines).
 static bool columns_pay(const Ctx *c, const Level &L) {
-  return !L.bcols.empty() && col_idx(c, L, 0).off && L.lay.start[1] <= (1 << 16) && L.lay.nz % 2 == 0 &&
+  return L.boffs && col_idx(c, L, 0).off && L.lay.start[1] <= (1 << 16) && L.lay.nz % 2 == 0 &&
          L.lay.nz / 2 <= kBlock / 4;
 }
 
@@ -277,7 +277,7 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
     t.inj = L.inj;
     t.frow = L.frow;
     t.sigma = L.sigma;
-    t.boffs = !L.bcols.empty() && L.diag_one ? L.boffs : nullptr;
+    t.boffs = L.diag_one ? L.boffs : nullptr;
     t.ninj = (int)L.ninj;
     t.row0 = (int)L.lay.start[L.lay.inj];
     t.npad = (int)L.lay.npad;

@@ -201,12 +201,11 @@ int ensure_stage(Ctx *c, int64_t n) {
 
 // One allocation per level for the forms: the slot values (27 in fp64, 27
 // each for the fp32 and fp16 copies as fp32), each block's usual distance from
-// a row to its slots' columns, the exact ones (BlockCols), the row masks and the slices'
+// a row to its slots' columns, the exact ones (block_off), the row masks and the slices'
 // column forms.
 constexpr size_t kOffsAt = 512, kBoffsAt = 1536;
-constexpr size_t kSlotvBytes = kBoffsAt + kColours * sizeof(BlockCols);
+constexpr size_t kSlotvBytes = kBoffsAt + kColours * kMeta * sizeof(int);
 static_assert(kOffsAt >= kSlots * 16 && kBoffsAt >= kOffsAt + kColours * kSlots * sizeof(int), "");
-static_assert(sizeof(BlockCols) == kMeta * sizeof(int), "");
 constexpr int kNoOffset = INT_MIN;
 static int *level_offs(const Level &L) { return reinterpret_cast<int *>(reinterpret_cast<char *>(L.slotv) + kOffsAt); }
 static size_t form_bytes(const Level &L) {
@@ -1217,6 +1216,10 @@ __global__ __launch_bounds__(kBlock) void k_compact_cols(const int *__restrict__
   }
 }
 
+__global__ void k_clear_flags(int *flags) {
+  if (threadIdx.x < kFormFlags) flags[threadIdx.x] = 0;
+}
+
 // The diagonals alone, after they were replaced.
 __global__ __launch_bounds__(kBlock) void k_check_diag(const double *__restrict__ vals, const uint32_t *__restrict__ vmask,
                                                        const double *__restrict__ slotv, int64_t npad, int *flags) {
@@ -1225,24 +1228,62 @@ __global__ __launch_bounds__(kBlock) void k_check_diag(const double *__restrict_
   if (__any(bad) && (threadIdx.x & 63) == 0) flags[kBadDiag] = 1;
 }
 
+// Distance of slot s's column from a row of block k where the level has even
+// extents in x and y and no strips (has_block_offs).
+__host__ __device__ inline int block_off(const LayoutDev &a, int k, int s) {
+  const int d[3] = {s % 3 - 1, s / 3 % 3 - 1, s / 9 - 1};
+  int64_t step[3];  // in the blocks' coordinates: row X of class bit c lies at 2 X + c
+  int cls = 0;
+  for (int ax = 0; ax < 3; ++ax) {
+    const int from = (a.cls[k] >> ax) & 1, to = (from + d[ax]) & 1;
+    cls |= to << ax;
+    step[ax] = (from + d[ax] - to) / 2;
+  }
+  const int64_t NX = a.nx / 2, NY = a.ny / 2;
+  return (int)(a.start[a.pos[cls]] - a.start[k] + (step[2] * NY + step[1]) * NX + step[0]);
+}
+
 // The candidate value of each slot: the first stored entry met in that slot
 // among 32 rows spread over each colour block (all rows of a small block; a
 // slot that they all miss keeps +0).  k_compact_cols then checks every row.
 // offs[k][s]: how far the column of slot s lies from the row, on the first
 // such row of block k (kNoOffset: none).
-// One workgroup, a row per thread; also clears the flags and derives the slot
-// values of the lower-precision copies with the roundings of k_to_f32 and
-// k_to_f16_scaled.
+// One workgroup a level, a row per thread; also clears the flags, writes the
+// blocks' distances (block_off) and derives the slot values of the
+// lower-precision copies with the roundings of k_to_f32 and k_to_f16_scaled.
+// All levels share the launch: it is a chain of a few loads, and one after
+// another, with a copy of the distances each, they made hpcgx_problem_generate
+// of 48^3 (4 levels) 505-528 us, now 445-463 (80x48x112: 696-725 -> 632-662).
 constexpr int kSampleRows = 32;
-__global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(LayoutDev L, const double *__restrict__ vals,
-                                                                        const int *__restrict__ cols, double *slotv,
-                                                                        int *offs, int *flags) {
+static_assert(kMeta == kSampleRows, "a thread per entry of the blocks' distances");
+struct FormLevel {
+  LayoutDev L;
+  const double *vals;  // null: a general level (flags only)
+  const int *cols;
+  double *slotv;
+  int *offs, *boffs, *flags;  // boffs null: no distances
+  int *cbase;
+  int64_t nslices;
+};
+struct FormLevels {
+  FormLevel lv[kMaxLevels];
+};
+static_assert(sizeof(FormLevels) <= 4096, "kernel argument");
+__global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(const FormLevels todo) {
+  const FormLevel &F = todo.lv[blockIdx.x];
+  const LayoutDev &L = F.L;
+  const double *__restrict__ vals = F.vals;
+  const int *__restrict__ cols = F.cols;
+  double *slotv = F.slotv;
+  int *offs = F.offs;
   __shared__ int first[kSlots];
   const int t = threadIdx.x;
   if (t < kSlots) first[t] = INT_MAX;
-  if (t < kFormFlags) flags[t] = 0;
+  if (t < kFormFlags) F.flags[t] = 0;
+  if (!vals) return;
   __syncthreads();
   const int k = t / kSampleRows, i = t % kSampleRows;
+  if (F.boffs) F.boffs[t] = i < kSlots ? block_off(L, k, i) : 0;
   const int64_t count = (int64_t)L.nb[k][0] * L.nb[k][1] * L.nb[k][2];
   const bool in = i < count;
   // evenly spaced and shifted by one row each, so the samples of a block do
@@ -1277,7 +1318,10 @@ __global__ __launch_bounds__(kColours * kSampleRows) void k_slot_values(LayoutDe
 }
 // Whether each slice continues in the next one: both are uniform and each
 // slot's base is 64 rows further.  Counts those that do, and the wide ones.
-__global__ __launch_bounds__(kBlock) void k_slice_runs(int *__restrict__ cbase, int64_t nslices, int *flags) {
+__global__ __launch_bounds__(kBlock) void k_slice_runs(const FormLevels todo) {
+  int *__restrict__ cbase = todo.lv[blockIdx.y].cbase;
+  int *flags = todo.lv[blockIdx.y].flags;
+  const int64_t nslices = todo.lv[blockIdx.y].nslices;
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   bool on = i + 1 < nslices;
   if (on) {
@@ -1295,62 +1339,24 @@ __global__ __launch_bounds__(kBlock) void k_slice_runs(int *__restrict__ cbase, 
   }
 }
 
-__global__ void k_clear_flags(int *flags) {
-  if (threadIdx.x < kFormFlags) flags[threadIdx.x] = 0;
+// Whether the distance of a slot's column from the row is one over each
+// block: a stencil level with even extents in x and y and its rows in natural
+// order numbers the rows of all its blocks alike (block_index).
+static bool has_block_offs(const Layout &a) {
+  return !a.general && !a.strip && a.nx % 2 == 0 && a.ny % 2 == 0 && a.npad < ((int64_t)1 << 30);
 }
 
-// The distances of the slots' columns from the rows of each block, where they
-// are one over the block: a stencil level with even extents in x and y and its
-// rows in natural order numbers the rows of all its blocks alike (block_index).
-static std::vector<BlockCols> block_cols(const Layout &a) {
-  if (a.general || a.strip || a.nx % 2 || a.ny % 2 || a.npad >= ((int64_t)1 << 30)) return {};
-  std::vector<BlockCols> out(kColours);
-  const int64_t NX = a.nx / 2, NY = a.ny / 2;
-  for (int k = 0; k < kColours; ++k) {
-    BlockCols &b = out[k];
-    for (int s = 0; s < kSlots; ++s) {
-      const int d[3] = {s % 3 - 1, s / 3 % 3 - 1, s / 9 - 1};
-      int64_t step[3];  // in the blocks' coordinates: row X of class bit c lies at 2 X + c
-      int cls = 0;
-      for (int ax = 0; ax < 3; ++ax) {
-        const int from = (a.cls[k] >> ax) & 1, to = (from + d[ax]) & 1;
-        cls |= to << ax;
-        step[ax] = (from + d[ax] - to) / 2;
-      }
-      b.off[s] = (int)(a.start[a.pos[cls]] - a.start[k] + (step[2] * NY + step[1]) * NX + step[0]);
-    }
-  }
-  return out;
-}
-
-// Launches the building of a level's compact columns and value forms; the
-// flags come back in read_forms.
-static int build_compact_cols(Ctx *c, Level &L, int *flags) {
+// Buffers of a level's compact columns and value forms.
+static int alloc_forms(Ctx *c, Level &L) {
   const int64_t ns = L.lay.npad / kSlice;
   int rc;
-  L.bcols = block_cols(L.lay);
   if ((rc = dalloc(c, (void **)&L.cbase, (size_t)ns * kMeta * sizeof(int), false))) return rc;
   if ((rc = dalloc(c, (void **)&L.cdelta, (size_t)L.lay.npad * kSlots * sizeof(int8_t), false))) return rc;
   if ((rc = dalloc(c, (void **)&L.slotv, form_bytes(L), false))) return rc;
   uint32_t *mask = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(L.slotv) + kSlotvBytes);
   L.cform = reinterpret_cast<uint8_t *>(mask + L.lay.npad);
-  if (!L.bcols.empty()) {
-    L.boffs = reinterpret_cast<int *>(reinterpret_cast<char *>(L.slotv) + kBoffsAt);
-    HPCGX_HIP(c, hipMemcpyAsync(L.boffs, L.bcols.data(), kColours * sizeof(BlockCols), hipMemcpyHostToDevice, c->stream));
-  }
-  if (!L.lay.general) {
-    L.vmask = mask;
-    k_slot_values<<<1, kColours * kSampleRows, 0, c->stream>>>(L.ldev, L.vals, L.cols, L.slotv, level_offs(L), flags);
-  } else {
-    k_clear_flags<<<1, 64, 0, c->stream>>>(flags);
-  }
-  HPCGX_CHECK_LAUNCH(c);
-  const int64_t grid = (ns + (kBlock / kSlice) - 1) / (kBlock / kSlice);
-  k_compact_cols<<<grid, kBlock, 0, c->stream>>>(L.cols, L.vals, L.dslot, L.cbase, L.cdelta, L.cform, ns,
-                                                 L.lay.npad, L.iperm, L.slotv, L.field, L.vmask, level_offs(L), L.ldev,
-                                                 flags);
-  k_slice_runs<<<nblk(ns), kBlock, 0, c->stream>>>(L.cbase, ns, flags);
-  HPCGX_CHECK_LAUNCH(c);
+  if (has_block_offs(L.lay)) L.boffs = reinterpret_cast<int *>(reinterpret_cast<char *>(L.slotv) + kBoffsAt);
+  if (!L.lay.general) L.vmask = mask;
   return HPCGX_OK;
 }
 
@@ -1361,12 +1367,33 @@ static int build_compact_all(Ctx *c) {
   int *dev = reinterpret_cast<int *>(c->scal + S_COUNT);
   bool built[kMaxLevels] = {};
   const int nl = (int)c->levels.size();
+  FormLevels todo = {};
+  unsigned nb = 0, runs_grid = 0;
   for (int l = 0; l < nl; ++l) {
     Level &L = c->levels[l];
     if (L.cbase) continue;
-    int rc = build_compact_cols(c, L, dev + l * kFormFlags);
+    int rc = alloc_forms(c, L);
     if (rc) return rc;
     built[l] = true;
+    const int64_t ns = L.lay.npad / kSlice;
+    todo.lv[nb++] = {L.ldev, L.vmask ? L.vals : nullptr, L.cols, L.slotv, level_offs(L), L.boffs, dev + l * kFormFlags,
+                     L.cbase, ns};
+    runs_grid = std::max(runs_grid, (unsigned)nblk(ns));
+  }
+  if (nb) {
+    k_slot_values<<<nb, kColours * kSampleRows, 0, c->stream>>>(todo);
+    HPCGX_CHECK_LAUNCH(c);
+    for (int l = 0; l < nl; ++l) {
+      if (!built[l]) continue;
+      Level &L = c->levels[l];
+      const int64_t ns = L.lay.npad / kSlice, grid = (ns + (kBlock / kSlice) - 1) / (kBlock / kSlice);
+      k_compact_cols<<<grid, kBlock, 0, c->stream>>>(L.cols, L.vals, L.dslot, L.cbase, L.cdelta, L.cform, ns,
+                                                     L.lay.npad, L.iperm, L.slotv, L.field, L.vmask, level_offs(L),
+                                                     L.ldev, dev + l * kFormFlags);
+      HPCGX_CHECK_LAUNCH(c);
+    }
+    k_slice_runs<<<dim3(runs_grid, nb), kBlock, 0, c->stream>>>(todo);
+    HPCGX_CHECK_LAUNCH(c);
   }
   int *flags = reinterpret_cast<int *>(c->hbuf);
   HPCGX_HIP(c, hipMemcpyAsync(flags, dev, kMaxLevels * kFormFlags * sizeof(int), hipMemcpyDeviceToHost, c->stream));

@@ -208,34 +208,47 @@ def index_bytes_per_slot(forms):
     return fd * 1.0 + fw * 4.0 + (fu + fd) * 4.0 / 64.0
 
 
-def implementation_bytes_per_iteration(nx, ny, nz, levels=4, v=8, s=8, forms=None, order=DEFAULT_ORDER):
+def implementation_bytes_per_iteration(nx, ny, nz, levels=4, v=8, s=8, forms=None, order=DEFAULT_ORDER, slot=False):
     """Bytes the FP64 iteration's kernels move as built, in the convention
-    of algorithmic_bytes_per_iteration (each array element once per pass,
-    neighbour gathers not counted), but counting matrix slots as loaded: all
+    of algorithmic_bytes_per_iteration (each array element once per pass),
+    but counting matrix slots as loaded: all
     27 slots of a row (the zeros of rows at the grid boundary included), only
     the slots of blocks swept before in the zero-start forward sweep (plus
     the diagonal), 15 colour steps per symmetric sweep (the last block's
     backward step is elided), column-index bytes per the level's column
     forms (forms[l], see index_bytes_per_slot), no separate r.z pass (its
     partials come from the post-smoother).  Even grids (every colour block
-    holds n/8 rows)."""
+    holds n/8 rows).
+
+    slot: the levels whose values are one constant per slot (the HPCG matrix
+    in compact columns): a row's matrix is a 4-byte mask.  The neighbours'
+    x is then most of what a pass moves and is counted, each block that the
+    pass reads once; without slot the gathers are not counted."""
     shapes = level_shapes(nx, ny, nz, levels)
     zs = zero_start_slots(order)
     total = 0.0
     for l, (n, m, d) in enumerate(shapes):
-        ib = index_bytes_per_slot(None if forms is None else forms[l])
         nb = n / 8.0
-        full = 27 * (v + ib) + 3 * s
-        # zero-start forward sweep: block k reads zs[k] neighbour slots, the diagonal, r; writes x
-        pre = sum(nb * (zs[k] * (v + ib) + v + 2 * s) for k in range(8)) + 7 * nb * full
-        total += pre
+        nc = shapes[l + 1][0] if l + 1 < levels else 0
+        if slot:
+            full = nb * (4 + 2 * s) + n * s       # mask, r, x out; x of the level
+            total += sum(nb * (4 + 2 * s) + k * nb * s for k in range(8)) + 7 * full
+            matrix_rows = nb * 4 + n * s          # the injected rows' residual
+        else:
+            ib = index_bytes_per_slot(None if forms is None else forms[l])
+            full = nb * (27 * (v + ib) + 3 * s)
+            # zero-start forward sweep: block k reads zs[k] neighbour slots, the diagonal, r; writes x
+            total += sum(nb * (zs[k] * (v + ib) + v + 2 * s) for k in range(8)) + 7 * full
+            matrix_rows = nb * 27 * (v + ib) + n * s
         if l + 1 < levels:
-            nc = shapes[l + 1][0]
-            total += 15 * nb * full                                   # post-smoother
-            total += nb * 27 * (v + ib) + n * s + nc * (4 + 2 * s)    # residual + restriction
+            total += 15 * full                                        # post-smoother
+            total += matrix_rows + nc * (4 + 2 * s)                   # residual + restriction
             total += nc * (4 + 3 * s)                                 # prolongation
     n0 = shapes[0][0]
-    ib0 = index_bytes_per_slot(None if forms is None else forms[0])
-    total += n0 * 27 * (8 + ib0) + 2 * n0 * 8                         # CG SpMV + p.Ap
+    if slot:
+        total += n0 * 4 + 2 * n0 * 8                                  # CG SpMV + p.Ap
+    else:
+        ib0 = index_bytes_per_slot(None if forms is None else forms[0])
+        total += n0 * 27 * (8 + ib0) + 2 * n0 * 8
     total += 40 * n0 + 24 * n0                                         # x and p updates; r update + r.r
     return total
