@@ -18,8 +18,9 @@
  * reference's natural row order.  Padding entries are zero after an upload.
  *
  * Calls are ordered on the context's stream (hpcgx_set_stream); calls that
- * return a scalar to the host (dot, cg) synchronise that stream.  A context
- * is used by one host thread at a time.
+ * return a scalar to the host (dot, waxpby_dot, cg) return when everything
+ * before it on that stream has run.  A context is used by one host thread at
+ * a time.
  */
 #ifndef HPCGX_H
 #define HPCGX_H
@@ -152,8 +153,12 @@ int hpcgx_level_export_packed(hpcgx_ctx *ctx, int level, uint8_t *nnz_row, int *
  * the slices keep explicit indices reads the explicit indices throughout
  * (faster there); HPCGX_COLS_COMPACT_ALWAYS reads the compact form on those
  * levels too.  HPCGX_COLS_EXPLICIT: the 32-bit index of every entry (the
- * reference's mtxIndL).  Results are the same bit for bit; only the bytes
- * read differ. */
+ * reference's mtxIndL).  On levels that read the compact form the values may be
+ * read in a shorter form too, where the stored ones equal it bit for bit (checked
+ * on the device): one value per slot and a mask per row, or, for fp64, the
+ * kappa field that the rows were generated from.  HPCGX_COLS_EXPLICIT reads
+ * every stored value.  Results are the same bit for bit; only the bytes read
+ * differ. */
 int hpcgx_set_column_format(hpcgx_ctx *ctx, int format);
 /* Slices of a level per column form: counts[0] int8 deltas, counts[1]
  * explicit indices, counts[2] no per-entry index (zeros before the compact
