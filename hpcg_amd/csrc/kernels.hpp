@@ -762,7 +762,7 @@ struct RunWave {
   int base[kSlots];
   __device__ __forceinline__ void init(const ColIdx &ci, int64_t row0, int64_t nrows, int64_t tile) {
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    take(ci, row0, nrows, (tile * (int64_t)(kBlock / kSlice) + w) * 2);
+    take(ci, row0, nrows, (tile * (int64_t)(blockDim.x >> 6) + w) * 2);
   }
   // slices g and g + 1 of the launch
   __device__ __forceinline__ void take(const ColIdx &ci, int64_t row0, int64_t nrows, int64_t g) {
@@ -798,7 +798,7 @@ inline int block_tiles(const Level &L) {
     if (L.lay.start[k + 1] - L.lay.start[k] != rows) return 0;
   return rows % (8 * 2 * kBlock) ? 0 : (int)(rows / (2 * kBlock));
 }
-inline unsigned run_tiles(int64_t rows) { return (unsigned)((rows + 2 * kBlock - 1) / (2 * kBlock)); }
+inline unsigned run_tiles(int64_t rows, int bs = kBlock) { return (unsigned)((rows + 2 * bs - 1) / (2 * bs)); }
 
 // y = A x over rows [0, nrows); ComputeSPMV_ref.cpp:61-70
 template <class VT, class XT, class ACC, int CF, int VF>
@@ -982,8 +982,8 @@ void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
   static_assert(!GEN || ZK <= 0, "general levels: full rows, or the first block from x = 0 (diagonal only)");
   static_assert(!RZ || ZK < 0, "r.z is taken from the post-smoother");
   static_assert(VF == kValsStored || (CF && !GEN), "value forms: stencil levels with compact columns");
-  // blocks of 256 threads, or of 64 for the small coarse fp64 steps (one wave
-  // per block spreads them over more CUs); the r.z form always takes 256
+  // blocks of 256 threads, or of 64 for small steps (one wave per block
+  // spreads them over more CUs: gs_block); the r.z form always takes 256
   const int64_t t = tile_id<HPCGX_FINE_ROT && FINE && sizeof(VT) == 8>() * (int64_t)blockDim.x + threadIdx.x;
   if constexpr (RZ) {
     // every thread reaches the block reduction; rows past the block add 0

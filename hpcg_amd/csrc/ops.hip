@@ -12,6 +12,15 @@ namespace hpcgx {
 
 static inline unsigned tiles(int64_t rows) { return (unsigned)((rows + kBlock - 1) / kBlock); }
 
+// Steps of blocks below this many rows take one wave per workgroup on every
+// level and in every precision: a block of 105105 rows is 411 workgroups of 256
+// threads, so that some of the 256 CUs take two and others one, and a step lasts as
+// long as the fullest.  By single waves the CUs take 6 or 7 of 1643.  SYMGS kappa
+// 97x65x129 201 -> 188 us, CG on general rows 64^3 19.6 -> 18.4 ms, CG 104^3 26.7 ->
+// 26.1.  Above, the split no longer shows and a workgroup's waves share the L1: up
+// to 2^20 rows the fp16 V-cycle of kappa 256x192x144 (884736 rows) ran 111 -> 114 ms.
+constexpr int64_t kOneWaveRows = 1 << 18;
+
 // rz (fp64 stencil levels only): the step also leaves the partials of r.x
 // over its rows there, tiles(rows) of them.
 template <class VT, class XT, class ACC, int ZK, bool FINE, bool SAFE = false>
@@ -26,12 +35,12 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
   // GFLOP/s at 192^3 (512^3 within its run-to-run spread); with paired values,
   // 94.6-95.4 ms per 192^3 set against 95.5-95.6 with the threshold at 2^16
   // (the 96^3 level's steps in 256-thread blocks) and 96.1-96.8 with none.
-  // The fine level, the other precisions and the r.z form keep 256-thread
-  // blocks.
+  // Below kOneWaveRows the fine level and the other precisions do so too; the r.z
+  // form keeps 256-thread blocks.
 #ifndef HPCGX_ONE_WAVE_ROWS
 #define HPCGX_ONE_WAVE_ROWS (1 << 20)
 #endif
-  const unsigned bs = (!FINE && sizeof(VT) == 8 && nr < (int64_t)(HPCGX_ONE_WAVE_ROWS)) ? kSlice : kBlock;
+  const unsigned bs = nr < kOneWaveRows || (!FINE && sizeof(VT) == 8 && nr < (int64_t)(HPCGX_ONE_WAVE_ROWS)) ? kSlice : kBlock;
   const unsigned g = (unsigned)((nr + bs - 1) / bs);
   hipStream_t st = c->stream;
   const ValSrc<VT, ACC> v = val_src<VT, ACC>(L);
@@ -62,7 +71,8 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
   with_forms<VT, true>(L, ci, [&](auto CF, auto VF) {
     if constexpr (VF() != kValsStored && sizeof(XT) == 8) {
       if (run_rows(L, nr)) {
-        k_gs_run<ZK, FINE, VF(), false, SAFE><<<run_tiles(nr), kBlock, 0, st>>>(ci, v, r, x, r0, nr);
+        const unsigned rbs = nr < kOneWaveRows ? kSlice : kBlock;
+        k_gs_run<ZK, FINE, VF(), false, SAFE><<<run_tiles(nr, rbs), rbs, 0, st>>>(ci, v, r, x, r0, nr);
         return;
       }
     }
