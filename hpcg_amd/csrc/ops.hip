@@ -108,6 +108,7 @@ static void gs_lines(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b) {
     return;
   }
   const int64_t ra = L.lay.start[a], rb = L.lay.start[b], nr = L.lay.start[a + 1] - ra;
+  if (nr <= 0) return;  // a grid of one plane has no rows of an odd z
   const int line = L.lay.nx / 2, rows = line <= kSlice ? kSlice / line * line : line;
   const unsigned grid = (unsigned)((nr + rows - 1) / rows), bs = (unsigned)(rows + kSlice - 1) / kSlice * kSlice;
   const ColIdx cia = col_idx(c, L, a), cib = col_idx(c, L, b);
@@ -127,6 +128,7 @@ static void gs_columns(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b)
     return;
   }
   const int64_t ra = L.lay.start[a], rb = L.lay.start[b], nr = L.lay.start[a + 1] - ra;
+  if (nr <= 0) return;
   const int plane = L.lay.nx / 2 * (L.lay.ny / 2), nz = L.lay.nz / 2, cols = kBlock / nz;
   const unsigned grid = (unsigned)((plane + cols - 1) / cols) + (nr > (int64_t)plane * nz ? 1 : 0);
   const ColIdx cia = col_idx(c, L, a), cib = col_idx(c, L, b);

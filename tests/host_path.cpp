@@ -1,0 +1,188 @@
+// Host paths of libhpcgx.so without a GPU: this program defines the HIP
+// runtime's functions itself, so the library's own calls land here.  Device
+// memory is host memory, kernels do not run.  Launches are counted by name and
+// checked as HIP checks them (an empty grid is an error); one may be made to
+// fail, and so may one allocation.
+//
+//   host_path SCENARIO    exits 0 if it holds, else prints what did not
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "hpcgx.h"
+
+namespace {
+
+constexpr int kOk = 0, kOutOfMemory = 2, kInvalidConfiguration = 9, kNotReady = 600;
+
+struct Dim3 {
+  uint32_t x, y, z;
+};
+
+// Host stub -> mangled kernel name; the library registers its kernels before
+// this program's own objects are made.
+std::map<const void *, std::string> &kernels() {
+  static std::map<const void *, std::string> k;
+  return k;
+}
+std::map<std::string, int> launched;
+int last_error = kOk;
+int handle_count = 0;
+
+int failed(int code) { return last_error = code; }
+void *handle() { return reinterpret_cast<void *>((uintptr_t)(0x1000 + 16 * ++handle_count)); }
+
+// Launches of kernels whose name holds `part`.
+int launches(const char *part) {
+  int n = 0;
+  for (const auto &k : launched)
+    if (k.first.find(part) != std::string::npos) n += k.second;
+  return n;
+}
+
+}  // namespace
+
+extern "C" {
+
+void **__hipRegisterFatBinary(const void *) { return reinterpret_cast<void **>(handle()); }
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *stub, char *, const char *name, unsigned, void *, void *, void *, void *,
+                           int *) {
+  kernels()[stub] = name;
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+
+static struct {
+  Dim3 grid, block;
+  size_t shared;
+  void *stream;
+} config;
+int __hipPushCallConfiguration(Dim3 grid, Dim3 block, size_t shared, void *stream) {
+  config = {grid, block, shared, stream};
+  return kOk;
+}
+int __hipPopCallConfiguration(Dim3 *grid, Dim3 *block, size_t *shared, void **stream) {
+  *grid = config.grid;
+  *block = config.block;
+  *shared = config.shared;
+  *stream = config.stream;
+  return kOk;
+}
+int hipLaunchKernel(const void *stub, Dim3 grid, Dim3 block, void **, size_t, void *) {
+  const std::string &name = kernels()[stub];
+  if (!grid.x || !grid.y || !grid.z || !block.x || !block.y || !block.z) {
+    std::printf("empty launch: %s\n", name.c_str());
+    return failed(kInvalidConfiguration);
+  }
+  ++launched[name];
+  return kOk;
+}
+
+int hipGetLastError() {
+  const int e = last_error;
+  last_error = kOk;
+  return e;
+}
+const char *hipGetErrorString(int) { return "error"; }
+
+int hipMalloc(void **p, size_t n) { return (*p = std::calloc(n, 1)) ? kOk : failed(kOutOfMemory); }
+int hipFree(void *p) {
+  std::free(p);
+  return kOk;
+}
+int hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+int hipHostFree(void *p) { return hipFree(p); }
+int hipMemcpy(void *d, const void *s, size_t n, int) {
+  std::memcpy(d, s, n);
+  return kOk;
+}
+int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) {
+  std::memcpy(d, s, n);
+  return kOk;
+}
+int hipMemsetAsync(void *d, int v, size_t n, void *) {
+  std::memset(d, v, n);
+  return kOk;
+}
+int hipGetSymbolAddress(void **p, const void *) { return hipMalloc(p, (size_t)4 << 20); }
+int hipFuncSetAttribute(const void *, int, int) { return kOk; }
+
+int hipSetDevice(int) { return kOk; }
+int hipStreamCreateWithFlags(void **s, unsigned) {
+  *s = handle();
+  return kOk;
+}
+int hipStreamDestroy(void *) { return kOk; }
+int hipStreamSynchronize(void *) { return kOk; }
+int hipStreamQuery(void *) { return kOk; }
+int hipEventCreate(void **e) {
+  *e = handle();
+  return kOk;
+}
+int hipEventCreateWithFlags(void **e, unsigned) { return hipEventCreate(e); }
+int hipEventDestroy(void *) { return kOk; }
+int hipEventRecord(void *, void *) { return kOk; }
+int hipEventSynchronize(void *) { return kOk; }
+int hipEventElapsedTime(float *ms, void *, void *) {
+  *ms = 0;
+  return kOk;
+}
+int hipStreamBeginCapture(void *, int) { return kOk; }
+int hipStreamEndCapture(void *, void **g) {
+  *g = handle();
+  return kOk;
+}
+int hipGraphInstantiate(void **g, void *, void *, void *, size_t) {
+  *g = handle();
+  return kOk;
+}
+int hipGraphLaunch(void *, void *) { return kOk; }
+int hipGraphDestroy(void *) { return kOk; }
+int hipGraphExecDestroy(void *) { return kOk; }
+
+}  // extern "C"
+
+#define CHECK(what)                                          \
+  do {                                                       \
+    if (!(what)) {                                           \
+      std::printf("line %d: not so: %s\n", __LINE__, #what); \
+      return 1;                                              \
+    }                                                        \
+  } while (0)
+
+// Levels with an empty colour block (grids of one plane) above the size that
+// one workgroup takes: every call launches what there is and succeeds.
+static int one_plane() {
+  for (const int flat : {0, 1, 2}) {
+    for (const int kappa : {0, 1}) {
+      int d[3] = {128, 128, 1};
+      std::swap(d[flat], d[2]);
+      hpcgx_ctx *c;
+      CHECK(hpcgx_create(0, &c) == HPCGX_OK);
+      const std::vector<double> k((size_t)128 * 128, 1.0);
+      CHECK(hpcgx_problem_generate(c, d[0], d[1], d[2], 1, kappa ? k.data() : nullptr) == HPCGX_OK);
+      double *r, *x;
+      CHECK(hpcgx_vec_alloc(c, 0, &r) == HPCGX_OK && hpcgx_vec_alloc(c, 0, &x) == HPCGX_OK);
+      CHECK(hpcgx_symgs(c, 0, r, x) == HPCGX_OK);
+      CHECK(hpcgx_mg(c, 0, r, x) == HPCGX_OK);
+      for (const int prec : {HPCGX_PREC_FP32, HPCGX_PREC_FP16}) {
+        CHECK(hpcgx_prepare_precision(c, prec) == HPCGX_OK);
+        CHECK(hpcgx_mg_mixed(c, prec, r, x) == HPCGX_OK);
+      }
+      CHECK(launches("k_gs") > 0 && launches("k_tail") == 0);
+      CHECK(hpcgx_destroy(c) == HPCGX_OK);
+    }
+  }
+  return 0;
+}
+
+int main(int argc, char **argv) {
+  const std::string s = argc > 1 ? argv[1] : "";
+  if (s == "one_plane") return one_plane();
+  std::printf("no scenario: %s\n", s.c_str());
+  return 2;
+}
