@@ -221,6 +221,17 @@ void drop_graphs(Ctx *c) {
   }
 }
 
+static void free_forms(Ctx *c, Level &L) {
+  dfree(c, L.cbase, (size_t)(L.lay.npad / kSlice) * kMeta * sizeof(int));
+  dfree(c, L.cdelta, (size_t)L.lay.npad * kSlots * sizeof(int8_t));
+  dfree(c, L.slotv, form_bytes(L));  // with boffs, vmask and cform
+  L.cbase = L.boffs = nullptr;
+  L.cdelta = nullptr;
+  L.slotv = nullptr;
+  L.vmask = nullptr;
+  L.cform = nullptr;
+}
+
 static void free_level(Ctx *c, Level &L) {
   drop_graphs(c);
   const size_t m = (size_t)L.lay.npad * kSlots;
@@ -228,9 +239,7 @@ static void free_level(Ctx *c, Level &L) {
   dfree(c, L.vals, m * sizeof(double));
   dfree(c, L.vals32, m * sizeof(float));
   dfree(c, L.vals16, m * sizeof(__half));
-  dfree(c, L.cbase, (size_t)(L.lay.npad / kSlice) * kMeta * sizeof(int));
-  dfree(c, L.cdelta, m * sizeof(int8_t));
-  dfree(c, L.slotv, form_bytes(L));  // with vmask and cform
+  free_forms(c, L);
   dfree(c, L.field, L.lay.npad * sizeof(double));
   dfree(c, L.dinv, L.lay.npad * sizeof(float));
   dfree(c, L.sigma, L.ninj * sizeof(float));
@@ -1360,21 +1369,19 @@ static int alloc_forms(Ctx *c, Level &L) {
   return HPCGX_OK;
 }
 
-// The compact index copies (the default column format) and value forms of
-// every level, with one wait for the host.
-static int build_compact_all(Ctx *c) {
-  if (c->col_format == kColsExplicit) return HPCGX_OK;
+// The compact index copies and value forms of the levels that have none yet,
+// with one wait for the host.  built: the levels that it has begun.
+static int build_forms(Ctx *c, bool (&built)[kMaxLevels]) {
   int *dev = reinterpret_cast<int *>(c->scal + S_COUNT);
-  bool built[kMaxLevels] = {};
   const int nl = (int)c->levels.size();
   FormLevels todo = {};
   unsigned nb = 0, runs_grid = 0;
   for (int l = 0; l < nl; ++l) {
     Level &L = c->levels[l];
     if (L.cbase) continue;
+    built[l] = true;
     int rc = alloc_forms(c, L);
     if (rc) return rc;
-    built[l] = true;
     const int64_t ns = L.lay.npad / kSlice;
     todo.lv[nb++] = {L.ldev, L.vmask ? L.vals : nullptr, L.cols, L.slotv, level_offs(L), L.boffs, dev + l * kFormFlags,
                      L.cbase, ns};
@@ -1409,6 +1416,21 @@ static int build_compact_all(Ctx *c) {
     L.runs = 10 * (int64_t)f[kRunSlices] >= 9 * (L.lay.npad / kSlice);
   }
   return HPCGX_OK;
+}
+
+// The forms of every level (the default column format).  A level has all of
+// them or none: after a failure those begun here are given back, so that a
+// later call builds them and no kernel reads what was never written.
+static int build_compact_all(Ctx *c) {
+  if (c->col_format == kColsExplicit) return HPCGX_OK;
+  bool built[kMaxLevels] = {};
+  const int rc = build_forms(c, built);
+  if (rc) {
+    (void)hipStreamSynchronize(c->stream);
+    for (int l = 0; l < (int)c->levels.size(); ++l)
+      if (built[l]) free_forms(c, c->levels[l]);
+  }
+  return rc;
 }
 
 static int build_precision(Ctx *c, int prec) {
@@ -1782,11 +1804,15 @@ int hpcgx_set_column_format(hpcgx_ctx *c, int format) {
                    "set_column_format: HPCGX_COLS_EXPLICIT, HPCGX_COLS_COMPACT or HPCGX_COLS_COMPACT_ALWAYS");
   HPCGX_HIP(c, hipSetDevice(c->device));
   drop_graphs(c);
+  const int before = c->col_format;
   c->col_format = format == HPCGX_COLS_COMPACT ? kColsCompact
                  : format == HPCGX_COLS_COMPACT_ALWAYS ? kColsCompactAlways : kColsExplicit;
   if (c->ready) {
     int rc = build_compact_all(c);
-    if (rc) return rc;
+    if (rc) {
+      c->col_format = before;
+      return rc;
+    }
     HPCGX_HIP(c, hipStreamSynchronize(c->stream));
   }
   return HPCGX_OK;

@@ -17,7 +17,7 @@
 
 namespace {
 
-constexpr int kOk = 0, kOutOfMemory = 2, kInvalidConfiguration = 9, kNotReady = 600;
+constexpr int kOk = 0, kOutOfMemory = 2, kInvalidConfiguration = 9, kLaunchFailure = 719;
 
 struct Dim3 {
   uint32_t x, y, z;
@@ -31,6 +31,8 @@ std::map<const void *, std::string> &kernels() {
 }
 std::map<std::string, int> launched;
 int last_error = kOk;
+int fail_malloc = 0;          // the coming hipMalloc that fails, counted from 1 (0: none)
+std::string fail_launch;      // launches of a kernel whose name holds this fail
 int handle_count = 0;
 
 int failed(int code) { return last_error = code; }
@@ -78,6 +80,7 @@ int hipLaunchKernel(const void *stub, Dim3 grid, Dim3 block, void **, size_t, vo
     std::printf("empty launch: %s\n", name.c_str());
     return failed(kInvalidConfiguration);
   }
+  if (!fail_launch.empty() && name.find(fail_launch) != std::string::npos) return failed(kLaunchFailure);
   ++launched[name];
   return kOk;
 }
@@ -89,7 +92,10 @@ int hipGetLastError() {
 }
 const char *hipGetErrorString(int) { return "error"; }
 
-int hipMalloc(void **p, size_t n) { return (*p = std::calloc(n, 1)) ? kOk : failed(kOutOfMemory); }
+int hipMalloc(void **p, size_t n) {
+  if (fail_malloc && --fail_malloc == 0) return failed(kOutOfMemory);
+  return (*p = std::calloc(n, 1)) ? kOk : failed(kOutOfMemory);
+}
 int hipFree(void *p) {
   std::free(p);
   return kOk;
@@ -180,9 +186,63 @@ static int one_plane() {
   return 0;
 }
 
+// The compact forms of three levels, with each of their allocations failing in
+// turn, then a launch: nothing is kept of a failed attempt, the format stays what
+// it was, and the next attempt builds every level.
+static int forms_after_failure() {
+  hpcgx_ctx *c;
+  CHECK(hpcgx_create(0, &c) == HPCGX_OK);
+  CHECK(hpcgx_set_column_format(c, HPCGX_COLS_EXPLICIT) == HPCGX_OK);
+  CHECK(hpcgx_problem_generate(c, 32, 32, 32, 3, nullptr) == HPCGX_OK);
+  double *x, *y;
+  CHECK(hpcgx_vec_alloc(c, 0, &x) == HPCGX_OK && hpcgx_vec_alloc(c, 0, &y) == HPCGX_OK);
+  const double bytes = hpcgx_memory_bytes(c);
+  const auto still_explicit = [&] {
+    const int before = launches("k_spmvIdddLi0E");
+    bool ok = hpcgx_memory_bytes(c) == bytes && hpcgx_spmv(c, 0, x, y) == HPCGX_OK &&
+              launches("k_spmvIdddLi0E") == before + 1;
+    for (int l = 0; l < 3; ++l) {
+      int64_t counts[4];
+      ok = ok && hpcgx_level_column_forms(c, l, counts) == HPCGX_OK && !counts[3];
+    }
+    return ok;
+  };
+  int failures = 0;
+  for (;; ++failures) {
+    const int before = launches("k_compact_cols");
+    fail_malloc = failures + 1;
+    const int rc = hpcgx_set_column_format(c, HPCGX_COLS_COMPACT_ALWAYS);
+    if (rc == HPCGX_OK) break;
+    CHECK(rc == HPCGX_ENOMEM && fail_malloc == 0);
+    CHECK(launches("k_compact_cols") == before);
+    CHECK(still_explicit());
+  }
+  fail_malloc = 0;
+  CHECK(failures >= 3);
+  CHECK(launches("k_compact_cols") == 3);
+  CHECK(hpcgx_destroy(c) == HPCGX_OK);
+
+  CHECK(hpcgx_create(0, &c) == HPCGX_OK);
+  CHECK(hpcgx_set_column_format(c, HPCGX_COLS_EXPLICIT) == HPCGX_OK);
+  CHECK(hpcgx_problem_generate(c, 32, 32, 32, 3, nullptr) == HPCGX_OK);
+  CHECK(hpcgx_vec_alloc(c, 0, &x) == HPCGX_OK && hpcgx_vec_alloc(c, 0, &y) == HPCGX_OK);
+  for (const char *kernel : {"k_slot_values", "k_compact_cols", "k_slice_runs"}) {
+    fail_launch = kernel;
+    CHECK(hpcgx_set_column_format(c, HPCGX_COLS_COMPACT_ALWAYS) == HPCGX_EHIP);
+    fail_launch.clear();
+    CHECK(still_explicit());
+  }
+  const int before = launches("k_compact_cols");
+  CHECK(hpcgx_set_column_format(c, HPCGX_COLS_COMPACT_ALWAYS) == HPCGX_OK);
+  CHECK(launches("k_compact_cols") == before + 3);
+  CHECK(hpcgx_destroy(c) == HPCGX_OK);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "one_plane") return one_plane();
+  if (s == "forms_after_failure") return forms_after_failure();
   std::printf("no scenario: %s\n", s.c_str());
   return 2;
 }
