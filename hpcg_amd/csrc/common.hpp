@@ -342,6 +342,7 @@ struct Ctx {
   std::vector<hipEvent_t> evpool;  // phase events of a deferred-stop batch (6 per iteration)
   double *hbuf = nullptr;      // pinned host scratch [64]
   double *hsum = nullptr;      // pinned total of a finishing kernel (wait_host)
+  bool total_due = false;      // a kernel that writes it may still be under way
   // solver buffers (level-0 length)
   double *cg_r = nullptr, *cg_z = nullptr, *cg_p = nullptr, *cg_Ap = nullptr;
   float *cg_r32 = nullptr, *cg_z32 = nullptr;

@@ -164,13 +164,20 @@ int wait_host(Ctx *c, const double *host, double *out) {
   }
   const uint64_t bits = *p;
   std::memcpy(out, &bits, sizeof *out);
+  c->total_due = false;
   return HPCGX_OK;
 }
 
 // One-block finishing kernel of a reduction over `grid` producer blocks.
 int finish(Ctx *c, int nv, int64_t grid, int op, double *slot, double *host) {
   const double *src = c->partials;
-  if (host) *reinterpret_cast<volatile uint64_t *>(host) = kNoTotal;
+  if (host) {
+    // a call that failed after its finishing kernel has not waited for the
+    // total: it must not be taken for this one
+    if (c->total_due) HPCGX_HIP(c, hipStreamSynchronize(c->stream));
+    *reinterpret_cast<volatile uint64_t *>(host) = kNoTotal;
+    c->total_due = true;
+  }
   if (grid > kFoldAbove) {
     const int64_t g2 = (grid + kFold - 1) / kFold;
     if (nv == 1)

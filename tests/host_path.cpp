@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <deque>
 #include <map>
 #include <string>
 #include <vector>
@@ -17,7 +18,7 @@
 
 namespace {
 
-constexpr int kOk = 0, kOutOfMemory = 2, kInvalidConfiguration = 9, kLaunchFailure = 719;
+constexpr int kOk = 0, kOutOfMemory = 2, kInvalidConfiguration = 9, kNotReady = 600, kLaunchFailure = 719;
 
 struct Dim3 {
   uint32_t x, y, z;
@@ -33,10 +34,27 @@ std::map<std::string, int> launched;
 int last_error = kOk;
 int fail_malloc = 0;          // the coming hipMalloc that fails, counted from 1 (0: none)
 std::string fail_launch;      // launches of a kernel whose name holds this fail
+int fail_after = 0;           // once so many of them have run
 int handle_count = 0;
 
 int failed(int code) { return last_error = code; }
 void *handle() { return reinterpret_cast<void *>((uintptr_t)(0x1000 + 16 * ++handle_count)); }
+
+// Finishing kernels on the stream: where each leaves its total, and the total,
+// which is the number of the launch.  They end one by one as the host asks
+// after the stream, and all of them when it waits for it.
+struct Total {
+  double *host;
+  double value;
+};
+std::deque<Total> under_way;
+double totals = 0;
+bool end_one() {
+  if (under_way.empty()) return false;
+  if (under_way.front().host) *under_way.front().host = under_way.front().value;
+  under_way.pop_front();
+  return true;
+}
 
 // Launches of kernels whose name holds `part`.
 int launches(const char *part) {
@@ -74,14 +92,17 @@ int __hipPopCallConfiguration(Dim3 *grid, Dim3 *block, size_t *shared, void **st
   *stream = config.stream;
   return kOk;
 }
-int hipLaunchKernel(const void *stub, Dim3 grid, Dim3 block, void **, size_t, void *) {
+int hipLaunchKernel(const void *stub, Dim3 grid, Dim3 block, void **args, size_t, void *) {
   const std::string &name = kernels()[stub];
   if (!grid.x || !grid.y || !grid.z || !block.x || !block.y || !block.z) {
     std::printf("empty launch: %s\n", name.c_str());
     return failed(kInvalidConfiguration);
   }
-  if (!fail_launch.empty() && name.find(fail_launch) != std::string::npos) return failed(kLaunchFailure);
+  if (!fail_launch.empty() && name.find(fail_launch) != std::string::npos && fail_after-- <= 0)
+    return failed(kLaunchFailure);
   ++launched[name];
+  if (name.find("k_finish") != std::string::npos)  // (partials, G, scal, op, slot, host)
+    under_way.push_back({*reinterpret_cast<double **>(args[5]), ++totals});
   return kOk;
 }
 
@@ -123,8 +144,11 @@ int hipStreamCreateWithFlags(void **s, unsigned) {
   return kOk;
 }
 int hipStreamDestroy(void *) { return kOk; }
-int hipStreamSynchronize(void *) { return kOk; }
-int hipStreamQuery(void *) { return kOk; }
+int hipStreamSynchronize(void *) {
+  while (end_one()) {}
+  return kOk;
+}
+int hipStreamQuery(void *) { return end_one() ? kNotReady : kOk; }
 int hipEventCreate(void **e) {
   *e = handle();
   return kOk;
@@ -239,10 +263,39 @@ static int forms_after_failure() {
   return 0;
 }
 
+// A solve that fails after its finishing kernel was launched, the total still on
+// its way: the next call that asks for one gets its own.
+static int total_after_failure() {
+  for (const int variant : {HPCGX_CG_FP64, HPCGX_CG_MIXED_FP32, HPCGX_CG_MIXED_FP16}) {
+    hpcgx_ctx *c;
+    CHECK(hpcgx_create(0, &c) == HPCGX_OK);
+    CHECK(hpcgx_problem_generate(c, 16, 16, 16, 3, nullptr) == HPCGX_OK);
+    CHECK(hpcgx_prepare_precision(c, HPCGX_PREC_FP32) == HPCGX_OK);
+    CHECK(hpcgx_prepare_precision(c, HPCGX_PREC_FP16) == HPCGX_OK);
+    double *b, *x, *w, got = 0;
+    CHECK(hpcgx_vec_alloc(c, 0, &b) == HPCGX_OK && hpcgx_vec_alloc(c, 0, &x) == HPCGX_OK);
+    CHECK(hpcgx_vec_alloc(c, 0, &w) == HPCGX_OK);
+    int iters;
+    double normr, normr0;
+    fail_launch = "k_tail";  // the V-cycle of the second iteration, launched ahead
+    fail_after = 1;
+    CHECK(hpcgx_cg(c, variant, b, x, 10, 1e-30, 1, &iters, &normr, &normr0, nullptr, nullptr) == HPCGX_EHIP);
+    fail_launch.clear();
+    CHECK(!under_way.empty());
+    CHECK(hpcgx_dot(c, 4096, b, x, &got) == HPCGX_OK);
+    CHECK(got == totals);
+    CHECK(hpcgx_waxpby_dot(c, 4096, 1.0, b, 2.0, x, w, &got) == HPCGX_OK);
+    CHECK(got == totals);
+    CHECK(hpcgx_destroy(c) == HPCGX_OK);
+  }
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "one_plane") return one_plane();
   if (s == "forms_after_failure") return forms_after_failure();
+  if (s == "total_after_failure") return total_after_failure();
   std::printf("no scenario: %s\n", s.c_str());
   return 2;
 }
