@@ -519,6 +519,13 @@ enum FinishOp : int {
   F_FCG,            // oldrtz = rtz; rtz = t0; beta = -alpha t1 / oldrtz
 };
 
+// The store must reach the host while it polls, so it has system scope.  It
+// orders nothing else: whatever the total stands for was written by kernels
+// before this one.
+__device__ __forceinline__ void give_host(double *host, double v) {
+  __hip_atomic_store(host, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 constexpr int kFinishThreads = 1024;
 constexpr int kFinishLoads = 32;  // partials per finishing thread read in one round
 
@@ -609,7 +616,7 @@ __global__ __launch_bounds__(kFinishThreads) void k_finish(const double *__restr
   switch (op) {
     case F_DOT:
       scal[S_DOT] = t[0];
-      if (host) *host = t[0];
+      if (host) give_host(host, t[0]);
       break;
     case F_RZ_FIRST: scal[S_RTZ] = t[0]; break;
     case F_RZ: {
@@ -637,7 +644,7 @@ __global__ __launch_bounds__(kFinishThreads) void k_finish(const double *__restr
         scal[S_STOP] = 0.0;
       }
       scal[S_NORMR2] = t[0];
-      if (host) *host = t[0];
+      if (host) give_host(host, t[0]);
       break;
     case F_FCG: {
       const double old = scal[S_RTZ];

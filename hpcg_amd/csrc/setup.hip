@@ -1541,7 +1541,8 @@ int hpcgx_create(int device, hpcgx_ctx **out) {
     hpcgx_destroy(c);
     return rc;
   }
-  if (hipHostMalloc((void **)&c->hbuf, 72 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+  // coherent: the host polls a total in it while the kernel that writes it runs
+  if (hipHostMalloc((void **)&c->hbuf, 72 * sizeof(double), hipHostMallocCoherent) != hipSuccess) {
     hpcgx_destroy(c);
     return HPCGX_ENOMEM;
   }

@@ -18,6 +18,7 @@
 
 namespace {
 
+constexpr unsigned kHostMallocCoherent = 0x40000000;
 constexpr int kOk = 0, kOutOfMemory = 2, kInvalidConfiguration = 9, kNotReady = 600, kLaunchFailure = 719;
 
 struct Dim3 {
@@ -49,8 +50,15 @@ struct Total {
 };
 std::deque<Total> under_way;
 double totals = 0;
+std::vector<std::pair<char *, size_t>> coherent;  // pinned memory made coherent by name
+bool all_coherent = true;                         // totals have only gone to such memory
 bool end_one() {
   if (under_way.empty()) return false;
+  if (char *p = reinterpret_cast<char *>(under_way.front().host)) {
+    bool in = false;
+    for (const auto &m : coherent) in = in || (p >= m.first && p < m.first + m.second);
+    all_coherent = all_coherent && in;
+  }
   if (under_way.front().host) *under_way.front().host = under_way.front().value;
   under_way.pop_front();
   return true;
@@ -121,7 +129,12 @@ int hipFree(void *p) {
   std::free(p);
   return kOk;
 }
-int hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+int hipHostMalloc(void **p, size_t n, unsigned flags) {
+  if (flags & kHostMallocCoherent) coherent.push_back({nullptr, n});
+  const int e = hipMalloc(p, n);
+  if (flags & kHostMallocCoherent) coherent.back().first = static_cast<char *>(*p);
+  return e;
+}
 int hipHostFree(void *p) { return hipFree(p); }
 int hipMemcpy(void *d, const void *s, size_t n, int) {
   std::memcpy(d, s, n);
@@ -291,11 +304,31 @@ static int total_after_failure() {
   return 0;
 }
 
+// The host polls totals while the kernels that write them run: they go to
+// memory that was asked to be coherent.
+static int totals_coherent() {
+  hpcgx_ctx *c;
+  CHECK(hpcgx_create(0, &c) == HPCGX_OK);
+  CHECK(hpcgx_problem_generate(c, 16, 16, 16, 3, nullptr) == HPCGX_OK);
+  double *x, *y, got;
+  CHECK(hpcgx_vec_alloc(c, 0, &x) == HPCGX_OK && hpcgx_vec_alloc(c, 0, &y) == HPCGX_OK);
+  CHECK(hpcgx_dot(c, 4096, x, y, &got) == HPCGX_OK);
+  CHECK(hpcgx_waxpby_dot(c, 4096, 1.0, x, 2.0, y, y, &got) == HPCGX_OK);
+  CHECK(hpcgx_dot_noalloc(c, 4096, x, y, &got) == HPCGX_OK);
+  int iters;
+  double normr, normr0;
+  CHECK(hpcgx_cg(c, HPCGX_CG_FP64, x, y, 3, 1e-30, 1, &iters, &normr, &normr0, nullptr, nullptr) == HPCGX_OK);
+  CHECK(totals > 3 && all_coherent);
+  CHECK(hpcgx_destroy(c) == HPCGX_OK);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "one_plane") return one_plane();
   if (s == "forms_after_failure") return forms_after_failure();
   if (s == "total_after_failure") return total_after_failure();
+  if (s == "totals_coherent") return totals_coherent();
   std::printf("no scenario: %s\n", s.c_str());
   return 2;
 }

@@ -19,7 +19,8 @@ def host_path(hip, tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["one_plane", "forms_after_failure", "total_after_failure"])
+@pytest.mark.parametrize("scenario", ["one_plane", "forms_after_failure", "total_after_failure",
+                                      "totals_coherent"])
 def test_scenario(host_path, scenario):
     out = subprocess.run([host_path, scenario], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
