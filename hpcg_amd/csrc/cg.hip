@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CF) void k_c
     const int slice = slice_of<true>(row);
     RowVals<VF, double, double, true, kAllSlots> v;
     v.load(src, row);
-    const double sum = with_cols<CF, true>(ci, slice, [&](auto cm, const int *base) {
+    double sum = with_cols<CF, true>(ci, slice, [&](auto cm, const int *base) {
       constexpr int CM = decltype(cm)::value;
       double acc_row = 0.0;
 #pragma unroll
@@ -135,6 +135,7 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(double, CF) void k_c
       }
       return acc_row;
     });
+    mend_nan<false>(sum, FromZero{}, ci.cols, src.vals, p, row, kAllSlots);
     Ap[row] = sum;
     acc = p[row] * sum;
   }
@@ -484,9 +485,9 @@ static int cg_fp64(Ctx *c, const double *b, double *x, int max_iter, double tol,
   // (F_NORMR2 with a slot), so the host launches up to kDeferBatch
   // iterations and reads their norms once instead of waiting for each.
   const bool deferred = tol == 0.0;
-  // The V-cycle's first sweep starts from z = 0 without reading most of z;
-  // the few old entries it does read (times a zero matrix entry) must be
-  // finite, which a solve that ended on a NaN may not have left.
+  // The V-cycle's first sweep starts from z = 0 without reading most of z; the
+  // few old entries it does read (times a zero matrix entry) are better finite
+  // (mend_nan), which a solve that ended on a NaN may not have left.
   if (precond && (rc = zero_vec(c, z, np))) return rc;
   if (deferred && (rc = ensure_hist(c, kDeferBatch))) return rc;
   if (times && (rc = ensure_evpool(c, 6 * (deferred ? kDeferBatch : 2)))) return rc;

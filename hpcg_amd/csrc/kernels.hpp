@@ -429,7 +429,7 @@ __device__ __forceinline__ int col_at(const ColIdx &ci, int64_t row, const int *
   } else if constexpr (CM == 2) {
     return base[s] + (int)(row & 63);
   } else {
-    return min(max((int)row + base[s], 0), ci.last);  // a zero entry's row may lie outside the level
+    return min(max((int)row + base[s], 0), ci.last);  // the row of a slot without an entry may lie outside the level
   }
 }
 
@@ -470,6 +470,43 @@ __device__ __forceinline__ auto with_cols(const ColIdx &ci, int slice, F &&f) {
     return f(cmode<0>{}, rec);
   }
 }
+
+// A slot without an entry (a neighbour outside the grid) is a zero that names some
+// other row, in the compact forms one far away in the grid: it adds an exact zero
+// unless that row's x is NaN or infinite, or not written yet.  The row's sum is NaN
+// then, and is taken again here over the entries alone, from the stored values and
+// the explicit columns, which every level has.  start() is what the sum starts from
+// (read again, so that no register holds it through the gathers).
+//
+// All other rows pay a compare and a branch that is not taken.  Solves, before ->
+// after: 104^3 fp64 25.8 -> 25.8 ms, 192^3 fp64 42.3 -> 42.2, fp32 78.4 -> 76.5, kappa
+// 256x192x144 fp16 111.2 -> 111.0, the adjoint at 128^3 (fp32, kappa) 96.5 -> 97.4.  A
+// select in every product cost the first and the last two of these 1 to 3 %.
+template <bool SUB, class VT, class XT, class ACC, class F>
+__device__ __forceinline__ void mend_nan(ACC &sum, F &&start, const int *cols, const VT *vals, const XT *x, int64_t row,
+                                         uint32_t mask) {
+  if (__builtin_expect(__ballot(sum != sum) == 0, 1)) return;
+  const bool again = sum != sum;
+  if (again) sum = start();
+#pragma unroll 1
+  for (; mask; mask &= mask - 1) {
+    const int s = __builtin_ctz(mask);
+    const ACC a = ld_val<ACC, false>(vals + val_pos<val_width<VT>>(row, s));
+    if (!again || a == (ACC)0) continue;
+    const ACC t = a * (ACC)x[cols[ell_base(row) + s * kSlice]];
+    if constexpr (SUB) sum -= t;
+    else sum += t;
+  }
+}
+// p[row] by a load of its own, whatever has been read from there before.
+template <class T>
+__device__ __forceinline__ T load_again(const T *p, int64_t row) {
+  asm("" : "+v"(row));
+  return p[row];
+}
+struct FromZero {
+  __device__ int operator()() const { return 0; }
+};
 
 // ---------------------------------------------------------------------------
 // deterministic reductions: fixed partition, fixed tree, last block finishes
@@ -732,11 +769,13 @@ struct RunVals {
 
 // sum[j] += (SUB: -=) a x over the slots in MASK, ascending.  base: the
 // first slice's slot bases (scalars); e0: the lane's first row, from the
-// run's start; xd: x of the rows themselves.  GUARD as in gs_value.
-template <int VF, uint32_t MASK, bool SUB, uint32_t GUARD>
-__device__ __forceinline__ void run_sum(const int (&base)[kSlots], unsigned e0, const ValSrc<double, double> &src,
-                                        const RunVals<VF> &v, const double *__restrict__ x, const double (&xd)[2],
-                                        double (&sum)[2]) {
+// run's start; row: the lane's first row; xd: x of the rows themselves; r: what the
+// sums start from, if not 0.
+template <int VF, uint32_t MASK, bool SUB>
+__device__ __forceinline__ void run_sum(const int *cols, const int (&base)[kSlots], unsigned e0,
+                                        const ValSrc<double, double> &src, const RunVals<VF> &v,
+                                        const double *r, const double *__restrict__ x, int64_t row,
+                                        const double (&xd)[2], double (&sum)[2]) {
 #pragma unroll
   for (int s = 0; s < kSlots; ++s) {
     if (!((MASK >> s) & 1u)) continue;
@@ -751,11 +790,14 @@ __device__ __forceinline__ void run_sum(const int (&base)[kSlots], unsigned e0, 
       if (s == kDiagSlot) a = v.d[j];
       else if constexpr (VF == kValsField) a = bit_select(v.m[j], s, -((v.ki[j] + kv[j]) * 0.5));
       else a = bit_select(v.m[j], s, src.slotv[s]);
-      const double t = a * (((GUARD >> s) & 1u) && a == 0.0 ? 0.0 : xv[j]);
+      const double t = a * xv[j];
       if constexpr (SUB) sum[j] -= t;
       else sum[j] += t;
     }
   }
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    mend_nan<SUB>(sum[j], [&] { return SUB ? load_again(r, row + j) : 0.0; }, cols, src.vals, x, row + j, MASK);
 }
 
 // A wave's place in a launch over the 64-row slices of [row0, row0 + nrows),
@@ -819,7 +861,7 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CF) void k_spmv(
   const int slice = slice_of<true>(row);
   RowVals<VF, VT, ACC, true, kAllSlots> v;
   v.load(src, row);
-  y[row] = (XT)with_cols<CF, true>(ci, slice, [&](auto cm, const int *base) {
+  ACC ax = with_cols<CF, true>(ci, slice, [&](auto cm, const int *base) {
     constexpr int CM = decltype(cm)::value;
     ACC sum = 0;
 #pragma unroll
@@ -829,6 +871,8 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CF) void k_spmv(
     }
     return sum;
   });
+  mend_nan<false>(ax, FromZero{}, ci.cols, src.vals, x, row, kAllSlots);
+  y[row] = (XT)ax;
 }
 
 // (A x) of a wave's rows (RunWave::lane_row), 0 where a lane has none.
@@ -843,7 +887,7 @@ __device__ __forceinline__ void run_ax(const ColIdx &ci, const ValSrc<double, do
     v.load(src, w.row + 2 * lane);
     double xd[2];
     ld_pair(x + w.row + 2 * lane, xd);
-    run_sum<VF, kAllSlots, false, 0>(w.base, 2 * lane, src, v, x, xd, out);
+    run_sum<VF, kAllSlots, false>(ci.cols, w.base, 2 * lane, src, v, nullptr, x, w.row + 2 * lane, xd, out);
     return;
   }
 #pragma unroll 1
@@ -851,7 +895,7 @@ __device__ __forceinline__ void run_ax(const ColIdx &ci, const ValSrc<double, do
     const int64_t row = w.row + j * kSlice + lane;
     RowVals<VF, double, double, false, kAllSlots> v;
     v.load(src, row);
-    put(out, j, with_cols<kColsSlice, true>(ci, slice_of<true>(row), [&](auto cm, const int *base) {
+    double ax = with_cols<kColsSlice, true>(ci, slice_of<true>(row), [&](auto cm, const int *base) {
       constexpr int CM = decltype(cm)::value;
       double sum = 0;
 #pragma unroll
@@ -860,7 +904,9 @@ __device__ __forceinline__ void run_ax(const ColIdx &ci, const ValSrc<double, do
         sum += v.at(s, c) * x[c];
       }
       return sum;
-    }));
+    });
+    mend_nan<false>(ax, FromZero{}, ci.cols, src.vals, x, row, kAllSlots);
+    put(out, j, ax);
   }
 }
 
@@ -924,20 +970,11 @@ static_assert(masks_keep_units(2) && masks_keep_units(4), "zero-start masks spli
 // ZK == 0 reads no neighbour at all (x_i = r_i / a_ii), which holds for the
 // first block of any order, general levels included.
 // GEN: general level, the diagonal's slot is dslot[row] (stencil: slot 13).
-// GUARD: slots in which a zero entry (a neighbour outside the grid) contributes
-// 0 * 0, as the reference's zeroed x gives, whatever the row it points at
-// holds.  SAFE guards them all, in a step from x = 0 into a vector that may hold
-// anything: such an entry may point at a row not written yet in this sweep.
-// The solvers clear their level-0 buffer when a solve begins, so their level-0
-// sweeps skip the select.
-template <int ZK, bool SAFE>
-constexpr uint32_t gs_guard = ZK >= 0 && SAFE ? kAllSlots : 0;
-
-// gs_value is a row's new value, from r_i; gs_row the update of one row, which
+// gs_value is a row's new value; gs_row the update of one row, which
 // returns r_i * x_i (new) for the fused r.z.
-template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, uint32_t GUARD>
-__device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &src, ACC ri, const XT *x, int64_t row,
-                                       const uint8_t *__restrict__ dslot) {
+template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN>
+__device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &src, const XT *r, const XT *x,
+                                       int64_t row, const uint8_t *__restrict__ dslot) {
   constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
   const size_t b = ell_base(row);
   const int slice = slice_of<true>(row);
@@ -946,30 +983,35 @@ __device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &
   ACC d;
   if constexpr (!GEN) d = vr.diag(src, row);
   else d = ld_val<ACC, FINE>(src.vals + val_pos<val_width<VT>>(row, (int)dslot[row]));
+  const ACC xi = ZK < 0 ? (ACC)x[row] : (ACC)0;
   auto row_sum = [&](auto cm, const int *base) {
     constexpr int CM = decltype(cm)::value;
-    ACC sum = ri;
+    ACC sum = (ACC)r[row];
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
       if (!((mask >> s) & 1u)) continue;
+      if (!GEN && s == kDiagSlot) {
+        sum -= vr.at(s, 0) * xi;
+        continue;
+      }
       const int c = col_at<CM, FINE>(ci, row, base, b, s);
-      const ACC v = vr.at(s, c);
-      const ACC xc = (ACC)x[c];
-      if ((GUARD >> s) & 1u) sum -= v * (v != (ACC)0 ? xc : (ACC)0);
-      else sum -= v * xc;
+      sum -= vr.at(s, c) * (ACC)x[c];
     }
     return sum;
   };
   ACC sum = with_cols<CF, true>(ci, slice, row_sum);
-  if (ZK < 0) sum += (ACC)x[row] * d;
+  // not on general levels: their slots without an entry name the row itself or its
+  // slice's neighbourhood
+  if constexpr (!GEN) mend_nan<true>(sum, [&] { return load_again(r, row); }, ci.cols, src.vals, x, row, mask);
+  if (ZK < 0) sum += xi * d;
   return (XT)(sum / d);
 }
 
-template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN, uint32_t GUARD>
+template <class VT, class XT, class ACC, int ZK, bool FINE, int CF, int VF, bool GEN>
 __device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC> &src,
                                          const XT *__restrict__ r, XT *__restrict__ x, int64_t row,
                                          const uint8_t *__restrict__ dslot) {
-  const XT xn = gs_value<VT, XT, ACC, ZK, FINE, CF, VF, GEN, GUARD>(ci, src, (ACC)r[row], x, row, dslot);
+  const XT xn = gs_value<VT, XT, ACC, ZK, FINE, CF, VF, GEN>(ci, src, r, x, row, dslot);
   x[row] = xn;
   return (double)r[row] * (double)xn;
 }
@@ -979,7 +1021,7 @@ __device__ __forceinline__ double gs_row(const ColIdx &ci, const ValSrc<VT, ACC>
 // also leaves its partial sum of r_i x_i in rz[blockIdx.x], so the solver's
 // r.z needs no pass of its own.
 template <class VT, class XT, class ACC, int ZK, bool FINE, int CF = kColsStored, int VF = kValsStored, bool GEN = false,
-          bool RZ = false, bool SAFE = false>
+          bool RZ = false>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(1, SparseOccupancy<VT, CF, ZK < 0 ? kSlots : __builtin_popcount(swept_before_mask(ZK))>::max_waves)))
 void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
@@ -995,13 +1037,13 @@ void k_gs(const ColIdx ci, const ValSrc<VT, ACC> src,
   if constexpr (RZ) {
     // every thread reaches the block reduction; rows past the block add 0
     double acc = 0.0;
-    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, gs_guard<ZK, SAFE>>(ci, src, r, x, row0 + t, dslot);
+    if (t < nrows) acc = gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN>(ci, src, r, x, row0 + t, dslot);
     const double v[1] = {acc};
     block_partials<1>(v, rz);
     return;
   }
   if (t >= nrows) return;
-  gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN, gs_guard<ZK, SAFE>>(ci, src, r, x, row0 + t, dslot);
+  gs_row<VT, XT, ACC, ZK, FINE, CF, VF, GEN>(ci, src, r, x, row0 + t, dslot);
 }
 
 // The partial sums of a value per row, as the one-row-per-lane launch leaves
@@ -1037,7 +1079,7 @@ __device__ __forceinline__ void run_partials(const RunWave &w, double (&v)[2], i
 }
 
 // One Gauss-Seidel step on a wave's two slices; acc[j]: r_i x_i of lane_row(j).
-template <int ZK, bool FINE, int VF, uint32_t GUARD>
+template <int ZK, bool FINE, int VF>
 __device__ __forceinline__ void gs_run_rows(const ColIdx &ci, const ValSrc<double, double> &src, const RunWave &w,
                                             const double *__restrict__ r, double *x, double (&acc)[2]) {
   constexpr uint32_t mask = ZK >= 0 ? swept_before_mask(ZK) : kAllSlots;
@@ -1051,7 +1093,7 @@ __device__ __forceinline__ void gs_run_rows(const ColIdx &ci, const ValSrc<doubl
     ld_pair(r + row, rv);
     if constexpr (ZK < 0) ld_pair(x + row, xd);
     double sum[2] = {rv[0], rv[1]};
-    run_sum<VF, mask, true, GUARD>(w.base, 2 * (threadIdx.x & 63), src, v, x, xd, sum);
+    run_sum<VF, mask, true>(ci.cols, w.base, 2 * (threadIdx.x & 63), src, v, r, x, row, xd, sum);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       if constexpr (ZK < 0) sum[j] += xd[j] * v.d[j];
@@ -1063,11 +1105,11 @@ __device__ __forceinline__ void gs_run_rows(const ColIdx &ci, const ValSrc<doubl
   }
 #pragma unroll 1
   for (int j = 0; j < w.slices; ++j)
-    put(acc, j, gs_row<double, double, double, ZK, FINE, kColsSlice, VF, false, GUARD>(ci, src, r, x, w.lane_row(j), nullptr));
+    put(acc, j, gs_row<double, double, double, ZK, FINE, kColsSlice, VF, false>(ci, src, r, x, w.lane_row(j), nullptr));
 }
 
 // One Gauss-Seidel step by row runs (k_gs on kValsSlot and kValsField levels).
-template <int ZK, bool FINE, int VF, bool RZ = false, bool SAFE = false>
+template <int ZK, bool FINE, int VF, bool RZ = false>
 __global__ __launch_bounds__(kBlock) void k_gs_run(const ColIdx ci, const ValSrc<double, double> src,
                                                    const double *__restrict__ r, double *__restrict__ x,
                                                    int64_t row0, int64_t nrows, double *rz = nullptr) {
@@ -1076,7 +1118,7 @@ __global__ __launch_bounds__(kBlock) void k_gs_run(const ColIdx ci, const ValSrc
   RunWave w;
   w.init(ci, row0, nrows, tile);
   double acc[2];
-  gs_run_rows<ZK, FINE, VF, gs_guard<ZK, SAFE>>(ci, src, w, r, x, acc);
+  gs_run_rows<ZK, FINE, VF>(ci, src, w, r, x, acc);
   if constexpr (RZ) run_partials<ROT>(w, acc, tile, (nrows + kBlock - 1) / kBlock, rz);
 }
 
@@ -1092,26 +1134,22 @@ __global__ __launch_bounds__(kBlock) void k_gs_run(const ColIdx ci, const ValSrc
 // 199 us, 104^3 371 -> 326 -> 324, 128^3 fp32 376 -> 325 -> 302, kappa 104^3 fp16 342 ->
 // 299 -> 293.
 //
-// Past the end of a line, the slots along it point at another line of the
-// other block, which another workgroup may be updating: they are guarded.
-// SAFE: so are the others, in the third step too (a zero entry's row may run on
-// from its block's end into the blocks that this launch writes first).
+// Past the end of a line, the slots along it name another line of the other
+// block, which another workgroup may be updating: times the slot's zero that adds
+// nothing, whichever value is read (mend_nan, should it be NaN).
 //
 // A row per lane, columns by the blocks' distances; a workgroup takes `rows`
 // rows (whole lines) of each block.  STEPS 3: the first block again.  ZA, ZB: the
 // steps' places in a sweep from x = 0 (ZK of k_gs), or -1.
-constexpr uint32_t kLineSlots = 1u << (kDiagSlot - 1) | 1u << (kDiagSlot + 1);
-
-template <class VT, class XT, class ACC, int ZA, int ZB, int STEPS, bool FINE, int VF, bool SAFE>
+template <class VT, class XT, class ACC, int ZA, int ZB, int STEPS, bool FINE, int VF>
 __global__ __launch_bounds__(kBlock) void k_gs_lines(const ColIdx cia, const ColIdx cib, const ValSrc<VT, ACC> src,
                                                      const XT *__restrict__ r, XT *x, int64_t rowa, int64_t rowb,
                                                      int64_t nrows, int rows) {
-  constexpr uint32_t guard = SAFE ? kAllSlots : kLineSlots;
   const int64_t i = tile_id() * rows + threadIdx.x;
   const bool in = (int)threadIdx.x < rows && i < nrows;
   auto step = [&](auto zk, const ColIdx &ci, int64_t row) {
     if (in)
-      x[row] = gs_value<VT, XT, ACC, decltype(zk)::value, FINE, kColsBlock, VF, false, guard>(ci, src, (ACC)r[row], x, row, nullptr);
+      x[row] = gs_value<VT, XT, ACC, decltype(zk)::value, FINE, kColsBlock, VF, false>(ci, src, r, x, row, nullptr);
   };
   step(std::integral_constant<int, ZA>{}, cia, rowa + i);
   __syncthreads();
@@ -1126,12 +1164,10 @@ __global__ __launch_bounds__(kBlock) void k_gs_lines(const ColIdx cia, const Col
 // back): their rows couple only along z, and a workgroup takes `cols` columns of
 // both blocks through all nz planes of `plane` rows; one more takes the rows that
 // pad the blocks.  Workgroups of 512 threads were slower (64^3 223 us).
-constexpr uint32_t kColumnSlots = 1u << (kDiagSlot - 9) | 1u << (kDiagSlot + 9);
-template <class VT, class XT, class ACC, int ZA, int ZB, bool FINE, int VF, bool SAFE>
+template <class VT, class XT, class ACC, int ZA, int ZB, bool FINE, int VF>
 __global__ __launch_bounds__(kBlock) void k_gs_columns(const ColIdx cia, const ColIdx cib, const ValSrc<VT, ACC> src,
                                                        const XT *__restrict__ r, XT *x, int64_t rowa, int64_t rowb,
                                                        int64_t nrows, int plane, int nz, int cols) {
-  constexpr uint32_t guard = SAFE ? kAllSlots : kColumnSlots;
   const int64_t tile = tile_id();
   const int z = (int)threadIdx.x / cols;
   const int64_t q = tile * cols + ((int)threadIdx.x - z * cols);
@@ -1143,7 +1179,7 @@ __global__ __launch_bounds__(kBlock) void k_gs_columns(const ColIdx cia, const C
   }
   auto step = [&](auto zk, const ColIdx &ci, int64_t row) {
     if (in)
-      x[row] = gs_value<VT, XT, ACC, decltype(zk)::value, FINE, kColsBlock, VF, false, guard>(ci, src, (ACC)r[row], x, row, nullptr);
+      x[row] = gs_value<VT, XT, ACC, decltype(zk)::value, FINE, kColsBlock, VF, false>(ci, src, r, x, row, nullptr);
   };
   step(std::integral_constant<int, ZA>{}, cia, rowa + i);
   __syncthreads();
@@ -1185,6 +1221,7 @@ __global__ __launch_bounds__(kBlock) HPCGX_SPARSE_OCCUPANCY(VT, CF) void k_restr
     const int slice = slice_of<true>(row);
     ax = with_cols<CF, true>(ci, slice, row_ax);
   }
+  mend_nan<false>(ax, FromZero{}, ci.cols, src.vals, x, row, kAllSlots);
   ACC res = (ACC)r[row] - ax;
   if (SCALE) res = res * (ACC)sigma[t];
   rc[inj[t]] = (XT)res;
@@ -1254,7 +1291,7 @@ struct TailLevel {
   int ninj, row0;
   const int *boffs;  // the blocks' distances (has_block_offs) where sweep_slot takes the level, else null
   int npad, ncol;
-  int xoff, roff;    // x and r in LDS, in elements
+  int xoff, roff;    // x (and a zero) and r in LDS, in elements
   int start[kTailColours + 1];
 };
 // r, x: the first level's.  load_x: start from x instead of 0.
@@ -1276,13 +1313,14 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
   // diagonal, and a slice or none for every wave.  A step then is LDS reads, a
   // chain of 27 sums, a division and a barrier: what comes from memory (the
   // row's mask) is fetched a step ahead, the slots' values and the level's
-  // fields are read once.  V-cycle on the device, sweep below -> this one: 8^3
+  // fields are read once.  A slot without an entry reads the zero that lies behind
+  // the level's x.  V-cycle on the device, sweep below -> this one: 8^3
   // (4 levels) 52 -> 41 us, 16^3 63 -> 54 (fp32 64 -> 56); 20^3, whose second
   // level has an odd size, 84 -> 81.
   auto sweep_slot = [&](const TailLevel<VT, XT, ACC> &L) {
     XT *x = lds + L.xoff;
     const XT *r = lds + L.roff;
-    const int last = L.npad - 1, ncol = L.ncol, steps = 2 * ncol - 1;
+    const int npad = L.npad, ncol = L.ncol, steps = 2 * ncol - 1;
     const int *boffs = L.boffs, *start = L.start;
     const uint32_t *mask = L.src.mask;
     ACC sv[kSlots];
@@ -1305,7 +1343,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
           if (s == kDiagSlot) sum -= d * xi;
-          else sum -= bit_select(m, s, sv[s]) * (ACC)x[min(max(row + off[s], 0), last)];
+          else sum -= sv[s] * (ACC)x[npad + ((row + off[s] - npad) & -(int)((m >> s) & 1u))];
         }
         sum += xi * d;
         x[row] = (XT)(sum / d);
@@ -1327,7 +1365,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
       const int end = L.start[k + 1] >> 6;
       for (int slice = (L.start[k] >> 6) + wave; slice < end; slice += nw) {
         const int row = slice * kSlice + lane;
-        x[row] = gs_value<VT, XT, ACC, -1, false, CF, VF, GEN, 0>(L.ci, L.src, (ACC)lds[L.roff + row], x, row, L.dslot);
+        x[row] = gs_value<VT, XT, ACC, -1, false, CF, VF, GEN>(L.ci, L.src, lds + L.roff, x, row, L.dslot);
       }
       __syncthreads();
     }
@@ -1337,6 +1375,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
     lds[F.xoff + i] = a.load_x ? a.x[i] : (XT)0;
     lds[F.roff + i] = a.r[i];
   }
+  for (int l = threadIdx.x; l < a.n; l += blockDim.x) lds[a.lv[l].xoff + a.lv[l].npad] = (XT)0;
   for (int l = 1; l < a.n; ++l)
     for (int i = threadIdx.x; i < a.lv[l].npad; i += blockDim.x) lds[a.lv[l].xoff + i] = lds[a.lv[l].roff + i] = (XT)0;
   __syncthreads();
@@ -1366,6 +1405,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
       ACC ax;
       if constexpr (GEN) ax = with_cols<CF, false>(L.ci, slice_of<false>(row), row_ax);  // rows from a list
       else ax = with_cols<CF, true>(L.ci, slice_of<true>(row), row_ax);
+      if constexpr (!GEN) mend_nan<false>(ax, FromZero{}, L.ci.cols, L.src.vals, x, row, kAllSlots);
       ACC res = (ACC)lds[L.roff + row] - ax;
       if (SCALE) res = res * (ACC)L.sigma[t];
       lds[a.lv[l + 1].roff + L.inj[t]] = (XT)res;

@@ -23,7 +23,7 @@ constexpr int64_t kOneWaveRows = 1 << 18;
 
 // rz (fp64 stencil levels only): the step also leaves the partials of r.x
 // over its rows there, tiles(rows) of them.
-template <class VT, class XT, class ACC, int ZK, bool FINE, bool SAFE = false>
+template <class VT, class XT, class ACC, int ZK, bool FINE>
 static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *rz = nullptr) {
   const int64_t r0 = L.lay.start[k], nr = L.lay.start[k + 1] - r0;
   if (nr <= 0) return;
@@ -72,11 +72,11 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
     if constexpr (VF() != kValsStored && sizeof(XT) == 8) {
       if (run_rows(L, nr)) {
         const unsigned rbs = nr < kOneWaveRows ? kSlice : kBlock;
-        k_gs_run<ZK, FINE, VF(), false, SAFE><<<run_tiles(nr, rbs), rbs, 0, st>>>(ci, v, r, x, r0, nr);
+        k_gs_run<ZK, FINE, VF()><<<run_tiles(nr, rbs), rbs, 0, st>>>(ci, v, r, x, r0, nr);
         return;
       }
     }
-    k_gs<VT, XT, ACC, ZK, FINE, CF(), VF(), false, false, SAFE><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
+    k_gs<VT, XT, ACC, ZK, FINE, CF(), VF()><<<g, bs, 0, st>>>(ci, v, r, x, r0, nr, nullptr);
   });
 }
 
@@ -99,11 +99,11 @@ static bool columns_pay(const Ctx *c, const Level &L) {
 }
 
 // Steps of blocks a, b (STEPS 3: and a again), whose classes differ in x alone.
-template <class VT, class XT, class ACC, int ZA, int ZB, int STEPS, bool FINE, bool SAFE = false>
+template <class VT, class XT, class ACC, int ZA, int ZB, int STEPS, bool FINE>
 static void gs_lines(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b) {
   if (!lines_pay(c, L)) {
-    gs_block<VT, XT, ACC, ZA, FINE, SAFE>(c, L, r, x, a);
-    gs_block<VT, XT, ACC, ZB, FINE, SAFE>(c, L, r, x, b);
+    gs_block<VT, XT, ACC, ZA, FINE>(c, L, r, x, a);
+    gs_block<VT, XT, ACC, ZB, FINE>(c, L, r, x, b);
     if constexpr (STEPS == 3) gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, a);
     return;
   }
@@ -114,17 +114,17 @@ static void gs_lines(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b) {
   const ColIdx cia = col_idx(c, L, a), cib = col_idx(c, L, b);
   with_forms<VT>(L, cia, [&](auto CF, auto VF) {
     if constexpr (CF() != kColsStored)
-      k_gs_lines<VT, XT, ACC, ZA, ZB, STEPS, FINE, VF(), SAFE>
+      k_gs_lines<VT, XT, ACC, ZA, ZB, STEPS, FINE, VF()>
           <<<grid, bs, 0, c->stream>>>(cia, cib, val_src<VT, ACC>(L), r, x, ra, rb, nr, rows);
   });
 }
 
 // Steps of blocks a, b, whose classes differ in z alone.
-template <class VT, class XT, class ACC, int ZA, int ZB, bool FINE, bool SAFE = false>
+template <class VT, class XT, class ACC, int ZA, int ZB, bool FINE>
 static void gs_columns(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b) {
   if (!columns_pay(c, L)) {
-    gs_block<VT, XT, ACC, ZA, FINE, SAFE>(c, L, r, x, a);
-    gs_block<VT, XT, ACC, ZB, FINE, SAFE>(c, L, r, x, b);
+    gs_block<VT, XT, ACC, ZA, FINE>(c, L, r, x, a);
+    gs_block<VT, XT, ACC, ZB, FINE>(c, L, r, x, b);
     return;
   }
   const int64_t ra = L.lay.start[a], rb = L.lay.start[b], nr = L.lay.start[a + 1] - ra;
@@ -134,19 +134,19 @@ static void gs_columns(Ctx *c, const Level &L, const XT *r, XT *x, int a, int b)
   const ColIdx cia = col_idx(c, L, a), cib = col_idx(c, L, b);
   with_forms<VT>(L, cia, [&](auto CF, auto VF) {
     if constexpr (CF() != kColsStored)
-      k_gs_columns<VT, XT, ACC, ZA, ZB, FINE, VF(), SAFE>
+      k_gs_columns<VT, XT, ACC, ZA, ZB, FINE, VF()>
           <<<grid, kBlock, 0, c->stream>>>(cia, cib, val_src<VT, ACC>(L), r, x, ra, rb, nr, plane, nz, cols);
   });
 }
 
 // The zero-start forward sweep of the default order: block k reads only the
 // blocks swept before it.  The backward step of block 6 comes with it.
-template <class VT, class XT, class ACC, bool FINE, bool SAFE>
+template <class VT, class XT, class ACC, bool FINE>
 static void zero_start_forward(Ctx *c, const Level &L, const XT *r, XT *x) {
-  gs_columns<VT, XT, ACC, 0, 1, FINE, SAFE>(c, L, r, x, 0, 1);
-  gs_lines<VT, XT, ACC, 2, 3, 2, FINE, SAFE>(c, L, r, x, 2, 3);
-  gs_columns<VT, XT, ACC, 4, 5, FINE, SAFE>(c, L, r, x, 4, 5);
-  gs_lines<VT, XT, ACC, 6, 7, 3, FINE, SAFE>(c, L, r, x, 6, 7);
+  gs_columns<VT, XT, ACC, 0, 1, FINE>(c, L, r, x, 0, 1);
+  gs_lines<VT, XT, ACC, 2, 3, 2, FINE>(c, L, r, x, 2, 3);
+  gs_columns<VT, XT, ACC, 4, 5, FINE>(c, L, r, x, 4, 5);
+  gs_lines<VT, XT, ACC, 6, 7, 3, FINE>(c, L, r, x, 6, 7);
 }
 
 // The remaining backward steps of the default order, from block 5.
@@ -210,19 +210,17 @@ static int64_t rz_pass(Ctx *c, const Level &L, const double *r, const double *x,
 // only its diagonal (x_i = r_i / a_ii, what the full step gives bit for bit).
 // rz: the steps that leave their rows final (forward step of the last block,
 // then the backward steps) write r.x partials at rz, *nrz of them in all.
-// untrusted_x: x may hold anything on a zero start (a caller's vector, or a
-// coarse level's vector after a V-cycle on a non-finite input); the solvers
-// clear their own level-0 buffer when a solve begins and skip the guard.
+// x may hold anything on a zero start (a caller's vector, or a coarse level's after
+// a V-cycle on a non-finite input): see mend_nan.
 template <class VT, class XT, class ACC, bool FINE>
 static void sweep(Ctx *c, const Level &L, const XT *r, XT *x, bool zero_start, double *rz = nullptr,
-                  int64_t *nrz = nullptr, bool untrusted_x = false) {
+                  int64_t *nrz = nullptr) {
   if (zero_start && !default_order(L)) {
     k_zero<XT><<<tiles(L.lay.npad), kBlock, 0, c->stream>>>(x, L.lay.npad);
     gs_block<VT, XT, ACC, 0, FINE>(c, L, r, x, 0);
     for (int k = 1; k < L.lay.ncol; ++k) gs_block<VT, XT, ACC, -1, FINE>(c, L, r, x, k);
   } else if (zero_start) {
-    if (untrusted_x) zero_start_forward<VT, XT, ACC, FINE, true>(c, L, r, x);
-    else zero_start_forward<VT, XT, ACC, FINE, false>(c, L, r, x);
+    zero_start_forward<VT, XT, ACC, FINE>(c, L, r, x);
     backward_from_5<VT, XT, ACC, FINE>(c, L, r, x);
     return;
   } else if (default_order(L) && (!rz || lines_pay(c, L))) {
@@ -254,10 +252,10 @@ static void sweep(Ctx *c, const Level &L, const XT *r, XT *x, bool zero_start, d
 
 template <class VT, class XT, class ACC>
 static int symgs_launch(Ctx *c, int l, const XT *r, XT *x, bool zero_start, double *rz = nullptr,
-                        int64_t *nrz = nullptr, bool untrusted_x = false) {
+                        int64_t *nrz = nullptr) {
   const Level &L = c->levels[l];
-  if (l == 0) sweep<VT, XT, ACC, true>(c, L, r, x, zero_start, rz, nrz, untrusted_x);
-  else sweep<VT, XT, ACC, false>(c, L, r, x, zero_start, rz, nrz, untrusted_x);
+  if (l == 0) sweep<VT, XT, ACC, true>(c, L, r, x, zero_start, rz, nrz);
+  else sweep<VT, XT, ACC, false>(c, L, r, x, zero_start, rz, nrz);
   HPCGX_CHECK_LAUNCH(c);
   return HPCGX_OK;
 }
@@ -300,8 +298,8 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
     if (slices > kTailThreads / kSlice) t.boffs = nullptr;
     waves = std::max(waves, slices);
     t.xoff = (int)off;
-    t.roff = (int)(off + L.lay.npad);
-    off += 2 * L.lay.npad;
+    t.roff = (int)(off + L.lay.npad + 1);
+    off += 2 * L.lay.npad + 1;
     if (off * (int64_t)sizeof(XT) > kTailLds) return false;
   }
   const unsigned lds = (unsigned)(off * sizeof(XT));
@@ -333,12 +331,9 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
 // V-cycle of ComputeMG_ref.cpp:39-63: x = 0; pre-smooth; residual + restrict;
 // recurse; prolong; post-smooth.  The coarsest level gets one smoothing step.
 // rz / nrz: r.x partials of the result from the post-smoother (see sweep);
-// fp64 stencil levels with a coarse level only.  untrusted_x: x at level l
-// may hold anything (the caller's vector); the coarse levels always take
-// this form.
+// fp64 stencil levels with a coarse level only.
 template <class VT, class XT, class ACC, bool SCALE>
-static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64_t *nrz = nullptr,
-                  bool untrusted_x = false) {
+static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64_t *nrz = nullptr) {
   const Level &L = c->levels[l];
   if (tail<VT, XT, ACC, SCALE>(c, l, r, x)) {
     if constexpr (sizeof(VT) == 8) {
@@ -347,7 +342,7 @@ static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64
     HPCGX_CHECK_LAUNCH(c);
     return HPCGX_OK;
   }
-  int rc = symgs_launch<VT, XT, ACC>(c, l, r, x, true, nullptr, nullptr, untrusted_x);
+  int rc = symgs_launch<VT, XT, ACC>(c, l, r, x, true);
   if (rc || l + 1 >= (int)c->levels.size()) return rc;
   Level &C = c->levels[l + 1];
   XT *rc_v, *xc_v;
@@ -371,9 +366,7 @@ static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64
         ci, val_src<VT, ACC>(L), r, x, rc_v, L.inj, L.sigma, r0, nc, L.frow);
   });
   HPCGX_CHECK_LAUNCH(c);
-  // the coarse level's x may hold anything: a V-cycle on a non-finite input
-  // leaves non-finite values in the context's coarse vectors
-  if ((rc = vcycle<VT, XT, ACC, SCALE>(c, l + 1, rc_v, xc_v, nullptr, nullptr, true))) return rc;
+  if ((rc = vcycle<VT, XT, ACC, SCALE>(c, l + 1, rc_v, xc_v))) return rc;
   k_prolong<XT, ACC, SCALE><<<tiles(nc), kBlock, 0, c->stream>>>(x, xc_v, L.inj, L.sigma, r0, nc, L.frow);
   HPCGX_CHECK_LAUNCH(c);
   return symgs_launch<VT, XT, ACC>(c, l, r, x, false, rz, nrz);
@@ -434,14 +427,14 @@ __global__ __launch_bounds__(kBlock) void k_waxpby_dot(int64_t n, double alpha,
 }
 
 
-int mg_fp64(Ctx *c, int level, const double *r, double *x, double *rz, int64_t *nrz, bool untrusted_x) {
+int mg_fp64(Ctx *c, int level, const double *r, double *x, double *rz, int64_t *nrz) {
   if (rz && (level + 1 >= (int)c->levels.size() || c->levels[level].lay.general))
     return set_err(c, HPCGX_EINVAL, "fused r.z needs a stencil level with a coarse level");
-  return vcycle<double, double, double, false>(c, level, r, x, rz, nrz, untrusted_x);
+  return vcycle<double, double, double, false>(c, level, r, x, rz, nrz);
 }
 
-int mg_fp32(Ctx *c, int level, const float *r, float *x, bool untrusted_x) {
-  return vcycle<float, float, float, false>(c, level, r, x, nullptr, nullptr, untrusted_x);
+int mg_fp32(Ctx *c, int level, const float *r, float *x) {
+  return vcycle<float, float, float, false>(c, level, r, x);
 }
 
 int zero_vec(Ctx *c, double *x, int64_t n) {
@@ -470,12 +463,12 @@ int mg_fp16_scaled(Ctx *c, const float *rhat, float *xhat) {
 
 // Scaled fp16 V-cycle on level 0: rhat = dinv r, V-cycle with D^-1/2 A D^-1/2,
 // x = dinv xhat.
-int mg_fp16(Ctx *c, const float *r, float *x, bool untrusted_x) {
+int mg_fp16(Ctx *c, const float *r, float *x) {
   Level &L = c->levels[0];
   const int64_t np = L.lay.npad;
   k_scale<<<tiles(np), kBlock, 0, c->stream>>>(r, L.dinv, L.r16, np);
   HPCGX_CHECK_LAUNCH(c);
-  int rc = vcycle<__half, float, float, true>(c, 0, L.r16, x, nullptr, nullptr, untrusted_x);
+  int rc = vcycle<__half, float, float, true>(c, 0, L.r16, x);
   if (rc) return rc;
   k_scale<<<tiles(np), kBlock, 0, c->stream>>>(x, L.dinv, x, np);
   HPCGX_CHECK_LAUNCH(c);
@@ -646,7 +639,7 @@ int hpcgx_mg(hpcgx_ctx *c, int level, const double *r, double *x) {
   if (rc) return rc;
   if ((rc = check_vecs(c, npad_of(c, level), "mg", {r, x}))) return rc;
   if (r == x) return set_err(c, HPCGX_EINVAL, "mg: r and x must be distinct device vectors");
-  return mg_fp64(c, level, r, x, nullptr, nullptr, true);
+  return mg_fp64(c, level, r, x);
 }
 
 int hpcgx_mg_mixed(hpcgx_ctx *c, int precision, const double *r, double *x) {
@@ -660,8 +653,8 @@ int hpcgx_mg_mixed(hpcgx_ctx *c, int precision, const double *r, double *x) {
   const int64_t np = c->levels[0].lay.npad;
   k_to_single<<<tiles(np), kBlock, 0, c->stream>>>(r, c->cg_r32, np);
   HPCGX_CHECK_LAUNCH(c);
-  rc = precision == HPCGX_PREC_FP32 ? mg_fp32(c, 0, c->cg_r32, c->cg_z32, true)
-                                    : mg_fp16(c, c->cg_r32, c->cg_z32, true);
+  rc = precision == HPCGX_PREC_FP32 ? mg_fp32(c, 0, c->cg_r32, c->cg_z32)
+                                    : mg_fp16(c, c->cg_r32, c->cg_z32);
   if (rc) return rc;
   k_to_double<<<tiles(np), kBlock, 0, c->stream>>>(c->cg_z32, x, np);
   HPCGX_CHECK_LAUNCH(c);
