@@ -840,13 +840,15 @@ __device__ __forceinline__ void put(double (&a)[2], int j, double v) {
   a[1] = j == 1 ? v : a[1];
 }
 
-// Blocks of a row-run launch over `rows` rows.
+// Workgroups of a row-run launch per colour block, where level_tile can take the
+// blocks together: equal ones, a multiple of 8 workgroups each (else 0).
 inline int block_tiles(const Level &L) {
   const int64_t rows = L.lay.start[1];
   for (int k = 0; k < kColours; ++k)
     if (L.lay.start[k + 1] - L.lay.start[k] != rows) return 0;
   return rows % (8 * 2 * kBlock) ? 0 : (int)(rows / (2 * kBlock));
 }
+// Workgroups of a row-run launch over `rows` rows.
 inline unsigned run_tiles(int64_t rows, int bs = kBlock) { return (unsigned)((rows + 2 * bs - 1) / (2 * bs)); }
 
 // y = A x over rows [0, nrows); ComputeSPMV_ref.cpp:61-70

@@ -21,8 +21,8 @@ static inline unsigned tiles(int64_t rows) { return (unsigned)((rows + kBlock - 
 // to 2^20 rows the fp16 V-cycle of kappa 256x192x144 (884736 rows) ran 111 -> 114 ms.
 constexpr int64_t kOneWaveRows = 1 << 18;
 
-// rz (fp64 stencil levels only): the step also leaves the partials of r.x
-// over its rows there, tiles(rows) of them.
+// rz (the finest level of an fp64 stencil hierarchy only): the step also leaves the
+// partials of r.x over its rows there, tiles(rows) of them.
 template <class VT, class XT, class ACC, int ZK, bool FINE>
 static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *rz = nullptr) {
   const int64_t r0 = L.lay.start[k], nr = L.lay.start[k + 1] - r0;
@@ -44,7 +44,7 @@ static void gs_block(Ctx *c, const Level &L, const XT *r, XT *x, int k, double *
   const unsigned g = (unsigned)((nr + bs - 1) / bs);
   hipStream_t st = c->stream;
   const ValSrc<VT, ACC> v = val_src<VT, ACC>(L);
-  if constexpr (ZK < 0 && sizeof(VT) == 8 && sizeof(XT) == 8) {
+  if constexpr (FINE && ZK < 0 && sizeof(VT) == 8 && sizeof(XT) == 8) {
     if (rz) {
       // 256-thread blocks: the partials are per block of 4 waves, tiles(nr) of them
       with_forms<VT, true>(L, ci, [&](auto CF, auto VF) {
@@ -255,7 +255,7 @@ static int symgs_launch(Ctx *c, int l, const XT *r, XT *x, bool zero_start, doub
                         int64_t *nrz = nullptr) {
   const Level &L = c->levels[l];
   if (l == 0) sweep<VT, XT, ACC, true>(c, L, r, x, zero_start, rz, nrz);
-  else sweep<VT, XT, ACC, false>(c, L, r, x, zero_start, rz, nrz);
+  else sweep<VT, XT, ACC, false>(c, L, r, x, zero_start);
   HPCGX_CHECK_LAUNCH(c);
   return HPCGX_OK;
 }
@@ -331,7 +331,7 @@ static bool tail(Ctx *c, int l, const XT *r, XT *x, bool load_x = false) {
 // V-cycle of ComputeMG_ref.cpp:39-63: x = 0; pre-smooth; residual + restrict;
 // recurse; prolong; post-smooth.  The coarsest level gets one smoothing step.
 // rz / nrz: r.x partials of the result from the post-smoother (see sweep);
-// fp64 stencil levels with a coarse level only.
+// from level 0 of an fp64 stencil hierarchy with a coarse level only.
 template <class VT, class XT, class ACC, bool SCALE>
 static int vcycle(Ctx *c, int l, const XT *r, XT *x, double *rz = nullptr, int64_t *nrz = nullptr) {
   const Level &L = c->levels[l];

@@ -323,12 +323,28 @@ static int totals_coherent() {
   return 0;
 }
 
+// r.z is left by the finest level's steps alone: no such kernel is built for others
+// (k_gs<VT, XT, ACC, ZK, FINE, CF, VF, GEN, RZ>, k_gs_run<ZK, FINE, VF, RZ>).
+static int rz_kernels() {
+  int fine = 0;
+  for (const auto &k : kernels()) {
+    const std::string &n = k.second;
+    const bool gs = n.find("4k_gsI") != std::string::npos, run = n.find("8k_gs_runI") != std::string::npos;
+    if ((!gs && !run) || n.find("ELb1EEEv") == std::string::npos) continue;  // RZ is the last argument
+    CHECK(n.find(gs ? "IdddLin1ELb1E" : "ILin1ELb1E") != std::string::npos);
+    ++fine;
+  }
+  CHECK(fine > 0);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "one_plane") return one_plane();
   if (s == "forms_after_failure") return forms_after_failure();
   if (s == "total_after_failure") return total_after_failure();
   if (s == "totals_coherent") return totals_coherent();
+  if (s == "rz_kernels") return rz_kernels();
   std::printf("no scenario: %s\n", s.c_str());
   return 2;
 }
