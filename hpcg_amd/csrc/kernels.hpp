@@ -992,7 +992,7 @@ __device__ __forceinline__ XT gs_value(const ColIdx &ci, const ValSrc<VT, ACC> &
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
       if (!((mask >> s) & 1u)) continue;
-      if (!GEN && s == kDiagSlot) {
+      if (!GEN && CF != kColsStored && s == kDiagSlot) {  // explicit columns: every index is read, its own too
         sum -= vr.at(s, 0) * xi;
         continue;
       }
