@@ -24,8 +24,8 @@ constexpr int kMaxLevels = 8;
 
 // Column forms of a 64-row slice in the compact index copy.  A zero-valued
 // slot (a neighbour outside the grid, an unused entry) may name any row of
-// the level, since its product is an exact zero; the diagonal always counts
-// as a stored entry.
+// the level, since its product is an exact zero (mend_nan, where that row's x
+// is not finite); the diagonal always counts as a stored entry.
 enum ColForm : uint8_t {
   kFormDelta = 0,    // column = base[slot] + lane + int8 delta[slot][lane]
   kFormWide = 1,     // some delta does not fit in int8: the explicit 32-bit column

@@ -1272,8 +1272,9 @@ __global__ __launch_bounds__(kBlock) void k_prolong(XT *__restrict__ x, const XT
 // barrier separates the colour steps, the matrix comes from L2.  The rows' sums
 // are those of the separate launches, in the same order.
 //
-// V-cycle, launches -> tail: 8^3 (3 levels) 289 -> 84 us, 16^3 299 -> 114 (fp32
-// 304 -> 107), 20^3 (2 levels) 133 -> 85 (fp32 141 -> 78).  The limit is a block of
+// V-cycles, called back to back, launches -> tail -> with sweep_slot: 8^3 (3 levels)
+// 151 -> 81 -> 70 us, 16^3 (4 levels) 220 -> 124 -> 105 (fp32 225 -> 133 -> 94), 20^3 (2
+// levels) 94 -> 82 -> 73 (fp32 100 -> 79 -> 64).  The limit is a block of
 // a slice per wave: a 24^3 level (27 slices a block) takes one CU as long as a
 // launch per step takes 256 (64 us against 47 to 57), a 26^3 one longer (187
 // against 132).
@@ -1316,9 +1317,8 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(const TailArgs<VT, XT, AC
   // chain of 27 sums, a division and a barrier: what comes from memory (the
   // row's mask) is fetched a step ahead, the slots' values and the level's
   // fields are read once.  A slot without an entry reads the zero that lies behind
-  // the level's x.  V-cycle on the device, sweep below -> this one: 8^3
-  // (4 levels) 52 -> 41 us, 16^3 63 -> 54 (fp32 64 -> 56); 20^3, whose second
-  // level has an odd size, 84 -> 81.
+  // the level's x.  (20^3: its second level has an odd size and takes the sweep
+  // below.)
   auto sweep_slot = [&](const TailLevel<VT, XT, ACC> &L) {
     XT *x = lds + L.xoff;
     const XT *r = lds + L.roff;

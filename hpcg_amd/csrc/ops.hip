@@ -16,8 +16,8 @@ static inline unsigned tiles(int64_t rows) { return (unsigned)((rows + kBlock - 
 // level and in every precision: a block of 105105 rows is 411 workgroups of 256
 // threads, so that some of the 256 CUs take two and others one, and a step lasts as
 // long as the fullest.  By single waves the CUs take 6 or 7 of 1643.  SYMGS kappa
-// 97x65x129 201 -> 188 us, CG on general rows 64^3 19.6 -> 18.4 ms, CG 104^3 26.7 ->
-// 26.1.  Above, the split no longer shows and a workgroup's waves share the L1: up
+// 97x65x129 199 -> 185 us, CG on general rows 64^3 19.7 -> 18.4 ms, CG 104^3 26.5 ->
+// 25.8.  Above, the split no longer shows and a workgroup's waves share the L1: up
 // to 2^20 rows the fp16 V-cycle of kappa 256x192x144 (884736 rows) ran 111 -> 114 ms.
 constexpr int64_t kOneWaveRows = 1 << 18;
 
