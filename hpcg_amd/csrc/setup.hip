@@ -1765,9 +1765,10 @@ int hpcgx_level_set_diagonal(hpcgx_ctx *c, int level, const double *diag) {
   int rc = ensure_stage(c, L.lay.n);
   if (rc) return rc;
   HPCGX_HIP(c, hipMemcpyAsync(c->stage, diag, L.lay.n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  L.diag_one = false;  // read from the array, unless it is found to be the slot's value on every row
   k_set_diag<<<nblk(L.lay.n), kBlock, 0, c->stream>>>(L.vals, L.dslot, L.perm, c->stage, L.lay.n);
   HPCGX_CHECK_LAUNCH(c);
-  if (L.vform == kValsSlot) {  // one value on every row, or read from the array from now on
+  if (L.vform == kValsSlot) {
     int *flags = reinterpret_cast<int *>(c->scal + S_COUNT), *bad = reinterpret_cast<int *>(c->hbuf);
     k_clear_flags<<<1, 64, 0, c->stream>>>(flags);
     k_check_diag<<<nblk(L.lay.npad), kBlock, 0, c->stream>>>(L.vals, L.vmask, L.slotv, L.lay.npad, flags);

@@ -36,6 +36,7 @@ int last_error = kOk;
 int fail_malloc = 0;          // the coming hipMalloc that fails, counted from 1 (0: none)
 std::string fail_launch;      // launches of a kernel whose name holds this fail
 int fail_after = 0;           // once so many of them have run
+int spmv_diag_one = -1;       // whether the last SpMV took the diagonals from the slot's value
 int handle_count = 0;
 
 int failed(int code) { return last_error = code; }
@@ -109,6 +110,8 @@ int hipLaunchKernel(const void *stub, Dim3 grid, Dim3 block, void **args, size_t
   if (!fail_launch.empty() && name.find(fail_launch) != std::string::npos && fail_after-- <= 0)
     return failed(kLaunchFailure);
   ++launched[name];
+  if (name.find("k_spmvI") != std::string::npos)  // (ci, src, ..): ValSrc is four pointers and diag_one
+    spmv_diag_one = *reinterpret_cast<int *>(static_cast<char *>(args[1]) + 4 * sizeof(void *));
   if (name.find("k_finish") != std::string::npos)  // (partials, G, scal, op, slot, host)
     under_way.push_back({*reinterpret_cast<double **>(args[5]), ++totals});
   return kOk;
@@ -338,6 +341,26 @@ static int rz_kernels() {
   return 0;
 }
 
+// A diagonal that was replaced and could not be looked over is read from the
+// value array, where it is, and not from the slot's value.
+static int diagonal_after_failure() {
+  hpcgx_ctx *c;
+  CHECK(hpcgx_create(0, &c) == HPCGX_OK);
+  CHECK(hpcgx_problem_generate(c, 16, 16, 16, 2, nullptr) == HPCGX_OK);
+  double *x, *y;
+  CHECK(hpcgx_vec_alloc(c, 0, &x) == HPCGX_OK && hpcgx_vec_alloc(c, 0, &y) == HPCGX_OK);
+  const std::vector<double> diag(4096, 31.0);
+  CHECK(hpcgx_spmv(c, 0, x, y) == HPCGX_OK && spmv_diag_one == 1);
+  fail_launch = "k_check_diag";
+  CHECK(hpcgx_level_set_diagonal(c, 0, diag.data()) == HPCGX_EHIP);
+  fail_launch.clear();
+  CHECK(hpcgx_spmv(c, 0, x, y) == HPCGX_OK && spmv_diag_one == 0);
+  CHECK(hpcgx_level_set_diagonal(c, 0, diag.data()) == HPCGX_OK);
+  CHECK(hpcgx_spmv(c, 0, x, y) == HPCGX_OK && spmv_diag_one == 1);
+  CHECK(hpcgx_destroy(c) == HPCGX_OK);
+  return 0;
+}
+
 int main(int argc, char **argv) {
   const std::string s = argc > 1 ? argv[1] : "";
   if (s == "one_plane") return one_plane();
@@ -345,6 +368,7 @@ int main(int argc, char **argv) {
   if (s == "total_after_failure") return total_after_failure();
   if (s == "totals_coherent") return totals_coherent();
   if (s == "rz_kernels") return rz_kernels();
+  if (s == "diagonal_after_failure") return diagonal_after_failure();
   std::printf("no scenario: %s\n", s.c_str());
   return 2;
 }

@@ -20,7 +20,7 @@ def host_path(hip, tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["one_plane", "forms_after_failure", "total_after_failure",
-                                      "totals_coherent", "rz_kernels"])
+                                      "totals_coherent", "rz_kernels", "diagonal_after_failure"])
 def test_scenario(host_path, scenario):
     out = subprocess.run([host_path, scenario], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
